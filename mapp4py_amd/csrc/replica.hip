@@ -8,8 +8,8 @@
 //   DynamicMD::decide (skin check, rebuild)           src/dynamic_md.cpp:90-105
 //
 // Design: a replica's minimisation is sequential, so the parallelism is
-// across replicas and, inside one, across its atoms. One wave (small
-// replicas) or a whole 256-thread workgroup (large ones) owns a replica for
+// across replicas and, inside one, across its atoms. One wave or
+// a whole 1024-thread workgroup owns a replica for
 // the entire minimisation: its full neighbor list (every periodic image,
 // 7-bit image codes), both EAM passes in FP64, the inner products and the
 // line search all run inside the one persistent launch, with no host round
@@ -51,12 +51,24 @@ __device__ inline double dhval(const double4 c, double p) { return (3.0 * c.w * 
 __device__ inline void spline_at(double v, double inv, int n, int& m, double& p)
 {
     p = v * inv;
-    long long mm = (long long)p;
-    if (mm > n - 2) mm = n - 2;
-    if (mm < 0) mm = 0;
+    int mm = (int)p;
+    mm = mm < n - 2 ? mm : n - 2;
+    mm = mm > 0 ? mm : 0;
     p -= (double)mm;
-    if (p > 1.0) p = 1.0;
-    m = (int)mm;
+    p = p < 1.0 ? p : 1.0;
+    m = mm;
+}
+
+// r = sqrt(x) and 1 / r to an ulp or so: the hardware's reciprocal root
+// (about 24 bits), one third-order step for the inverse, one for the root
+__device__ inline void root_inv(double x, double& r, double& r_inv)
+{
+    double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-(x * y), y, 1.0);
+    y = fma(y * e, fma(0.375, e, 0.5), y);
+    const double t = x * y;
+    r = fma(fma(-t, t, x), 0.5 * y, t);
+    r_inv = y;
 }
 
 __device__ inline int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -67,6 +79,25 @@ __device__ inline double uni(double v)
     const int hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
     return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
 }
+
+// Waves of the workgroup that owns a replica. The largest replica's chain of
+// steps ends the launch, so it gets every wave a CU can hold at 128 registers
+// a lane. 1024 Ni-H cells of 108 to 4,076 atoms, 20 steps each: 390 ms with
+// four waves, all-pairs list builds and one entry after another in the passes,
+// 59 ms now. In the largest cell a density pass takes 0.31 ms (its issue
+// bound, 4 atoms a lane, is about 0.15), a force pass 0.44 and a list build
+// 2.3, of 20 steps' 40 density and 20 force passes and 8 builds.
+constexpr int kWide = 16;
+constexpr int kShifts = 125;  // image codes
+
+struct Shared {
+    double red[2][kWide];             // partial sums, two rows in turn
+    double shift[kWide][kShifts][3];  // n H of every image code: row 0 of a workgroup's replica, row w of a wave's
+    int own0[65 * kWide];             // list build: where each cell's (segment's) atoms start in ord,
+    int cand0[65 * kWide];            // and its candidates; 65 a wave or all for a workgroup
+    double cut_sq[kMaxElems * kMaxElems], cutsk_sq[kMaxElems * kMaxElems];
+    int next;
+};
 
 template <int W>
 __device__ inline void group_sync()
@@ -79,38 +110,46 @@ __device__ inline void group_sync()
     }
 }
 
+struct Ctx {
+    int off, n, maxn, nt, t, w;
+    int lg;    // log2 of the lanes that share an atom in the EAM passes
+    int flip;  // row of Shared::red of the next sum
+    long long loff;
+    double h[6], b[6], cs[3];
+    Shared* S;
+};
+
 // sums and maxima over the replica's lanes, in a fixed order, returned alike
-// to every lane
-template <int W>
-__device__ inline double group_sum(double v, double* red, int w)
+// to every lane. A row of partial sums is written again only after the
+// barrier of the reduction in between, so one barrier each is enough; it also
+// orders the replica's memory, as group_sync does.
+template <int W, class Op>
+__device__ inline double group_fold(double v, Ctx& C, Op op)
 {
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    for (int off = 32; off > 0; off >>= 1) v = op(v, __shfl_xor(v, off, 64));
     v = uni(v);
     if constexpr (W == 1) {
+        group_sync<1>();
         return v;
     } else {
-        red[w] = v;
+        double* row = C.S->red[C.flip];
+        C.flip ^= 1;
+        row[C.w] = v;
         __syncthreads();
-        const double s = (red[0] + red[1]) + (red[2] + red[3]);
-        __syncthreads();
+        double s = row[0];
+        for (int k = 1; k < W; ++k) s = op(s, row[k]);
         return uni(s);
     }
 }
-
 template <int W>
-__device__ inline double group_max(double v, double* red, int w)
+__device__ inline double group_sum(double v, Ctx& C)
 {
-    for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
-    v = uni(v);
-    if constexpr (W == 1) {
-        return v;
-    } else {
-        red[w] = v;
-        __syncthreads();
-        const double s = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
-        __syncthreads();
-        return uni(s);
-    }
+    return group_fold<W>(v, C, [](double a, double b) { return a + b; });
+}
+template <int W>
+__device__ inline double group_max(double v, Ctx& C)
+{
+    return group_fold<W>(v, C, [](double a, double b) { return fmax(a, b); });
 }
 
 // x -> s = x B without the wrap (the positions move freely during a
@@ -122,161 +161,337 @@ __device__ inline void to_s(const double* b, const double4& x, double* s)
     s[2] = b[5] * x.z;
 }
 
-__device__ inline void image_dx(const double* h, const double4& xi, const double4& xj, uint32_t code, double& dx,
-                                double& dy, double& dz)
+// x_i - (x_j + n H) of an image code
+__device__ inline void image_dx(const double (*shift)[3], const double4& xi, const double4& xj, uint32_t code,
+                                double& dx, double& dy, double& dz)
 {
-    const int n2 = (int)(code / 25u) - 2;
-    const int rem = (int)(code % 25u);
-    const int n1 = rem / 5 - 2, n0 = rem % 5 - 2;
-    dx = xi.x - (xj.x + (h[0] * n0 + h[1] * n1 + h[2] * n2));
-    dy = xi.y - (xj.y + (h[3] * n1 + h[4] * n2));
-    dz = xi.z - (xj.z + h[5] * n2);
+    const double* sh = shift[code];
+    dx = xi.x - (xj.x + sh[0]);
+    dy = xi.y - (xj.y + sh[1]);
+    dz = xi.z - (xj.z + sh[2]);
 }
-
-struct Ctx {
-    int off, n, maxn, nt, t;
-    long long loff;
-    double h[6], b[6], cs[3];
-};
 
 // The full list of the replica: every (j, image) with |x_i - x_j - n H| below
 // r_c + skin, except i itself at the zero image. Returns a failure code (0 ok).
+// The atoms are binned into cells at least as wide as the cut-off's extent
+// along each box vector (their s wrapped into the box), and the candidates of
+// a cell's atoms are the atoms of the 27 cells around it; comparing all pairs
+// took 7.5 ms a build at 4,076 atoms, most of the launch (2.3 ms now). Candidates are
+// collected in index order (a group of lanes scans all atoms for each cell, a
+// segment each), so a row lists its neighbors in the order of (j, image): its
+// sums do not depend on when it was built. Rows are worked on in cell order,
+// so that the lanes of a wave read the same candidates.
 template <int W>
-__device__ int build_list(const RepArgs& A, const Ctx& C, const RepArrays& R, double* red, int w)
+__device__ int build_list(const RepArgs& A, Ctx& C, const RepArrays& R)
 {
+    constexpr int kCells = 64 * W;  // most cells, and cells times segments
     const int ne = A.ne;
-    double fail = 0.0;
+    const double(*shift)[3] = C.S->shift[W == 1 ? C.w : 0];
+    int* own0 = C.S->own0 + (W == 1 ? (64 + 1) * C.w : 0);
+    int* cand0 = C.S->cand0 + (W == 1 ? (64 + 1) * C.w : 0);
+    int* ord = R.ord + C.off;
+    uint32_t* cand = R.cand + 27 * (size_t)C.off;
+    int nc[3];
+    for (int d = 0; d < 3; ++d) {
+        const double k = 1.0 / (C.cs[d] * 1.0000001), most = kCells < 256 ? kCells : 256;
+        nc[d] = (int)(k < most ? k : most);
+        nc[d] = nc[d] > 1 ? nc[d] : 1;
+    }
+    while (nc[0] * nc[1] * nc[2] > kCells) {
+        const int d = nc[0] >= nc[1] && nc[0] >= nc[2] ? 0 : nc[1] >= nc[2] ? 1 : 2;
+        nc[d] = (nc[d] + 1) / 2;
+    }
+    const int ncell = nc[0] * nc[1] * nc[2];
+    int nseg = 1;
+    while (2 * nseg * ncell <= C.nt && nseg < 16) nseg *= 2;
+    const int seg = (C.n + nseg - 1) / nseg;
+    // how many boxes away from the origin the atoms lie, per box vector
+    double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
+    for (int i = C.t; i < C.n; i += C.nt) {
+        double s[3];
+        to_s(C.b, R.x[C.off + i], s);
+        for (int d = 0; d < 3; ++d) {
+            lo[d] = fmin(lo[d], floor(s[d]));
+            hi[d] = fmax(hi[d], floor(s[d]));
+        }
+    }
+    // In a box of at least 3 cells along each vector, whose atoms lie in one
+    // box or the next, a candidate can be listed at one image only, which its
+    // cell gives: the entry of cand then holds the image's code too.
+    bool fast = true;
+    for (int d = 0; d < 3; ++d) {
+        lo[d] = -group_max<W>(-lo[d], C);
+        hi[d] = group_max<W>(hi[d], C);
+        fast = fast && nc[d] >= 3 && hi[d] - lo[d] <= 1.0;
+    }
+    // cid: 8 bits of cell per box vector, then one each for lying in the next box
     for (int i = C.t; i < C.n; i += C.nt) {
         const double4 xi = R.x[C.off + i];
         R.xb[C.off + i] = xi;
+        double s[3];
+        to_s(C.b, xi, s);
+        int id = 0;
+        for (int d = 0; d < 3; ++d) {
+            const double w = floor(s[d]);
+            const int c = (int)((s[d] - w) * nc[d]);
+            id |= (c < nc[d] - 1 ? c : nc[d] - 1) << (8 * d) | (w > lo[d] ? 1 << (24 + d) : 0);
+        }
+        R.cid[C.off + i] = id;
+    }
+    group_sync<W>();
+    // 0: own cell, 1: a cell next to it (through the box faces too), 2: neither;
+    // the code of the candidate's image
+    auto relation = [&](int id, const int* c, uint32_t& code) {
+        int rel = 0, step = 1, k = kZeroImage;
+        for (int d = 0; d < 3; ++d, step *= 5) {
+            const int e = (id >> (8 * d) & 255) - c[d];
+            const int r = e == 0 ? 0 : e == 1 || e == -1 || e == nc[d] - 1 || e == 1 - nc[d] ? 1 : 2;
+            rel = r > rel ? r : rel;
+            k += step * ((e == 1 - nc[d] ? 1 : e == nc[d] - 1 ? -1 : 0) - (id >> (24 + d) & 1));
+        }
+        code = fast ? (uint32_t)k << kIndexBits : 0u;
+        return rel;
+    };
+    for (int fill = 0; fill < 2; ++fill) {
+        for (int u = C.t; u < ncell * nseg; u += C.nt) {
+            const int cc = u / nseg;
+            const int c[3] = {cc % nc[0], cc / nc[0] % nc[1], cc / (nc[0] * nc[1])};
+            const int j0 = (u & (nseg - 1)) * seg, j1 = j0 + seg < C.n ? j0 + seg : C.n;
+            int ko = fill ? own0[u] : 0, kc = fill ? cand0[u] : 0;
+            for (int jb = j0; jb < j1; jb += 4) {
+                int id[4];
+                for (int b = 0; b < 4; ++b) id[b] = R.cid[C.off + (jb + b < j1 ? jb + b : jb)];
+                for (int b = 0; b < 4; ++b) {
+                    const int j = jb + b;
+                    uint32_t code = 0u;
+                    const int rel = j < j1 ? relation(id[b], c, code) : 2;
+                    if (rel < 2 && fill) cand[kc] = (uint32_t)j | code;
+                    if (rel == 0 && fill) ord[ko] = j;
+                    kc += rel < 2 ? 1 : 0;
+                    ko += rel == 0 ? 1 : 0;
+                }
+            }
+            if (!fill) {
+                own0[u] = ko;
+                cand0[u] = kc;
+            }
+        }
+        group_sync<W>();
+        if (!fill && C.t == 0) {
+            int ko = 0, kc = 0;
+            for (int u = 0; u < ncell * nseg; ++u) {
+                const int o = own0[u], k = cand0[u];
+                own0[u] = ko;
+                cand0[u] = kc;
+                ko += o;
+                kc += k;
+            }
+            cand0[ncell * nseg] = kc;
+        }
+        group_sync<W>();
+    }
+    // a sphere thinner than half the box along every box vector holds one
+    // image of an atom at most, the nearest
+    const bool nearest = C.cs[0] < 0.499 && C.cs[1] < 0.499 && C.cs[2] < 0.499;
+    double fail = 0.0;
+    for (int q = C.t; q < C.n; q += C.nt) {
+        const int i = ord[q];
+        const int id = R.cid[C.off + i];
+        const double4 xi = R.x[C.off + i];
         const int ei = (int)xi.w;
+        const int cell = (id & 255) + nc[0] * ((id >> 8 & 255) + nc[1] * (id >> 16 & 255));
         double si[3];
         to_s(C.b, xi, si);
         int cnt = 0;
-        for (int j = 0; j < C.n; ++j) {
-            const double4 xj = R.x[C.off + j];
-            const int ej = (int)xj.w;
-            double sj[3];
-            to_s(C.b, xj, sj);
-            int lo[3], hi[3];
-            for (int d = 0; d < 3; ++d) {
-                const double ds = si[d] - sj[d];
-                lo[d] = (int)ceil(ds - C.cs[d]);
-                hi[d] = (int)floor(ds + C.cs[d]);
+        auto visit = [&](int j, const double4& xj, uint32_t code) {
+            double dx, dy, dz;
+            image_dx(shift, xi, xj, code, dx, dy, dz);
+            const double rsq = dx * dx + (dy * dy + dz * dz);
+            if (rsq < C.S->cutsk_sq[ei * ne + (int)xj.w] && (j != i || code != (uint32_t)kZeroImage)) {
+                if (cnt < C.maxn) R.list[C.loff + (long long)cnt * C.n + i] = (uint32_t)j | (code << kIndexBits);
+                ++cnt;
             }
-            for (int n2 = lo[2]; n2 <= hi[2]; ++n2)
-                for (int n1 = lo[1]; n1 <= hi[1]; ++n1)
-                    for (int n0 = lo[0]; n0 <= hi[0]; ++n0) {
-                        if (j == i && n0 == 0 && n1 == 0 && n2 == 0) continue;
-                        if (n0 < -kRepMaxImages || n0 > kRepMaxImages || n1 < -kRepMaxImages ||
-                            n1 > kRepMaxImages || n2 < -kRepMaxImages || n2 > kRepMaxImages) {
+        };
+        // the next candidate's position and the entry after it are loaded
+        // while one is looked at
+        const int kb = cand0[cell * nseg], ke = cand0[(cell + 1) * nseg];
+        const uint32_t wrap = (uint32_t)((id >> 24 & 1) + 5 * (id >> 25 & 1) + 25 * (id >> 26 & 1));
+        uint32_t en = cand[kb], enn = cand[kb + 1 < ke ? kb + 1 : kb];
+        double4 xn = R.x[C.off + (int)(en & kIndexMask)];
+        for (int k = kb; k < ke; ++k) {
+            const uint32_t e = en;
+            const int j = (int)(e & kIndexMask);
+            const double4 xj = xn;
+            en = enn;
+            xn = R.x[C.off + (int)(en & kIndexMask)];
+            enn = cand[k + 2 < ke ? k + 2 : ke - 1];
+            if (fast) {
+                visit(j, xj, (e >> kIndexBits) + wrap);
+                continue;
+            }
+            double ds[3];
+            to_s(C.b, xj, ds);
+            for (int d = 0; d < 3; ++d) ds[d] = si[d] - ds[d];
+            if (nearest) {
+                const double n0 = rint(ds[0]), n1 = rint(ds[1]), n2 = rint(ds[2]);
+                if (fmax(fabs(ds[0] - n0) - C.cs[0], fmax(fabs(ds[1] - n1) - C.cs[1], fabs(ds[2] - n2) - C.cs[2])) > 0.0)
+                    continue;
+                if (fmax(fabs(n0), fmax(fabs(n1), fabs(n2))) > (double)kRepMaxImages)
+                    fail = fmax(fail, (double)FAIL_IMAGE);
+                else
+                    visit(j, xj, (uint32_t)(int)(n0 + 5.0 * n1 + 25.0 * n2 + (double)kZeroImage));
+                continue;
+            }
+            for (double n2 = ceil(ds[2] - C.cs[2]); n2 <= floor(ds[2] + C.cs[2]); n2 += 1.0)
+                for (double n1 = ceil(ds[1] - C.cs[1]); n1 <= floor(ds[1] + C.cs[1]); n1 += 1.0)
+                    for (double n0 = ceil(ds[0] - C.cs[0]); n0 <= floor(ds[0] + C.cs[0]); n0 += 1.0) {
+                        if (fmax(fabs(n0), fmax(fabs(n1), fabs(n2))) > (double)kRepMaxImages)
                             fail = fmax(fail, (double)FAIL_IMAGE);
-                            continue;
-                        }
-                        const uint32_t code = (uint32_t)((n0 + 2) + 5 * (n1 + 2) + 25 * (n2 + 2));
-                        double dx, dy, dz;
-                        image_dx(C.h, xi, xj, code, dx, dy, dz);
-                        const double rsq = dx * dx + (dy * dy + dz * dz);
-                        if (rsq < A.cutsk_sq[ei * ne + ej]) {
-                            if (cnt < C.maxn)
-                                R.list[C.loff + (long long)cnt * C.n + i] = (uint32_t)j | (code << kIndexBits);
-                            ++cnt;
-                        }
+                        else
+                            visit(j, xj, (uint32_t)(int)(n0 + 5.0 * n1 + 25.0 * n2 + (double)kZeroImage));
                     }
         }
         if (cnt > C.maxn) fail = fmax(fail, (double)FAIL_LIST);
         R.nn[C.off + i] = cnt < C.maxn ? cnt : C.maxn;
     }
-    const double f = group_max<W>(fail, red, w);
-    group_sync<W>();
-    return (int)f;
+    return (int)group_max<W>(fail, C);
 }
 
-// ForceFieldEAM's energy (and with forces, its forces): E = sum_i F(rho_i)
-// + 1/2 sum over the full list of phi; F extended linearly past rho_max
-// (src/ff_eam.cpp:181-192,313-314).
-template <int W>
-__device__ double eam_energy(const RepArgs& A, const Ctx& C, const RepArrays& R, bool forces, double* red, int w)
+// B list entries k0 .. k0 + B - 1 of atom i with their neighbors' positions,
+// all loads in flight together (a pass on its own waits for list, position
+// and spline row of one entry after another): entries past the row's end
+// repeat its last one and are marked out.
+template <int B>
+__device__ inline void fetch(const Ctx& C, const RepArrays& R, int i, int cnt, int k0, uint32_t (&e)[B],
+                             double4 (&xj)[B])
 {
-    const int ne = A.ne, nr = A.nr;
+    for (int b = 0; b < B; ++b) {
+        const int k = k0 + b < cnt ? k0 + b : cnt - 1;
+        e[b] = R.list[C.loff + (long long)k * C.n + i];
+    }
+    for (int b = 0; b < B; ++b) xj[b] = R.x[C.off + (int)(e[b] & kIndexMask)];
+}
+
+// The density pass of ForceFieldEAM: E = sum_i F(rho_i) + 1/2 sum over the
+// full list of phi; F extended linearly past rho_max (src/ff_eam.cpp:181-192,
+// 313-314); leaves F'(rho_i) in dF. 2^lg lanes share an atom's entries.
+template <int W>
+__device__ double eam_energy(const RepArgs& A, Ctx& C, const RepArrays& R)
+{
+    constexpr int B = 4;
+    const int ne = A.ne, nr = A.nr, G = 1 << C.lg, g = C.t & (G - 1), units = C.nt >> C.lg;
+    const double(*shift)[3] = C.S->shift[W == 1 ? C.w : 0];
     double part = 0.0;
-    for (int i = C.t; i < C.n; i += C.nt) {
-        const double4 xi = R.x[C.off + i];
+    for (int i0 = 0; i0 < C.n; i0 += units) {
+        const int i = i0 + (C.t >> C.lg);
+        const bool own = i < C.n;
+        const double4 xi = R.x[C.off + (own ? i : 0)];
         const int ei = (int)xi.w;
-        const int cnt = R.nn[C.off + i];
+        const int cnt = own ? R.nn[C.off + i] : 0;
         double rho = 0.0, ephi = 0.0;
-        for (int k = 0; k < cnt; ++k) {
-            const uint32_t e = R.list[C.loff + (long long)k * C.n + i];
-            const double4 xj = R.x[C.off + (int)(e & kIndexMask)];
-            const int ej = (int)xj.w;
-            double dx, dy, dz;
-            image_dx(C.h, xi, xj, e >> kIndexBits, dx, dy, dz);
-            const double rsq = dx * dx + (dy * dy + dz * dz);
-            if (rsq >= A.cut_sq[ei * ne + ej]) continue;
-            const double r = sqrt(rsq);
+        for (int k0 = g * B; k0 < cnt; k0 += G * B) {
+            uint32_t e[B];
+            double4 xj[B], cr[B], cp[B];
+            double p[B], ri[B];
+            bool in[B];
+            fetch<B>(C, R, i, cnt, k0, e, xj);
+            for (int b = 0; b < B; ++b) {
+                const int ej = (int)xj[b].w;
+                double dx, dy, dz, r;
+                image_dx(shift, xi, xj[b], e[b] >> kIndexBits, dx, dy, dz);
+                const double rsq = dx * dx + (dy * dy + dz * dz);
+                in[b] = k0 + b < cnt && rsq < C.S->cut_sq[ei * ne + ej];
+                int m;
+                root_inv(in[b] ? rsq : 1.0, r, ri[b]);
+                spline_at(r, A.dr_inv, nr, m, p[b]);
+                cr[b] = A.rho[(size_t)(ej * ne + ei) * nr + m];
+                cp[b] = A.phi[(size_t)(ei * ne + ej) * nr + m];
+            }
+            for (int b = 0; b < B; ++b) {
+                rho += in[b] ? hval(cr[b], p[b]) : 0.0;
+                ephi += in[b] ? hval(cp[b], p[b]) * ri[b] : 0.0;
+            }
+        }
+        for (int o = 1; o < G; o <<= 1) {
+            rho += __shfl_xor(rho, o, 64);
+            ephi += __shfl_xor(ephi, o, 64);
+        }
+        if (own && g == 0) {
             int m;
             double p;
-            spline_at(r, A.dr_inv, nr, m, p);
-            rho += hval(A.rho[(size_t)(ej * ne + ei) * nr + m], p);
-            ephi += hval(A.phi[(size_t)(ei * ne + ej) * nr + m], p) / r;
+            spline_at(rho, A.drho_inv, A.nrho, m, p);
+            const double4 c = A.F[(size_t)ei * A.nrho + m];
+            double Fi = hval(c, p);
+            const double dFi = dhval(c, p) * A.drho_inv;
+            if (rho > A.rho_max) Fi += dFi * (rho - A.rho_max);
+            R.dF[C.off + i] = dFi;
+            part += Fi + 0.5 * ephi;
         }
-        int m;
-        double p;
-        spline_at(rho, A.drho_inv, A.nrho, m, p);
-        const double4 c = A.F[(size_t)ei * A.nrho + m];
-        double Fi = hval(c, p);
-        const double dFi = dhval(c, p) * A.drho_inv;
-        if (rho > A.rho_max) Fi += dFi * (rho - A.rho_max);
-        R.dF[C.off + i] = dFi;
-        part += Fi + 0.5 * ephi;
     }
-    const double en = group_sum<W>(part, red, w);
-    if (!forces) return en;
-    group_sync<W>();
-    for (int i = C.t; i < C.n; i += C.nt) {
-        const double4 xi = R.x[C.off + i];
+    return group_sum<W>(part, C);
+}
+
+// The force pass at the positions of the last density pass.
+template <int W>
+__device__ void eam_force(const RepArgs& A, Ctx& C, const RepArrays& R)
+{
+    constexpr int B = 2;
+    const int ne = A.ne, nr = A.nr, G = 1 << C.lg, g = C.t & (G - 1), units = C.nt >> C.lg;
+    const double(*shift)[3] = C.S->shift[W == 1 ? C.w : 0];
+    for (int i0 = 0; i0 < C.n; i0 += units) {
+        const int i = i0 + (C.t >> C.lg);
+        const bool own = i < C.n;
+        const double4 xi = R.x[C.off + (own ? i : 0)];
         const int ei = (int)xi.w;
-        const double dFi = R.dF[C.off + i];
-        const int cnt = R.nn[C.off + i];
+        const double dFi = R.dF[C.off + (own ? i : 0)];
+        const int cnt = own ? R.nn[C.off + i] : 0;
         double fx = 0.0, fy = 0.0, fz = 0.0;
-        for (int k = 0; k < cnt; ++k) {
-            const uint32_t e = R.list[C.loff + (long long)k * C.n + i];
-            const int j = (int)(e & kIndexMask);
-            const double4 xj = R.x[C.off + j];
-            const int ej = (int)xj.w;
-            double dx, dy, dz;
-            image_dx(C.h, xi, xj, e >> kIndexBits, dx, dy, dz);
-            const double rsq = dx * dx + (dy * dy + dz * dz);
-            if (rsq >= A.cut_sq[ei * ne + ej]) continue;
-            const double r = sqrt(rsq);
-            const double r_inv = 1.0 / r;
-            int m;
-            double p;
-            spline_at(r, A.dr_inv, nr, m, p);
-            const double4 cz = A.phi[(size_t)(ei * ne + ej) * nr + m];
-            const double z = hval(cz, p);
-            const double zp = dhval(cz, p) * A.dr_inv;
-            const double phi = z * r_inv;
-            const double dphi = (zp - phi) * r_inv;
-            const double drho_ji = dhval(A.rho[(size_t)(ej * ne + ei) * nr + m], p) * A.dr_inv;
-            const double drho_ij = dhval(A.rho[(size_t)(ei * ne + ej) * nr + m], p) * A.dr_inv;
-            const double fpair = -(dphi + dFi * drho_ji + R.dF[C.off + j] * drho_ij) * r_inv;
-            fx += fpair * dx;
-            fy += fpair * dy;
-            fz += fpair * dz;
+        for (int k0 = g * B; k0 < cnt; k0 += G * B) {
+            uint32_t e[B];
+            double4 xj[B], cz[B], ca[B], cb[B];
+            double dx[B], dy[B], dz[B], p[B], ri[B], dFj[B];
+            bool in[B];
+            fetch<B>(C, R, i, cnt, k0, e, xj);
+            for (int b = 0; b < B; ++b) {
+                const int ej = (int)xj[b].w;
+                double r;
+                dFj[b] = R.dF[C.off + (int)(e[b] & kIndexMask)];
+                image_dx(shift, xi, xj[b], e[b] >> kIndexBits, dx[b], dy[b], dz[b]);
+                const double rsq = dx[b] * dx[b] + (dy[b] * dy[b] + dz[b] * dz[b]);
+                in[b] = k0 + b < cnt && rsq < C.S->cut_sq[ei * ne + ej];
+                int m;
+                root_inv(in[b] ? rsq : 1.0, r, ri[b]);
+                spline_at(r, A.dr_inv, nr, m, p[b]);
+                cz[b] = A.phi[(size_t)(ei * ne + ej) * nr + m];
+                ca[b] = A.rho[(size_t)(ej * ne + ei) * nr + m];
+                cb[b] = A.rho[(size_t)(ei * ne + ej) * nr + m];
+            }
+            for (int b = 0; b < B; ++b) {
+                const double phi = hval(cz[b], p[b]) * ri[b];
+                const double dphi = (dhval(cz[b], p[b]) * A.dr_inv - phi) * ri[b];
+                const double drho_ji = dhval(ca[b], p[b]) * A.dr_inv;
+                const double drho_ij = dhval(cb[b], p[b]) * A.dr_inv;
+                const double u = -(dphi + dFi * drho_ji + dFj[b] * drho_ij) * ri[b];
+                fx += in[b] ? u * dx[b] : 0.0;
+                fy += in[b] ? u * dy[b] : 0.0;
+                fz += in[b] ? u * dz[b] : 0.0;
+            }
         }
-        R.f[C.off + i] = make_double4(fx, fy, fz, 0.0);
+        for (int o = 1; o < G; o <<= 1) {
+            fx += __shfl_xor(fx, o, 64);
+            fy += __shfl_xor(fy, o, 64);
+            fz += __shfl_xor(fz, o, 64);
+        }
+        if (own && g == 0) R.f[C.off + i] = make_double4(fx, fy, fz, 0.0);
     }
     group_sync<W>();
-    return en;
 }
 
 // MinMDHandler::F(alpha) / F_reset: x = x0 + alpha h, the skin check of
 // DynamicMD::update (a rebuild when any atom moved more than skin / 2 since
 // the last build), then the energy
 template <int W>
-__device__ double trial(const RepArgs& A, const Ctx& C, const RepArrays& R, double alpha, bool energy, int& builds,
-                        int& fail, double* red, int w)
+__device__ double trial(const RepArgs& A, Ctx& C, const RepArrays& R, double alpha, bool energy, int& builds, int& fail)
 {
     double moved = 0.0;
     for (int i = C.t; i < C.n; i += C.nt) {
@@ -287,14 +502,13 @@ __device__ double trial(const RepArgs& A, const Ctx& C, const RepArrays& R, doub
         const double d0 = x.x - b.x, d1 = x.y - b.y, d2 = x.z - b.z;
         moved = fmax(moved, d0 * d0 + (d1 * d1 + d2 * d2));
     }
-    moved = group_max<W>(moved, red, w);
-    group_sync<W>();
+    moved = group_max<W>(moved, C);
     if (moved > A.skin_sq4) {
-        fail = build_list<W>(A, C, R, red, w);
+        fail = build_list<W>(A, C, R);
         ++builds;
     }
     if (!energy || fail) return 0.0;
-    return eam_energy<W>(A, C, R, false, red, w);
+    return eam_energy<W>(A, C, R);
 }
 
 // One replica, the whole MinCG::__run on W waves (w = this wave's index in
@@ -303,7 +517,7 @@ __device__ double trial(const RepArgs& A, const Ctx& C, const RepArrays& R, doub
 // group sums that every lane receives alike, and every lane stores the
 // results alike.
 template <int W>
-__device__ void run_rep(const RepArgs& A, RepCell* __restrict__ cells, int r, const RepArrays& R, double* red, int w,
+__device__ void run_rep(const RepArgs& A, RepCell* __restrict__ cells, int r, const RepArrays& R, Shared& S, int w,
                         int lane)
 {
     Ctx C;
@@ -322,13 +536,35 @@ __device__ void run_rep(const RepArgs& A, RepCell* __restrict__ cells, int r, co
         for (int d = 0; d < 3; ++d) C.cs[d] = uni(hd.cs[d]);
     }
     C.nt = 64 * W;
+    C.w = w;
     C.t = W == 1 ? lane : w * 64 + lane;
+    C.flip = 0;
+    C.S = &S;
+    // lanes per atom: the fewest rounds of a pass over about 70 entries in
+    // batches of 4, with the constant work of a round (its loads and sums)
+    // taken as 8 entries
+    C.lg = 0;
+    for (int lg = 1, best = ((C.n + C.nt - 1) / C.nt) * 80; lg <= 4; ++lg) {
+        const int cost = (((C.n << lg) + C.nt - 1) / C.nt) * (((72 >> lg) + 3) / 4 * 4 + 8 + 2 * lg);
+        if (cost < best) {
+            best = cost;
+            C.lg = lg;
+        }
+    }
+    for (int c = C.t; c < kShifts; c += C.nt) {
+        const int n2 = c / 25 - 2, n1 = c % 25 / 5 - 2, n0 = c % 5 - 2;
+        double* sh = S.shift[W == 1 ? w : 0][c];
+        sh[0] = C.h[0] * n0 + C.h[1] * n1 + C.h[2] * n2;
+        sh[1] = C.h[3] * n1 + C.h[4] * n2;
+        sh[2] = C.h[5] * n2;
+    }
     int builds = 1, evals = 0;
-    int fail = build_list<W>(A, C, R, red, w);
+    int fail = build_list<W>(A, C, R);
     double e_curr = 0.0, e0 = 0.0;
     int err = LS_S, istep = 0;
     if (!fail) {
-        e_curr = eam_energy<W>(A, C, R, true, red, w);
+        e_curr = eam_energy<W>(A, C, R);
+        eam_force<W>(A, C, R);
         ++evals;
         e0 = e_curr;
         double ff = 0.0;
@@ -337,7 +573,7 @@ __device__ void run_rep(const RepArgs& A, RepCell* __restrict__ cells, int r, co
             R.h[C.off + i] = f;
             ff += f.x * f.x + (f.y * f.y + f.z * f.z);
         }
-        double f0_f0 = group_sum<W>(ff, red, w);
+        double f0_f0 = group_sum<W>(ff, C);
         err = A.max_nsteps == 0 ? MIN_F_MAX_ITER : LS_S;
         double prev_val = -1.0;  // LineSearchBackTrack's memory (init_flag 1)
         while (err == LS_S) {
@@ -354,7 +590,7 @@ __device__ void run_rep(const RepArgs& A, RepCell* __restrict__ cells, int r, co
                 fh += f.x * hh.x + (f.y * hh.y + f.z * hh.z);
             }
             const double e_prev = e_curr;
-            double f_h = group_sum<W>(fh, red, w);
+            double f_h = group_sum<W>(fh, C);
             if (f_h < 0.0) {
                 for (int i = C.t; i < C.n; i += C.nt) R.h[C.off + i] = R.f[C.off + i];
                 f_h = f0_f0;
@@ -367,8 +603,8 @@ __device__ void run_rep(const RepArgs& A, RepCell* __restrict__ cells, int r, co
                 hh2 += hh.x * hh.x + (hh.y * hh.y + hh.z * hh.z);
                 hmax = fmax(hmax, fmax(fabs(hh.x), fmax(fabs(hh.y), fabs(hh.z))));
             }
-            const double h_norm = group_sum<W>(hh2, red, w);
-            hmax = group_max<W>(hmax, red, w);
+            const double h_norm = group_sum<W>(hh2, C);
+            hmax = group_max<W>(hmax, C);
             double dfa = -f_h, max_a;
             if (h_norm == 0.0) {
                 dfa = 0.0;
@@ -394,7 +630,7 @@ __device__ void run_rep(const RepArgs& A, RepCell* __restrict__ cells, int r, co
                     double alpha = max_a;
                     while (true) {
                         const double ideal = e_curr + alpha * A.ls_c * dfa;
-                        const double cur = trial<W>(A, C, R, alpha, true, builds, fail, red, w);
+                        const double cur = trial<W>(A, C, R, alpha, true, builds, fail);
                         ++evals;
                         if (fail) break;
                         if (cur <= ideal) {
@@ -404,7 +640,7 @@ __device__ void run_rep(const RepArgs& A, RepCell* __restrict__ cells, int r, co
                         }
                         alpha *= A.ls_rho;
                         if (alpha <= A.ls_min_alpha || alpha != alpha) {
-                            trial<W>(A, C, R, 0.0, false, builds, fail, red, w);  // F_reset
+                            trial<W>(A, C, R, 0.0, false, builds, fail);  // F_reset
                             err = LS_MIN_ALPHA;
                             break;
                         }
@@ -413,7 +649,8 @@ __device__ void run_rep(const RepArgs& A, RepCell* __restrict__ cells, int r, co
             }
             if (fail) break;
             if (err != LS_S) continue;
-            eam_energy<W>(A, C, R, true, red, w);  // force_calc at the accepted point
+            // force_calc at the accepted point, whose density pass was the trial's
+            eam_force<W>(A, C, R);
             ++evals;
             if (e_prev - e_curr < A.e_tol) err = MIN_S_TOLERANCE;
             if (istep + 1 == A.max_nsteps) err = MIN_F_MAX_ITER;
@@ -427,8 +664,8 @@ __device__ void run_rep(const RepArgs& A, RepCell* __restrict__ cells, int r, co
                 s_ff += f.x * f.x + (f.y * f.y + f.z * f.z);
                 s_ff0 += f.x * g.x + (f.y * g.y + f.z * g.z);
             }
-            const double f_f = group_sum<W>(s_ff, red, w);
-            const double f_f0 = group_sum<W>(s_ff0, red, w);
+            const double f_f = group_sum<W>(s_ff, C);
+            const double f_f0 = group_sum<W>(s_ff0, C);
             const double ratio = (f_f - f_f0) / f0_f0;
             for (int i = C.t; i < C.n; i += C.nt) {
                 const double4 hh = R.h[C.off + i], f = R.f[C.off + i];
@@ -445,7 +682,7 @@ __device__ void run_rep(const RepArgs& A, RepCell* __restrict__ cells, int r, co
             const double4 f = R.f[C.off + i];
             fm = fmax(fm, fmax(fabs(f.x), fmax(fabs(f.y), fabs(f.z))));
         }
-    fm = group_max<W>(fm, red, w);
+    fm = group_max<W>(fm, C);
     if (w == 0 || W == 1) {
         RepCell& o = cells[r];
         o.status = fail ? fail : err;
@@ -458,34 +695,38 @@ __device__ void run_rep(const RepArgs& A, RepCell* __restrict__ cells, int r, co
     }
 }
 
-// Persistent launch: workgroups first take the four-wave replicas (largest
-// first) from queue[0]; then each wave takes one-wave replicas from queue[1]
-// on its own. Every lane of a wave joins the queue atomic (lane 0 adds 1, the
-// others 0) and the ticket is read from the first lane, so the replica index
-// is wave-uniform.
-__global__ __launch_bounds__(256) void k_replica_cg(RepArgs A, RepCell* cells, const int* __restrict__ q4, int n4,
-                                                    const int* __restrict__ q1, int n1, int* queue, RepArrays R)
+// Persistent launch: workgroups first take the replicas that a whole
+// workgroup owns (largest first) from queue[0]; then each wave takes one-wave
+// replicas from queue[1] on its own. Every lane of a wave joins the queue
+// atomic (lane 0 adds 1, the others 0) and the ticket is read from the first
+// lane, so the replica index is wave-uniform.
+__global__ __launch_bounds__(64 * kWide) void k_replica_cg(RepArgs A, RepCell* cells, const int* __restrict__ q4,
+                                                           int n4, const int* __restrict__ q1, int n1, int* queue,
+                                                           RepArrays R)
 {
-    __shared__ double red[8];
-    __shared__ int next_sh;
+    __shared__ Shared S;
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (int k = threadIdx.x; k < A.ne * A.ne; k += 64 * kWide) {
+        S.cut_sq[k] = A.cut_sq[k];
+        S.cutsk_sq[k] = A.cutsk_sq[k];
+    }
     while (true) {
         if (w == 0) {
             const int t = __builtin_amdgcn_readfirstlane(atomicAdd(&queue[0], lane == 0 ? 1 : 0));
-            next_sh = t;
+            S.next = t;
         }
         __syncthreads();
-        const int t = __builtin_amdgcn_readfirstlane(next_sh);
+        const int t = __builtin_amdgcn_readfirstlane(S.next);
         __syncthreads();
         if (t >= n4) break;
-        run_rep<4>(A, cells, q4[t], R, red, w, lane);
+        run_rep<kWide>(A, cells, q4[t], R, S, w, lane);
         __syncthreads();
     }
     while (true) {
         const int t = __builtin_amdgcn_readfirstlane(atomicAdd(&queue[1], lane == 0 ? 1 : 0));
         if (t >= n1) break;
-        run_rep<1>(A, cells, q1[t], R, nullptr, 0, lane);
+        run_rep<1>(A, cells, q1[t], R, S, w, lane);
     }
 }
 
@@ -589,6 +830,9 @@ ReplicaBatch::ReplicaBatch(std::shared_ptr<EamForceField> ff, int nrep, const in
     f0_.reserve(natot_);
     dF_.reserve(natot_);
     nn_.reserve(natot_);
+    cid_.reserve(natot_);
+    ord_.reserve(natot_);
+    cand_.reserve(27 * natot_);
     list_.reserve(ltot_);
     queue_.reserve(2);
     {
@@ -612,7 +856,7 @@ ReplicaBatch::ReplicaBatch(std::shared_ptr<EamForceField> ff, int nrep, const in
     int dev = 0, ncu = 0, per = 0;
     MAPP_HIP(hipGetDevice(&dev));
     MAPP_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-    MAPP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_replica_cg, 256, 0));
+    MAPP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_replica_cg, 64 * kWide, 0));
     grid_ = std::max(1, ncu * std::max(1, per));
 }
 
@@ -659,10 +903,11 @@ void ReplicaBatch::build_queues(const int* waves, DevBuf<int>& q4, int& n4, DevB
 
 void ReplicaBatch::launch(State& st, const RepArgs& A, const int* q4, int n4, const int* q1, int n1)
 {
-    RepArrays R{st.x.get(), x0_.get(), xb_.get(), h_.get(), f_.get(), f0_.get(), dF_.get(), list_.get(), nn_.get()};
+    RepArrays R{st.x.get(), x0_.get(), xb_.get(), h_.get(), f_.get(), f0_.get(), dF_.get(), list_.get(), nn_.get(),
+                cid_.get(), ord_.get(), cand_.get()};
     k_replica_reset<<<1, 64, 0, stream_>>>(queue_.get());
-    const int blocks = std::max(1, std::min(grid_, std::max(n4, (n1 + 3) / 4)));
-    k_replica_cg<<<blocks, 256, 0, stream_>>>(A, st.cells.get(), q4, n4, q1, n1, queue_.get(), R);
+    const int blocks = std::max(1, std::min(grid_, std::max(n4, (n1 + kWide - 1) / kWide)));
+    k_replica_cg<<<blocks, 64 * kWide, 0, stream_>>>(A, st.cells.get(), q4, n4, q1, n1, queue_.get(), R);
     MAPP_HIP(hipGetLastError());
 }
 

@@ -97,3 +97,4 @@ using std::min;
 inline int __builtin_amdgcn_readfirstlane(int v) { return __shfl(v, 0, 64); }
 inline long long __double_as_longlong(double d) { long long b; memcpy(&b, &d, 8); return b; }
 inline double __longlong_as_double(long long b) { double d; memcpy(&d, &b, 8); return d; }
+inline double __builtin_amdgcn_rsq(double x) { return 1.0 / std::sqrt(x); }

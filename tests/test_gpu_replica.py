@@ -133,3 +133,27 @@ def test_rejects_a_box_thinner_than_the_cutoff(M):
     x, H = pot.fcc(3.615, (1, 3, 3))
     with pytest.raises(M.MappError, match="thinner than r_c"):
         M.ReplicaBatch(M.ForceFieldEAM.from_knots(p), [(H, x, np.zeros(len(x), np.uint8))])
+
+
+@pytest.mark.parametrize("shape", [(6, 6, 6), (6, 7, 9), (4, 6, 11)])
+@pytest.mark.parametrize("waves", [1, 4])
+def test_cells_of_the_list_build(M, shape, waves):
+    # boxes of at least three build cells along each vector, one of fewer along
+    # the shortest, atoms on the box faces (they cross while they are moved), a
+    # round that is not full, and three elements
+    rng = np.random.default_rng(sum(shape))
+    x, H = pot.fcc(3.52, shape)
+    h = np.argwhere(np.ones(shape, bool))[rng.choice(int(np.prod(shape)), 9, replace=False)] * 3.52
+    x = np.concatenate([x + rng.normal(0.0, 0.1, x.shape), h + np.array([1.76, 0.0, 0.0])])
+    elem = np.zeros(len(x), np.uint8)
+    elem[len(x) - 9:] = 2
+    elem[:5] = 1
+    ro, xo = oracle_min(O.OEam.read(pot.NIALH_JEA), H, x, elem)
+    b = M.ReplicaBatch(M.ForceFieldEAM.setfl(pot.NIALH_JEA), [(H, x, elem)], skin=0.5)
+    b.set_waves([waves] * 5)
+    res = b.min_cg(NSTEPS, e_tol=0.0, max_dx=1.0)
+    # FP64 sums in another order, as in check()
+    assert res["status"][0] == ro["status"] and res["steps"][0] == ro["steps"]
+    assert abs(res["e0"][0] - ro["e0"]) < 1e-10 * abs(ro["e0"])
+    assert abs(res["e"][0] - ro["e"]) < 1e-10 * abs(ro["e"])
+    assert wrapped_diff(b.x(0), xo, H) < 1e-7
