@@ -65,6 +65,29 @@ struct DevBuf {
     T* get() const { return p; }
 };
 
+// Pinned host memory that kernels can write.
+template <class T>
+struct HostBuf {
+    T* p = nullptr;
+    size_t n = 0;
+    HostBuf() = default;
+    HostBuf(const HostBuf&) = delete;
+    HostBuf& operator=(const HostBuf&) = delete;
+    ~HostBuf()
+    {
+        if (p) (void)hipHostFree(p);
+    }
+    void reserve(size_t count)
+    {
+        if (count <= n && p) return;
+        if (p) (void)hipHostFree(p);
+        p = nullptr;
+        MAPP_HIP(hipHostMalloc((void**)&p, (count ? count : 1) * sizeof(T), 0));
+        n = count;
+    }
+    T* get() const { return p; }
+};
+
 constexpr int kWave = 64;
 
 // Per-kernel timing with HIP events recorded on the stream the kernels run

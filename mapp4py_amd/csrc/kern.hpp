@@ -23,24 +23,73 @@ __device__ inline int xcd_block()
     return (blockIdx.x % kXcd) * q + blockIdx.x / kXcd;
 }
 
-// K FP64 sums over a workgroup of NT threads, written as one row of kPartW
-template <int K, int NT = kBlock>
-__device__ inline void block_sum_store(double (&v)[K], double* out)
+// P sums (a power of two) over the 64 lanes of a wave, in a fixed order: lanes
+// a bit apart each keep half of the values and give the other half away, until
+// one is left, so 8 values take 4 + 2 + 1 + 3 exchanges instead of 48. Lane l
+// (l < P) ends with the sum of value lane_value<P>(l) in v[0].
+template <int P, class T>
+__device__ inline void wave_sums(T (&v)[P])
 {
-    for (int off = 32; off > 0; off >>= 1)
-        for (int k = 0; k < K; ++k) v[k] += __shfl_xor(v[k], off, 64);
-    __shared__ double sh[NT / 64][K];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    if (lane == 0)
-        for (int k = 0; k < K; ++k) sh[w][k] = v[k];
-    __syncthreads();
-    // the whole row is written (zeros past K) so any column count can be reduced
-    if (threadIdx.x < kPartW) {
-        double s = 0.0;
-        if ((int)threadIdx.x < K)
-            for (int q = 0; q < NT / 64; ++q) s += sh[q][threadIdx.x];
-        out[threadIdx.x] = s;
+    const int lane = threadIdx.x & 63;
+    int off = 1;
+#pragma unroll
+    for (int half = P / 2; half > 0; half /= 2, off *= 2) {
+        const bool up = (lane & off) != 0;
+#pragma unroll
+        for (int k = 0; k < half; ++k) {
+            const T a = v[k], b = v[k + half];
+            const T keep = up ? b : a, give = up ? a : b;
+            v[k] = keep + __shfl_xor(give, off, 64);
+        }
     }
+#pragma unroll
+    for (; off < 64; off *= 2) v[0] += __shfl_xor(v[0], off, 64);
+}
+template <int P>
+__device__ inline int lane_value(int l)
+{
+    int k = 0;
+#pragma unroll
+    for (int half = P / 2, off = 1; half > 0; half /= 2, off *= 2) k += (l & off) ? half : 0;
+    return k;
+}
+
+// wave_sums of K (at most 8) values that start at v[O], to row[O ..]
+template <int O, int K, int N>
+__device__ inline void wave_sums_to(const double (&v)[N], double* row)
+{
+    constexpr int P = K <= 1 ? 1 : K <= 2 ? 2 : K <= 4 ? 4 : 8;
+    double t[P];
+#pragma unroll
+    for (int k = 0; k < P; ++k) t[k] = v[O + (k < K ? k : 0)];
+    wave_sums<P>(t);
+    const int lane = threadIdx.x & 63, k = lane_value<P>(lane);
+    if (lane < P && k < K) row[O + k] = t[0];
+}
+
+// K FP64 sums over a workgroup of NT threads: thread k < K returns the k-th
+// (the others 0)
+template <int K, int NT = kBlock>
+__device__ inline double block_sums(const double (&v)[K])
+{
+    __shared__ double sh[NT / 64][K];
+    double* row = sh[threadIdx.x >> 6];
+    wave_sums_to<0, (K < 8 ? K : 8)>(v, row);
+    if constexpr (K > 8) wave_sums_to<8, K - 8>(v, row);
+    __syncthreads();
+    double s = 0.0;
+    if ((int)threadIdx.x < K)
+        for (int q = 0; q < NT / 64; ++q) s += sh[q][threadIdx.x];
+    return s;
+}
+
+// the same, written as one row of kPartW (zeros past K, so that any column
+// count can be reduced)
+template <int K, int NT = kBlock>
+__device__ inline void block_sum_store(const double (&v)[K], double* out)
+{
+    const double s = block_sums<K, NT>(v);
+    if (threadIdx.x < kPartW) out[threadIdx.x] = s;
 }
 
 // Fixed-order reduction of rows of partial sums: out[k] = sum_r part[r*W + k].

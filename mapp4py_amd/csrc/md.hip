@@ -39,6 +39,10 @@ struct GridArgs {
     // every pair the record quantisation could misplace)
     double rec_in_sq[kMaxElems * kMaxElems], rec_out_sq[kMaxElems * kMaxElems];
 };
+// flags: the largest row of a list build that overflowed, an atom moved half
+// the skin, a run's steps are halted there, steps a run has finished
+enum { FL_OVER = 0, FL_REBUILD = 1, FL_HALT = 2, FL_DONE = 3 };
+
 // ---------------- neighbor build ----------------
 
 // wrap into the box, remember s, sort key = Morton rank of the cell
@@ -243,7 +247,7 @@ __global__ __launch_bounds__(kBlock) void k_build_list(int n, const double4* __r
     // the last, partly filled block (its entries past cnt are never read)
     if ((cnt & 3) != 0 && (cnt >> 2) < maxb) list4[(size_t)(cnt >> 2) * ldl + i] = make_uint4(p0, p1, p2, p3);
     nn[i] = cnt;
-    if (cnt > 4 * maxb) atomicMax(&flags[0], cnt);
+    if (cnt > 4 * maxb) atomicMax(&flags[FL_OVER], cnt);
 }
 
 // ---------------- EAM ----------------
@@ -397,16 +401,36 @@ __global__ __launch_bounds__(kBlock) void k_make_records(int n, const double4* _
                         (unsigned)__double2ll_rn(xi.z * R.inv_q), (unsigned)(int)xi.w);
 }
 
+// Lanes sharing an atom: 2^lg neighboring lanes take the batches of its row
+// in turn and meet in a butterfly, so that a small system still fills the
+// chip (one lane an atom leaves most CUs without work below 262,144 atoms).
+// Every lane of the group ends with the same sum.
+template <class T>
+__device__ inline T lane_sum(T v, int lg)
+{
+    for (int o = 1; o < (1 << lg); o <<= 1) v += __shfl_xor(v, o, 64);
+    return v;
+}
+
+// The lanes take the entries in blocks of 4 whatever the batch length B is, so
+// the sums do not depend on it: entry after k0's batch of a lane.
+template <int B>
+__device__ inline int next_batch(int k0, int lg)
+{
+    return k0 + B + (B >= 4 || ((k0 + B) & 3) == 0 ? (4 << lg) - 4 : 0);
+}
+
 // pass 1 per atom: rho_i = sum_j rho_{j->i}(r_ij), an FP64 sum of FP32 spline
-// values. Tab supplies the spline rows (global table or an LDS window).
+// values, over the batches of lane g of the 2^lg that share the atom. Tab
+// supplies the spline rows (global table or an LDS window).
 template <int B, bool ONE, class Tab>
 __device__ inline double rho_atom(int i, const uint4& ri, int cnt, const uint4* __restrict__ rec,
                                   const uint4* __restrict__ list4, int ldl, int maxb, const EamArgs& P,
-                                  const Rec16Frame& R, const Tab& T)
+                                  const Rec16Frame& R, const Tab& T, int lg, int g)
 {
     const int ti = ONE ? 0 : (int)ri.w;
     double rho = 0.0;
-    for (int k0 = 0; k0 < cnt; k0 += B) {
+    for (int k0 = 4 * g; k0 < cnt; k0 = next_batch<B>(k0, lg)) {
         uint32_t e[B];
         uint4 rj[B];
         int row[B];
@@ -482,14 +506,14 @@ template <int B, bool ONE, bool EV, class Tab>
 __device__ inline void force_atom(int i, const uint4& ri, int ti, float dFi, int cnt, const uint4* __restrict__ rec,
                                   const uint4* __restrict__ xr, const float* __restrict__ dF,
                                   const uint4* __restrict__ list4, int ldl, int maxb, const EamArgs& P,
-                                  const Rec16Frame& R, const Tab& T, float& fx, float& fy, float& fz,
-                                  double (&ev)[7])
+                                  const Rec16Frame& R, const Tab& T, int lg, int g0, float& fx, float& fy,
+                                  float& fz, double (&ev)[7])
 {
     // the list entries of the next batch are loaded one batch ahead (this
     // pass's batches are short, so one memory round trip less per batch pays)
     uint32_t en[B];
-    list_entries<B>(list4, ldl, maxb, 0, i, cnt, en);
-    for (int k0 = 0; k0 < cnt; k0 += B) {
+    list_entries<B>(list4, ldl, maxb, 4 * g0, i, cnt, en);
+    for (int k0 = 4 * g0; k0 < cnt; k0 = next_batch<B>(k0, lg)) {
         uint32_t e[B];
         uint4 rj[B];
         float dFj[B];
@@ -508,7 +532,7 @@ __device__ inline void force_atom(int i, const uint4& ri, int ti, float dFi, int
                 dFj[b] = dF[j];
             }
         }
-        list_entries<B>(list4, ldl, maxb, k0 + B, i, cnt, en);
+        list_entries<B>(list4, ldl, maxb, next_batch<B>(k0, lg), i, cnt, en);
         const bool any_img = wave_has_image(e);
 #pragma unroll
         for (int b = 0; b < B; ++b) {
@@ -638,40 +662,57 @@ __device__ inline void kick_atom(int i, int ti, float fx, float fy, float fz, co
     fm[2] += (double)fz / m;
 }
 
-// pass 1 (one thread per atom, 256-thread workgroups): rho_i, F(rho_i) and
-// F'(rho_i); embedding energy reduced per workgroup. With one element,
-// F'(rho_i) goes into the fourth word of the pass-2 record (xr); otherwise
-// into dF.
+// the workgroup's rows of the kick's sums
+template <int NT>
+__device__ inline void kick_rows(const double (&mvv)[6], const double (&fm)[3], double* row_mvv, double* row_fm)
+{
+    const double v[9] = {mvv[0], mvv[1], mvv[2], mvv[3], mvv[4], mvv[5], fm[0], fm[1], fm[2]};
+    const double s = block_sums<9, NT>(v);
+    if (threadIdx.x < 6) row_mvv[threadIdx.x] = s;
+    else if (threadIdx.x < 9) row_fm[threadIdx.x - 6] = s;
+}
+
+// pass 1 (2^lg lanes per atom, 256-thread workgroups, global tables): rho_i,
+// F(rho_i) and F'(rho_i); embedding energy reduced per workgroup. With one
+// element, F'(rho_i) goes into the fourth word of the pass-2 record (xr);
+// otherwise into dF. stop: nothing is done where it is set (a run's steps are
+// launched ahead of the skin check's answer).
 template <int B, bool ONE>
-__global__ __launch_bounds__(kBlock) void k_eam_rho(int n, const uint4* __restrict__ rec, const int* __restrict__ nn,
+__global__ __launch_bounds__(kBlock) void k_eam_rho(int n, int lg, const int* __restrict__ stop,
+                                                    const uint4* __restrict__ rec, const int* __restrict__ nn,
                                                     const uint4* __restrict__ list4, int ldl, int maxb, EamArgs P,
                                                     Rec16Frame R, double* __restrict__ rho_out,
                                                     uint4* __restrict__ xr, float* __restrict__ dF_out,
                                                     double* __restrict__ part)
 {
+    if (stop && *stop) return;
     const int blk = xcd_block();
-    const int i = blk * kBlock + threadIdx.x;
+    const int i = (int)(((long)blk * kBlock + threadIdx.x) >> lg), g = threadIdx.x & ((1 << lg) - 1);
     double acc[1] = {0.0};
     if (i < n) {
         const uint4 ri = rec[i];
         const int ti = ONE ? 0 : (int)ri.w;
-        const double rho = rho_atom<B, ONE>(i, ri, nn[i], rec, list4, ldl, maxb, P, R, RhoRowsGlobal{P.tabA});
-        double F, dF;
-        embed(P, ti, rho, F, dF);
-        rho_out[i] = rho;
-        if (ONE)
-            xr[i] = make_uint4(ri.x, ri.y, ri.z, __float_as_uint((float)dF));
-        else
-            dF_out[i] = (float)dF;
-        acc[0] = F;
+        const double rho = lane_sum(
+            rho_atom<B, ONE>(i, ri, nn[i], rec, list4, ldl, maxb, P, R, RhoRowsGlobal{P.tabA}, lg, g), lg);
+        if (g == 0) {
+            double F, dF;
+            embed(P, ti, rho, F, dF);
+            rho_out[i] = rho;
+            if (ONE)
+                xr[i] = make_uint4(ri.x, ri.y, ri.z, __float_as_uint((float)dF));
+            else
+                dF_out[i] = (float)dF;
+            acc[0] = F;
+        }
     }
     block_sum_store<1>(acc, part + (size_t)blk * kPartW);
 }
 
-// pass 2 (one thread per atom, 256-thread workgroups) with the fused second
+// pass 2 (2^lg lanes per atom, 256-thread workgroups) with the fused second
 // half kick when K.on; energy and virial partials only with EV
 template <int B, bool ONE, bool EV>
-__global__ __launch_bounds__(kBlock) void k_eam_force(int n, const uint4* __restrict__ rec,
+__global__ __launch_bounds__(kBlock) void k_eam_force(int n, int lg, const int* __restrict__ stop,
+                                                      const uint4* __restrict__ rec,
                                                       const uint4* __restrict__ xr, const float* __restrict__ dF,
                                                       Rec16Frame R, const int* __restrict__ nn,
                                                       const uint4* __restrict__ list4, int ldl, int maxb, EamArgs P,
@@ -679,8 +720,9 @@ __global__ __launch_bounds__(kBlock) void k_eam_force(int n, const uint4* __rest
                                                       KickArgs K, double4* __restrict__ v,
                                                       double* __restrict__ part_mvv, double* __restrict__ part_cv)
 {
+    if (stop && *stop) return;
     const int blk = xcd_block();
-    const int i = blk * kBlock + threadIdx.x;
+    const int i = (int)(((long)blk * kBlock + threadIdx.x) >> lg), g = threadIdx.x & ((1 << lg) - 1);
     double acc[7] = {0, 0, 0, 0, 0, 0, 0};
     double mvv[6] = {0, 0, 0, 0, 0, 0};
     double fm[3] = {0, 0, 0};
@@ -690,9 +732,14 @@ __global__ __launch_bounds__(kBlock) void k_eam_force(int n, const uint4* __rest
         const float dFi = ONE ? __uint_as_float(ri.w) : dF[i];
         float fx = 0.f, fy = 0.f, fz = 0.f;
         force_atom<B, ONE, EV>(i, ri, ti, dFi, nn[i], rec, xr, dF, list4, ldl, maxb, P, R,
-                               ForceRowsGlobal<ONE>{ONE ? P.tabC : P.tabB}, fx, fy, fz, acc);
-        f_out[i] = make_float4(fx, fy, fz, 0.f);
-        if (K.on) kick_atom(i, ti, fx, fy, fz, K, v, mvv, fm);
+                               ForceRowsGlobal<ONE>{ONE ? P.tabC : P.tabB}, lg, g, fx, fy, fz, acc);
+        fx = lane_sum(fx, lg);
+        fy = lane_sum(fy, lg);
+        fz = lane_sum(fz, lg);
+        if (g == 0) {
+            f_out[i] = make_float4(fx, fy, fz, 0.f);
+            if (K.on) kick_atom(i, ti, fx, fy, fz, K, v, mvv, fm);
+        }
     }
     if (EV) {
         // half of each full-list pair: energy phi / 2, virial (q/2) u dx dy
@@ -703,9 +750,7 @@ __global__ __launch_bounds__(kBlock) void k_eam_force(int n, const uint4* __rest
     }
     if (K.on) {
         if (EV) __syncthreads();
-        block_sum_store<6>(mvv, part_mvv + (size_t)blk * kPartW);
-        __syncthreads();
-        block_sum_store<3>(fm, part_cv + (size_t)blk * kPartW);
+        kick_rows<kBlock>(mvv, fm, part_mvv + (size_t)blk * kPartW, part_cv + (size_t)blk * kPartW);
     }
 }
 
@@ -721,9 +766,10 @@ constexpr int kBigBlock = 1024;
 struct ChunkWalk {
     int c, end, step;
 };
-__device__ inline ChunkWalk chunk_walk(int n)
+// chunks of `size` atoms
+__device__ inline ChunkWalk chunk_walk(int n, int size)
 {
-    const int nchunks = (n + kBigBlock - 1) / kBigBlock;
+    const int nchunks = (n + size - 1) / size;
     const int per = (nchunks + kXcd - 1) / kXcd;
     const int x = blockIdx.x % kXcd;
     ChunkWalk w;
@@ -734,7 +780,8 @@ __device__ inline ChunkWalk chunk_walk(int n)
 }
 
 template <int B>
-__global__ __launch_bounds__(kBigBlock) void k_eam_rho_lds(int n, const uint4* __restrict__ rec,
+__global__ __launch_bounds__(kBigBlock) void k_eam_rho_lds(int n, int lg, const int* __restrict__ stop,
+                                                           const uint4* __restrict__ rec,
                                                            const int* __restrict__ nn,
                                                            const uint4* __restrict__ list4, int ldl, int maxb,
                                                            EamArgs P, Rec16Frame R, int m_lo, int nwin,
@@ -742,15 +789,25 @@ __global__ __launch_bounds__(kBigBlock) void k_eam_rho_lds(int n, const uint4* _
                                                            double* __restrict__ part)
 {
     extern __shared__ float4 lds_rows[];
-    for (int r = threadIdx.x; r < nwin; r += kBigBlock) lds_rows[r] = P.tabA[m_lo + r];
+    for (int r0 = threadIdx.x; r0 < nwin; r0 += 5 * kBigBlock) {
+        float4 t[5];
+#pragma unroll
+        for (int q = 0; q < 5; ++q) t[q] = P.tabA[m_lo + min(r0 + q * kBigBlock, nwin - 1)];
+#pragma unroll
+        for (int q = 0; q < 5; ++q)
+            if (r0 + q * kBigBlock < nwin) lds_rows[r0 + q * kBigBlock] = t[q];
+    }
     __syncthreads();
+    if (stop && *stop) return;
     const RhoRowsLds T{P.tabA, lds_rows, m_lo};
+    const int g = threadIdx.x & ((1 << lg) - 1), size = kBigBlock >> lg;
     double acc[1] = {0.0};
-    for (ChunkWalk w = chunk_walk(n); w.c < w.end; w.c += w.step) {
-        const int i = w.c * kBigBlock + threadIdx.x;
+    for (ChunkWalk w = chunk_walk(n, size); w.c < w.end; w.c += w.step) {
+        const int i = w.c * size + (threadIdx.x >> lg);
         if (i >= n) continue;
         const uint4 ri = rec[i];
-        const double rho = rho_atom<B, true>(i, ri, nn[i], rec, list4, ldl, maxb, P, R, T);
+        const double rho = lane_sum(rho_atom<B, true>(i, ri, nn[i], rec, list4, ldl, maxb, P, R, T, lg, g), lg);
+        if (g != 0) continue;
         double F, dF;
         embed(P, 0, rho, F, dF);
         rho_out[i] = rho;
@@ -761,7 +818,8 @@ __global__ __launch_bounds__(kBigBlock) void k_eam_rho_lds(int n, const uint4* _
 }
 
 template <int B, bool EV>
-__global__ __launch_bounds__(kBigBlock) void k_eam_force_lds(int n, const uint4* __restrict__ xr, Rec16Frame R,
+__global__ __launch_bounds__(kBigBlock) void k_eam_force_lds(int n, int lg, const int* __restrict__ stop,
+                                                             const uint4* __restrict__ xr, Rec16Frame R,
                                                              const int* __restrict__ nn,
                                                              const uint4* __restrict__ list4, int ldl, int maxb,
                                                              EamArgs P, int m_lo, int nwin,
@@ -773,24 +831,42 @@ __global__ __launch_bounds__(kBigBlock) void k_eam_force_lds(int n, const uint4*
     extern __shared__ float4 lds_rows[];
     float2* w2 = (float2*)(lds_rows + nwin);
     float* w1 = (float*)(w2 + nwin);
-    for (int r = threadIdx.x; r < nwin; r += kBigBlock) {
-        const float4 a = P.tabC[(size_t)(m_lo + r) * 2], c = P.tabC[(size_t)(m_lo + r) * 2 + 1];
-        lds_rows[r] = a;
-        w2[r] = make_float2(c.x, c.y);
-        w1[r] = c.z;
+    for (int r0 = threadIdx.x; r0 < nwin; r0 += 3 * kBigBlock) {
+        float4 a[3], c[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const size_t r = m_lo + min(r0 + q * kBigBlock, nwin - 1);
+            a[q] = P.tabC[r * 2];
+            c[q] = P.tabC[r * 2 + 1];
+        }
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const int r = r0 + q * kBigBlock;
+            if (r < nwin) {
+                lds_rows[r] = a[q];
+                w2[r] = make_float2(c[q].x, c[q].y);
+                w1[r] = c[q].z;
+            }
+        }
     }
     __syncthreads();
+    if (stop && *stop) return;
     const ForceRowsLds T{P.tabC, lds_rows, w2, w1, m_lo};
+    const int g = threadIdx.x & ((1 << lg) - 1), size = kBigBlock >> lg;
     double acc[7] = {0, 0, 0, 0, 0, 0, 0};
     double mvv[6] = {0, 0, 0, 0, 0, 0};
     double fm[3] = {0, 0, 0};
-    for (ChunkWalk cw = chunk_walk(n); cw.c < cw.end; cw.c += cw.step) {
-        const int i = cw.c * kBigBlock + threadIdx.x;
+    for (ChunkWalk cw = chunk_walk(n, size); cw.c < cw.end; cw.c += cw.step) {
+        const int i = cw.c * size + (threadIdx.x >> lg);
         if (i >= n) continue;
         const uint4 ri = xr[i];
         float fx = 0.f, fy = 0.f, fz = 0.f;
         force_atom<B, true, EV>(i, ri, 0, __uint_as_float(ri.w), nn[i], nullptr, xr, nullptr, list4, ldl, maxb, P,
-                                R, T, fx, fy, fz, acc);
+                                R, T, lg, g, fx, fy, fz, acc);
+        fx = lane_sum(fx, lg);
+        fy = lane_sum(fy, lg);
+        fz = lane_sum(fz, lg);
+        if (g != 0) continue;
         f_out[i] = make_float4(fx, fy, fz, 0.f);
         if (K.on) kick_atom(i, 0, fx, fy, fz, K, v, mvv, fm);
     }
@@ -803,9 +879,7 @@ __global__ __launch_bounds__(kBigBlock) void k_eam_force_lds(int n, const uint4*
     }
     if (K.on) {
         if (EV) __syncthreads();
-        block_sum_store<6, kBigBlock>(mvv, part_mvv + (size_t)blockIdx.x * kPartW);
-        __syncthreads();
-        block_sum_store<3, kBigBlock>(fm, part_cv + (size_t)blockIdx.x * kPartW);
+        kick_rows<kBigBlock>(mvv, fm, part_mvv + (size_t)blockIdx.x * kPartW, part_cv + (size_t)blockIdx.x * kPartW);
     }
 }
 
@@ -840,7 +914,7 @@ __global__ __launch_bounds__(kBlock) void k_shift_decide(int n, double4* __restr
         rec[i] = make_uint4((unsigned)__double2ll_rn(xi.x * R.inv_q), (unsigned)__double2ll_rn(xi.y * R.inv_q),
                             (unsigned)__double2ll_rn(xi.z * R.inv_q), (unsigned)(int)xi.w);
     const double4 a = x0[i];
-    if (rsq_exact(a.x, a.y, a.z, xi.x, xi.y, xi.z) > skin_sq4) atomicOr(&flags[1], 1);
+    if (rsq_exact(a.x, a.y, a.z, xi.x, xi.y, xi.z) > skin_sq4) atomicOr(&flags[FL_REBUILD], 1);
 }
 
 // The first half of a velocity-Verlet step in one pass (update_x_d__x,
@@ -850,20 +924,26 @@ __global__ __launch_bounds__(kBlock) void k_shift_decide(int n, double4* __restr
 // pass from the sums of v and f / m the previous force pass left; then the
 // skin check against x0 and the 16-byte position record. Partial sums of the
 // new v go to part_sv.
+// At most kStepRows workgroups walk the atoms, so that one workgroup can sum
+// their rows (k_nvt_end).
+constexpr int kStepRows = 2048;
 __global__ __launch_bounds__(kBlock) void k_step(int n, double4* __restrict__ x, double4* __restrict__ v,
                                                  const float4* __restrict__ f, NvtArgs A,
                                                  const double* __restrict__ nh, const double4* __restrict__ x0,
                                                  double skin_sq4, int* __restrict__ flags, Rec16Frame R,
                                                  uint4* __restrict__ rec, double* __restrict__ part_sv)
 {
-    const int blk = xcd_block();
-    const int i = blk * kBlock + threadIdx.x;
+    if (flags[FL_HALT]) return;
     double sv[3] = {0.0, 0.0, 0.0};
-    if (i < n) {
-        const double fac = nh[NH_FAC];
+    const double fac = nh[NH_FAC], c0 = nh[NH_COM], c1 = nh[NH_COM + 1], c2 = nh[NH_COM + 2];
+    bool moved = false;
+    for (ChunkWalk w = chunk_walk(n, kBlock); w.c < w.end; w.c += w.step) {
+        const int i = w.c * kBlock + threadIdx.x;
+        if (i >= n) continue;
         double4 xi = x[i];
         double4 vi = v[i];
         const float4 fi = f[i];
+        const double4 a = x0[i];
         const double m = A.mass[(int)xi.w];
         vi.x = vi.x * fac + (double)fi.x * A.dt2 / m;
         vi.y = vi.y * fac + (double)fi.y * A.dt2 / m;
@@ -871,20 +951,20 @@ __global__ __launch_bounds__(kBlock) void k_step(int n, double4* __restrict__ x,
         xi.x += vi.x * A.dt;
         xi.y += vi.y * A.dt;
         xi.z += vi.z * A.dt;
-        xi.x -= nh[NH_COM];
-        xi.y -= nh[NH_COM + 1];
-        xi.z -= nh[NH_COM + 2];
+        xi.x -= c0;
+        xi.y -= c1;
+        xi.z -= c2;
         x[i] = xi;
         v[i] = vi;
         rec[i] = make_uint4((unsigned)__double2ll_rn(xi.x * R.inv_q), (unsigned)__double2ll_rn(xi.y * R.inv_q),
                             (unsigned)__double2ll_rn(xi.z * R.inv_q), (unsigned)(int)xi.w);
-        const double4 a = x0[i];
-        if (rsq_exact(a.x, a.y, a.z, xi.x, xi.y, xi.z) > skin_sq4) atomicOr(&flags[1], 1);
-        sv[0] = vi.x;
-        sv[1] = vi.y;
-        sv[2] = vi.z;
+        moved |= rsq_exact(a.x, a.y, a.z, xi.x, xi.y, xi.z) > skin_sq4;
+        sv[0] += vi.x;
+        sv[1] += vi.y;
+        sv[2] += vi.z;
     }
-    block_sum_store<3>(sv, part_sv + (size_t)blk * kPartW);
+    if (moved) atomicOr(&flags[FL_REBUILD], 1);
+    block_sum_store<3>(sv, part_sv + (size_t)blockIdx.x * kPartW);
 }
 
 // second half kick (when kick), the kinetic tensor sum m v (x) v, and the sums
@@ -960,10 +1040,9 @@ __device__ inline double nhc_half(double* e, const NvtArgs& A, double T_r)
 // mode 2: T from the new mvv, the sums of v after the kick (cv[0..2], the
 // step's v, plus dt/2 cv[3..5], the new f / m), thermostat after the step
 // (fac = s)
-__global__ void k_nhc(double* __restrict__ nh, const double* __restrict__ mvv, const double* __restrict__ cv,
-                      NvtArgs A, int mode)
+__device__ inline void nhc_update(double* __restrict__ nh, const double* mvv, const double* cv, const NvtArgs& A,
+                                  int mode)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
     if (mode == 0)
         for (int k = 0; k < 3; ++k) {
             nh[NH_SV + k] = cv[k];
@@ -990,6 +1069,53 @@ __global__ void k_nhc(double* __restrict__ nh, const double* __restrict__ mvv, c
     if (mode == 1)
         for (int k = 0; k < 3; ++k)
             nh[NH_COM + k] = (nh[NH_FAC] * nh[NH_SV + k] + A.dt2 * nh[NH_SF + k]) * A.dt / A.natms;
+}
+
+// the start of a run: modes 0 and 1
+__global__ void k_nhc(double* __restrict__ nh, const double* __restrict__ mvv, const double* __restrict__ cv,
+                      NvtArgs A)
+{
+    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+    nhc_update(nh, mvv, cv, A, 0);
+    nhc_update(nh, mvv, cv, A, 1);
+}
+
+// The end of an NVT step on one workgroup: the sums of the new velocities
+// (rows of k_step), of the kinetic tensor and of f / m (rows of the force
+// pass), then the thermostat after the step and, unless it was the last, the
+// one that starts the next step. One launch in place of six reductions and two
+// thermostat launches of 3 to 4 us each. told: the steps done and whether a
+// rebuild is due, in host memory. Where the step found that the list is
+// to be rebuilt, the run is halted instead: what was launched after it does
+// nothing until the host has rebuilt the list.
+// A wave sums one column.
+constexpr int kEndThreads = 768;
+__global__ __launch_bounds__(kEndThreads) void k_nvt_end(double* __restrict__ nh, const double* __restrict__ rows_sv,
+                                                         int nsv, const double* __restrict__ rows_mvv,
+                                                         const double* __restrict__ rows_fm, int nf, NvtArgs A,
+                                                         int last, double* __restrict__ hist_T,
+                                                         int* __restrict__ flags, volatile int* __restrict__ told)
+{
+    __shared__ double sum[12];
+    const int col = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const double* rows = col < 3 ? rows_sv + col : col < 6 ? rows_fm + (col - 3) : rows_mvv + (col - 6);
+    const int nr = col < 3 ? nsv : nf;
+    const int rebuild = flags[FL_REBUILD];
+    double s[1] = {0.0};
+    for (int r = lane; r < nr; r += 64) s[0] += rows[(size_t)r * kPartW];
+    wave_sums<1>(s);
+    if (lane == 0) sum[col] = s[0];
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    if (rebuild) {
+        flags[FL_HALT] = 1;
+        told[1] = 1;
+        return;
+    }
+    nhc_update(nh, sum + 6, sum, A, 2);
+    if (hist_T) *hist_T = nh[NH_T];
+    if (!last) nhc_update(nh, nullptr, nullptr, A, 1);
+    told[0] = flags[FL_DONE] += 1;
 }
 
 __global__ __launch_bounds__(kBlock) void k_scale_v(int n, double4* __restrict__ v, const double* __restrict__ nh)
@@ -1153,9 +1279,11 @@ MDSystem::MDSystem(std::shared_ptr<EamForceField> ff, int natms, const double* H
     keys_.reserve(n_); keys_alt_.reserve(n_); vals_.reserve(n_); vals_alt_.reserve(n_); s_tmp_.reserve(n_);
     nn_.reserve(n_);
     flags_.reserve(4);
-    part_.reserve((size_t)5 * grid_for(n_) * kPartW + 64);  // rho, force, integrator, two centre-of-mass rows
+    MAPP_HIP(hipMemsetAsync(flags_.get(), 0, sizeof(int) * 4, stream_));
+    part_.reserve((size_t)5 * part_rows() * kPartW + 64);  // rho, force, integrator, two centre-of-mass rows
     red_.reserve(64);
-    red2_.reserve(256 * kPartW);
+    red2_.reserve(512 * kPartW);
+    told_.reserve(2);
     std::vector<double4> xh(n_);
     std::vector<int> idh(n_);
     for (int i = 0; i < n_; ++i) {
@@ -1208,7 +1336,7 @@ void MDSystem::reset_atoms(int natms, const double* x, const uint8_t* elem, cons
     f_.reserve(n_); rho_.reserve(n_); dF_.reserve(n_); xr_.reserve(n_); rec_.reserve(n_);
     keys_.reserve(n_); keys_alt_.reserve(n_); vals_.reserve(n_); vals_alt_.reserve(n_); s_tmp_.reserve(n_);
     nn_.reserve(n_);
-    part_.reserve((size_t)5 * grid_for(n_) * kPartW + 64);
+    part_.reserve((size_t)5 * part_rows() * kPartW + 64);
     std::vector<double4> xh(n_), vh(n_);
     std::vector<int> idh(n_);
     for (int i = 0; i < n_; ++i) {
@@ -1238,6 +1366,10 @@ MDSystem::~MDSystem()
         (void)hipStreamDestroy(stream_);
     }
 }
+
+// rows of one region of the partial-sum buffer: one per 256 atoms, and where a
+// small system's passes use more workgroups than that, at most kMinPartRows
+int MDSystem::part_rows() const { return std::max(grid_for(n_), kMinPartRows); }
 
 void MDSystem::sync() { MAPP_HIP(hipStreamSynchronize(stream_)); }
 
@@ -1469,15 +1601,47 @@ void MDSystem::build_list()
     throw Error(ERR_STATE, "neighbor list capacity did not converge");
 }
 
-void MDSystem::force_passes(const KickArgs* kick, bool records_fresh, float4* f_out, double* rho_out, bool ev)
+// log2 of the lanes that share an atom: the fewest rounds of 4-entry batches.
+// A workgroup of the LDS passes works on 1024 / 2^lg atoms at a time, and the
+// CUs on as many chunks side by side; a round costs its lane's batches and,
+// for the atom's own loads, embedding and sums, about two more (three once
+// lanes have to meet).
+int MDSystem::lanes_lds() const
 {
-    const int nb = grid_for(n_);
+    const int batches = (int)((maxn_ - 16) / 1.25 / 4.0) + 1;  // the expected row, see setup_grid
+    int best = 0;
+    long least = 0;
+    for (int lg = 0; lg <= 4; ++lg) {
+        const int size = kBigBlock >> lg;
+        const long chunks = (n_ + size - 1) / size;
+        const long cost = ((chunks + lds_grid_ - 1) / lds_grid_) * (((batches - 1) >> lg) + (lg ? 4 : 3));
+        if (lg == 0 || cost < least) {
+            least = cost;
+            best = lg;
+        }
+    }
+    return best;
+}
+
+// the passes with global tables: as many lanes as keep every CU at 8 waves of
+// 64 (the rows come from L2, and waves hide its latency)
+int MDSystem::lanes_global() const
+{
+    int lg = 0;
+    while (lg < 4 && ((long)n_ << (lg + 1)) <= 256L * 2048) ++lg;
+    return lg;
+}
+
+void MDSystem::force_passes(const KickArgs* kick, bool records_fresh, float4* f_out, double* rho_out, bool ev,
+                            const int* stop)
+{
     float4* fo = f_out ? f_out : f_.get();
     double* ro = rho_out ? rho_out : rho_.get();
     const EamArgs P = ff_->args();
     prof_.begin(K_EAM_RHO, stream_);
     if (!records_fresh)
-        hipLaunchKernelGGL(k_make_records, dim3(nb), dim3(kBlock), 0, stream_, n_, x_.get(), r16_, rec_.get());
+        hipLaunchKernelGGL(k_make_records, dim3(grid_for(n_)), dim3(kBlock), 0, stream_, n_, x_.get(), r16_,
+                           rec_.get());
     const bool one = P.ne == 1;
     const bool lds = one && use_lds_;
     KickArgs K{};
@@ -1485,16 +1649,19 @@ void MDSystem::force_passes(const KickArgs* kick, bool records_fresh, float4* f_
         K = *kick;
         K.on = 1;
     }
-    double* p3 = part_.get() + (size_t)2 * nb * kPartW;
-    double* p4 = part_.get() + (size_t)3 * nb * kPartW;
+    double* p3 = part_.get() + (size_t)2 * part_rows() * kPartW;
+    double* p4 = part_.get() + (size_t)3 * part_rows() * kPartW;
     const int maxb = maxn_ / 4;
     if (lds) {
-        // at most one workgroup per CU, and never more rows than the partial-sum buffer has per pass
-        const int G = std::min(lds_grid_, nb);
-#define MAPP_RHO(B) hipLaunchKernelGGL((k_eam_rho_lds<B>), dim3(G), dim3(kBigBlock), rho_lds_bytes_, stream_, n_, \
-                                       rec_.get(), nn_.get(), list4(), ldl_, maxb, P, r16_, rho_m_lo_, rho_nwin_, \
-                                       ro, xr_.get(), part_.get())
-        switch (batch_rho_) {
+        const int lg = lanes_lds();
+        const int chunks = (n_ + (kBigBlock >> lg) - 1) / (kBigBlock >> lg);
+        // at most one workgroup per CU, and one per chunk (rounded up to the 8 XCDs)
+        const int G = std::min(lds_grid_, (chunks + kXcd - 1) / kXcd * kXcd);
+        const int br = lg && batch_rho_ > 4 ? 4 : batch_rho_;
+#define MAPP_RHO(B) hipLaunchKernelGGL((k_eam_rho_lds<B>), dim3(G), dim3(kBigBlock), rho_lds_bytes_, stream_, n_, lg, \
+                                       stop, rec_.get(), nn_.get(), list4(), ldl_, maxb, P, r16_, rho_m_lo_, \
+                                       rho_nwin_, ro, xr_.get(), part_.get())
+        switch (br) {
             case 1: MAPP_RHO(1); break;
             case 2: MAPP_RHO(2); break;
             case 4: MAPP_RHO(4); break;
@@ -1505,8 +1672,8 @@ void MDSystem::force_passes(const KickArgs* kick, bool records_fresh, float4* f_
         prof_.begin(K_EAM_FORCE, stream_);
         double* p2 = part_.get() + (size_t)G * kPartW;
 #define MAPP_FORCE(B, EV) hipLaunchKernelGGL((k_eam_force_lds<B, EV>), dim3(G), dim3(kBigBlock), f_lds_bytes_, \
-                                             stream_, n_, xr_.get(), r16_, nn_.get(), list4(), ldl_, maxb, P, f_m_lo_, \
-                                             f_nwin_, fo, p2, K, v_.get(), p3, p4)
+                                             stream_, n_, lg, stop, xr_.get(), r16_, nn_.get(), list4(), ldl_, maxb, \
+                                             P, f_m_lo_, f_nwin_, fo, p2, K, v_.get(), p3, p4)
         // 1024-thread workgroups leave 128 VGPRs per lane: batches of 4 fit
         // without the FP64 energy and virial sums only
         if (batch_force_ == 1) {
@@ -1518,14 +1685,17 @@ void MDSystem::force_passes(const KickArgs* kick, bool records_fresh, float4* f_
         }
 #undef MAPP_FORCE
         prof_.end(stream_);
-        mvv_rows_ = G;
+        pass_rows_ = G;
         if (ev) reduce_rows(part_.get(), 2 * G, 7, red_.get());
         return;
     }
-#define MAPP_RHO(B, ONE) hipLaunchKernelGGL((k_eam_rho<B, ONE>), dim3(nb), dim3(kBlock), 0, stream_, n_, rec_.get(), \
-                                            nn_.get(), list4(), ldl_, maxb, P, r16_, ro, xr_.get(), \
+    const int lg = lanes_global();
+    const int nb = (int)((((long)n_ << lg) + kXcd * kBlock - 1) / (kXcd * kBlock)) * kXcd;
+    const int br = lg && batch_rho_ > 4 ? 4 : batch_rho_, bf = lg && batch_force_ > 4 ? 4 : batch_force_;
+#define MAPP_RHO(B, ONE) hipLaunchKernelGGL((k_eam_rho<B, ONE>), dim3(nb), dim3(kBlock), 0, stream_, n_, lg, stop, \
+                                            rec_.get(), nn_.get(), list4(), ldl_, maxb, P, r16_, ro, xr_.get(), \
                                             dF_.get(), part_.get())
-    switch (batch_rho_) {
+    switch (br) {
         case 1: if (one) MAPP_RHO(1, true); else MAPP_RHO(1, false); break;
         case 2: if (one) MAPP_RHO(2, true); else MAPP_RHO(2, false); break;
         case 4: if (one) MAPP_RHO(4, true); else MAPP_RHO(4, false); break;
@@ -1536,8 +1706,8 @@ void MDSystem::force_passes(const KickArgs* kick, bool records_fresh, float4* f_
     prof_.begin(K_EAM_FORCE, stream_);
     double* p2 = part_.get() + (size_t)nb * kPartW;
 #define MAPP_FORCE(B, ONE, EV) hipLaunchKernelGGL((k_eam_force<B, ONE, EV>), dim3(nb), dim3(kBlock), 0, stream_, n_, \
-                                                  rec_.get(), xr_.get(), dF_.get(), r16_, nn_.get(), list4(), ldl_, \
-                                                  maxb, P, fo, p2, K, v_.get(), p3, p4)
+                                                  lg, stop, rec_.get(), xr_.get(), dF_.get(), r16_, nn_.get(), \
+                                                  list4(), ldl_, maxb, P, fo, p2, K, v_.get(), p3, p4)
 #define MAPP_FORCE_EV(B, ONE) \
     do {                      \
         if (ev)               \
@@ -1545,7 +1715,7 @@ void MDSystem::force_passes(const KickArgs* kick, bool records_fresh, float4* f_
         else                  \
             MAPP_FORCE(B, ONE, false); \
     } while (0)
-    switch (batch_force_) {
+    switch (bf) {
         case 1: if (one) MAPP_FORCE_EV(1, true); else MAPP_FORCE_EV(1, false); break;
         case 2: if (one) MAPP_FORCE_EV(2, true); else MAPP_FORCE_EV(2, false); break;
         case 8: if (one) MAPP_FORCE_EV(8, true); else MAPP_FORCE_EV(8, false); break;
@@ -1554,7 +1724,7 @@ void MDSystem::force_passes(const KickArgs* kick, bool records_fresh, float4* f_
 #undef MAPP_FORCE_EV
 #undef MAPP_FORCE
     prof_.end(stream_);
-    mvv_rows_ = nb;
+    pass_rows_ = nb;
     if (ev) reduce_rows(part_.get(), 2 * nb, 7, red_.get());
 }
 
@@ -1804,7 +1974,6 @@ int MDSystem::nvt_run(const double* masses, double kB, double T, double dt, int 
                       const ExchangeHook* hook, double* hist_T)
 {
     MAPP_REQUIRE(nsteps >= 0 && dt > 0.0 && T > 0.0 && kB > 0.0, ERR_ARG, "invalid NVT parameters");
-    int nb = grid_for(n_);
     const EamTables& t = ff_->tables();
     NvtArgs A{};
     A.dt = dt;
@@ -1824,59 +1993,108 @@ int MDSystem::nvt_run(const double* masses, double kB, double T, double dt, int 
     double* nh = red_.get() + 32;  // NH_SIZE doubles of thermostat state
     double* cv = red_.get() + 24;  // sums of v and f / m for the centre-of-mass shift
     double* mvv = red_.get() + 8;
-    double* rows_mvv = part_.get() + (size_t)2 * nb * kPartW;
-    double* rows_cv = part_.get() + (size_t)3 * nb * kPartW;
-    double* rows_sv = part_.get() + (size_t)4 * nb * kPartW;
+    const auto region = [&](int k) { return part_.get() + (size_t)k * part_rows() * kPartW; };
     const int nevery = hook && hook->run ? hook->nevery : 0;
     MAPP_HIP(hipMemsetAsync(nh, 0, sizeof(double) * NH_SIZE, stream_));
+    MAPP_HIP(hipMemsetAsync(flags_.get() + 1, 0, sizeof(int) * 3, stream_));
+    if (hist_T) hist_.reserve(std::max(1, nsteps));
     const int rebuilds0 = nrebuild_;
     force_passes(nullptr);
-    hipLaunchKernelGGL(k_kick2, dim3(nb), dim3(kBlock), 0, stream_, n_, x_.get(), v_.get(), f_.get(), A, 0, rows_mvv,
-                       rows_cv);
-    reduce_rows(rows_mvv, nb, 6, mvv);
-    reduce_rows(rows_cv, nb, 6, cv);
-    hipLaunchKernelGGL(k_nhc, dim3(1), dim3(64), 0, stream_, nh, mvv, cv, A, 0);
+    {
+        const int nb = grid_for(n_);
+        hipLaunchKernelGGL(k_kick2, dim3(nb), dim3(kBlock), 0, stream_, n_, x_.get(), v_.get(), f_.get(), A, 0,
+                           region(2), region(3));
+        reduce_rows(region(2), nb, 6, mvv);
+        reduce_rows(region(3), nb, 6, cv);
+    }
+    hipLaunchKernelGGL(k_nhc, dim3(1), dim3(64), 0, stream_, nh, mvv, cv, A);
     const double skin_sq4 = 0.25 * skin_ * skin_;
     KickArgs kick{};
     kick.dt2 = A.dt2;
     for (int a = 0; a < t.ne; ++a) kick.mass[a] = A.mass[a];
-    int flag = 0;
-    for (int step = 0; step < nsteps; ++step) {
+    int nsv = 0;  // rows of velocity sums of the step
+    const auto first_half = [&]() {
+        nsv = std::min(kStepRows, grid_for(n_));
         prof_.begin(K_INTEGRATE, stream_);
-        hipLaunchKernelGGL(k_nhc, dim3(1), dim3(64), 0, stream_, nh, mvv, cv, A, 1);
-        MAPP_HIP(hipMemsetAsync(flags_.get() + 1, 0, sizeof(int), stream_));
-        hipLaunchKernelGGL(k_step, dim3(nb), dim3(kBlock), 0, stream_, n_, x_.get(), v_.get(), f_.get(), A, nh,
-                           x0_.get(), skin_sq4, flags_.get(), r16_, rec_.get(), rows_sv);
-        reduce_rows(rows_sv, nb, 3, cv);
+        hipLaunchKernelGGL(k_step, dim3(nsv), dim3(kBlock), 0, stream_, n_, x_.get(), v_.get(), f_.get(), A, nh,
+                           x0_.get(), skin_sq4, flags_.get(), r16_, rec_.get(), region(4));
         prof_.end(stream_);
-        MAPP_HIP(hipMemcpyAsync(&flag, flags_.get() + 1, sizeof(int), hipMemcpyDeviceToHost, stream_));
-        MAPP_HIP(hipStreamSynchronize(stream_));
-        if (nevery > 0 && (step + 1) % nevery == 0) {
+    };
+    // the passes (energy and virial only where they are read: after the last
+    // step) and the step's end
+    const auto second_half = [&](int step) {
+        force_passes(&kick, true, nullptr, nullptr, step == nsteps - 1, flags_.get() + FL_REBUILD);
+        prof_.begin(K_INTEGRATE, stream_);
+        const double *mv = region(2), *fm = region(3);
+        int rows = pass_rows_;
+        if (rows > kMinPartRows) {  // a first level where one workgroup would read many rows
+            rows = 256;
+            const int chunk = (pass_rows_ + rows - 1) / rows;
+            hipLaunchKernelGGL(k_reduce_rows, dim3(rows), dim3(kBlock), 0, stream_, pass_rows_, 6, mv, red2_.get(),
+                               chunk);
+            hipLaunchKernelGGL(k_reduce_rows, dim3(rows), dim3(kBlock), 0, stream_, pass_rows_, 3, fm,
+                               red2_.get() + (size_t)rows * kPartW, chunk);
+            mv = red2_.get();
+            fm = red2_.get() + (size_t)rows * kPartW;
+        }
+        hipLaunchKernelGGL(k_nvt_end, dim3(1), dim3(kEndThreads), 0, stream_, nh, region(4), nsv, mv, fm, rows, A,
+                           step == nsteps - 1 ? 1 : 0, hist_T ? hist_.get() + step : nullptr, flags_.get(),
+                           told_.get());
+        prof_.end(stream_);
+    };
+    // Steps are launched ahead in groups and the host reads the skin check's
+    // answers after a group, not after every step (a round trip of 20 to 30 us
+    // each): once a step finds that the list is to be rebuilt, the launches
+    // after it return at once. The first group after a rebuild ends two steps
+    // before the next rebuild is due, if it comes after as many steps as the
+    // last one; then come groups of two. With the kernels timed, one step.
+    volatile int* told = told_.get();
+    int interval = 12, since = 0, step = 0, base = 0;
+    told[0] = told[1] = 0;
+    const auto resume = [&]() {  // after a rebuild
+        MAPP_HIP(hipMemsetAsync(flags_.get() + 1, 0, sizeof(int) * 3, stream_));
+        told[0] = told[1] = 0;
+        second_half(step);
+        ++step;
+        since = 0;
+        base = 1;
+    };
+    while (step < nsteps) {
+        const int to_exchange = nevery > 0 ? nevery - 1 - step % nevery : nsteps;
+        if (to_exchange == 0) {
             // the exchange takes the place of the skin check (MDMuVT::run,
             // src/md_muvt.cpp:172-195); it ends with a rebuild, and the atom
             // count, ndof_part = 3 natms and the sums of v follow it
+            first_half();
             hook->run();
-            nb = grid_for(n_);
-            rows_mvv = part_.get() + (size_t)2 * nb * kPartW;
-            rows_cv = part_.get() + (size_t)3 * nb * kPartW;
-            rows_sv = part_.get() + (size_t)4 * nb * kPartW;
             A.ndof = 3 * n_;
             A.natms = n_;
-            hipLaunchKernelGGL(k_sum_v, dim3(nb), dim3(kBlock), 0, stream_, n_, v_.get(), rows_sv);
-            reduce_rows(rows_sv, nb, 3, cv);
-        } else if (flag) {
-            rebuild();  // the permute rewrites the records
+            nsv = grid_for(n_);
+            hipLaunchKernelGGL(k_sum_v, dim3(nsv), dim3(kBlock), 0, stream_, n_, v_.get(), region(4));
+            MAPP_HIP(hipStreamSynchronize(stream_));
+            resume();
+            continue;
         }
-        // energy and virial only where they are read: after the last step
-        force_passes(&kick, true, nullptr, nullptr, step == nsteps - 1);
-        prof_.begin(K_INTEGRATE, stream_);
-        reduce_rows(rows_mvv, mvv_rows_, 6, mvv);
-        reduce_rows(rows_cv, mvv_rows_, 3, cv + 3);
-        hipLaunchKernelGGL(k_nhc, dim3(1), dim3(64), 0, stream_, nh, mvv, cv, A, 2);
-        prof_.end(stream_);
-        if (hist_T) MAPP_HIP(hipMemcpyAsync(hist_T + step, nh + NH_T, sizeof(double), hipMemcpyDeviceToHost, stream_));
+        int group = prof_.on ? 1 : std::max(2, std::min(64, interval - 2 - since));
+        group = std::min(std::min(group, nsteps - step), to_exchange);
+        for (int k = 0; k < group; ++k) {
+            first_half();
+            second_half(step + k);
+        }
+        MAPP_HIP(hipStreamSynchronize(stream_));
+        const int done = told[0] - base;
+        step += done;
+        since += done;
+        base += done;
+        if (told[1]) {
+            interval = since + 1;
+            rebuild();  // the permute rewrites the records
+            resume();
+        }
     }
-    hipLaunchKernelGGL(k_scale_v, dim3(nb), dim3(kBlock), 0, stream_, n_, v_.get(), nh);
+    if (hist_T && nsteps > 0)
+        MAPP_HIP(hipMemcpyAsync(hist_T, hist_.get(), sizeof(double) * nsteps, hipMemcpyDeviceToHost, stream_));
+    hipLaunchKernelGGL(k_scale_v, dim3(grid_for(n_)), dim3(kBlock), 0, stream_, n_, v_.get(), nh);
     double nhh[NH_SIZE];
     MAPP_HIP(hipMemcpyAsync(nhh, nh, sizeof(double) * NH_SIZE, hipMemcpyDeviceToHost, stream_));
     MDReport r = reduce_report(7);

@@ -13,6 +13,7 @@ namespace mapp {
 constexpr int kMaxElems = 8;
 constexpr int kIndexBits = 25;                 // neighbor entry: j in the low bits,
 constexpr uint32_t kIndexMask = (1u << kIndexBits) - 1u;  // image code in the high 7
+constexpr int kMinPartRows = 4096;              // see MDSystem::part_rows
 constexpr int kZeroImage = 62;                  // code of the (0,0,0) shift
 
 // Kernel argument block describing the EAM tables on the device.
@@ -199,9 +200,12 @@ private:
     void build_list();
     // records_fresh: rec_ already holds the current positions (written by the skin check or a rebuild)
     // the two EAM passes; f_out / rho_out (nullptr: f_ and rho_) receive the
-    // forces and densities
+    // forces and densities; nothing is computed where *stop is set
     void force_passes(const KickArgs* kick, bool records_fresh = false, float4* f_out = nullptr,
-                      double* rho_out = nullptr, bool ev = true);
+                      double* rho_out = nullptr, bool ev = true, const int* stop = nullptr);
+    int part_rows() const;
+    int lanes_lds() const;
+    int lanes_global() const;
     MDReport reduce_report(int nparts);
     void reduce_rows(const double* part, int nrows, int ncols, double* out);
     bool decide();
@@ -256,7 +260,9 @@ private:
     int lds_grid_ = 0;
     int rho_m_lo_ = 0, rho_nwin_ = 0, f_m_lo_ = 0, f_nwin_ = 0;
     size_t rho_lds_bytes_ = 0, f_lds_bytes_ = 0;
-    int mvv_rows_ = 0;               // rows of kinetic partial sums written by the last force pass
+    int pass_rows_ = 0;              // rows of kinetic partial sums written by the last force pass
+    DevBuf<double> hist_;            // a run's T_part after each step
+    HostBuf<int> told_;              // what a run's steps tell the host
     // minimiser vectors in slot order: line-search origin, direction, forces
     // at the origin, L-BFGS pairs; a spare for permutations
     DevBuf<double4> mn_x0_, mn_h_, mn_f0_, mn_tmp_;
