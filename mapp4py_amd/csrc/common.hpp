@@ -82,7 +82,7 @@ struct HostBuf {
         if (count <= n && p) return;
         if (p) (void)hipHostFree(p);
         p = nullptr;
-        MAPP_HIP(hipHostMalloc((void**)&p, (count ? count : 1) * sizeof(T), 0));
+        MAPP_HIP(hipHostMalloc(&p, (count ? count : 1) * sizeof(T), 0));
         n = count;
     }
     T* get() const { return p; }

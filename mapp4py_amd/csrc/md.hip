@@ -158,6 +158,44 @@ __global__ __launch_bounds__(kBlock) void k_cell_order(int ncells, GridArgs g, c
 // several, the element pairs' cut-offs are read from LDS (an indexed
 // kernel-argument array would cost a memory round trip per candidate).
 template <bool ONE>
+struct ListTest {
+    const GridArgs& g;
+    const double (*cut)[kMaxElems * kMaxElems];  // LDS: rec_in_sq, rec_out_sq, cut_sk_sq
+    const BoxDev& bd;
+    const double4* s4;
+    int ti;
+    double xi0, xi1, xi2;
+    // rs: i's record less the image shift (n0, n1, n2), rj: j's record
+    __device__ bool operator()(const uint4& rs, const uint4& rj, int j, int n0, int n1, int n2) const
+    {
+        const double dx = (double)(int)(rs.x - rj.x), dy = (double)(int)(rs.y - rj.y), dz = (double)(int)(rs.z - rj.z);
+        const double rsq_u = dx * dx + dy * dy + dz * dz;
+        const int tt = ONE ? 0 : ti * g.ne + (int)rj.w;
+        bool in = rsq_u < (ONE ? g.rec_in_sq[0] : cut[0][tt]);
+        if (!in && rsq_u <= (ONE ? g.rec_out_sq[0] : cut[1][tt])) {
+            const double4 sj = s4[j];
+            double xj0, xj1, xj2;
+            s_to_x(bd.h, shift_unit(sj.x, n0), shift_unit(sj.y, n1), shift_unit(sj.z, n2), xj0, xj1, xj2);
+            in = rsq_exact(xi0, xi1, xi2, xj0, xj1, xj2) < (ONE ? g.cut_sk_sq[0] : cut[2][tt]);
+        }
+        return in;
+    }
+};
+
+// the cut-offs of the element pairs in LDS
+template <bool ONE>
+__device__ inline void stage_cuts(const GridArgs& g, double (*cut)[kMaxElems * kMaxElems])
+{
+    if (ONE) return;
+    for (int k = threadIdx.x; k < g.ne * g.ne; k += kBlock) {
+        cut[0][k] = g.rec_in_sq[k];
+        cut[1][k] = g.rec_out_sq[k];
+        cut[2][k] = g.cut_sk_sq[k];
+    }
+    __syncthreads();
+}
+
+template <bool ONE>
 __global__ __launch_bounds__(kBlock) void k_build_list(int n, const double4* __restrict__ s4,
                                                        const uint4* __restrict__ rec, Rec16Frame R, BoxDev bd,
                                                        GridArgs g, const int* __restrict__ cell_rank,
@@ -167,14 +205,7 @@ __global__ __launch_bounds__(kBlock) void k_build_list(int n, const double4* __r
                                                        int* __restrict__ flags)
 {
     __shared__ double cut_lds[3][kMaxElems * kMaxElems];
-    if (!ONE) {
-        for (int k = threadIdx.x; k < g.ne * g.ne; k += kBlock) {
-            cut_lds[0][k] = g.rec_in_sq[k];
-            cut_lds[1][k] = g.rec_out_sq[k];
-            cut_lds[2][k] = g.cut_sk_sq[k];
-        }
-        __syncthreads();
-    }
+    stage_cuts<ONE>(g, cut_lds);
     const int i = xcd_block() * kBlock + threadIdx.x;
     if (i >= n) return;
     const double4 si = s4[i];
@@ -183,6 +214,7 @@ __global__ __launch_bounds__(kBlock) void k_build_list(int n, const double4* __r
     double xi0, xi1, xi2;
     s_to_x(bd.h, si.x, si.y, si.z, xi0, xi1, xi2);
     const int c0 = cell_coord(si.x, g.nc[0]), c1 = cell_coord(si.y, g.nc[1]), c2 = cell_coord(si.z, g.nc[2]);
+    const ListTest<ONE> listed{g, cut_lds, bd, s4, ti, xi0, xi1, xi2};
     int cnt = 0;
     uint32_t p0 = 0u, p1 = 0u, p2 = 0u, p3 = 0u;  // the block being filled
     // candidates of the stencil cell at offset (o0, o1, o2)
@@ -203,17 +235,7 @@ __global__ __launch_bounds__(kBlock) void k_build_list(int n, const double4* __r
             const uint4 rj = rn;
             rn = rec[j + 1 < je ? j + 1 : j];
             if (self_img && j == i) continue;
-            const double dx = (double)(int)(rs.x - rj.x), dy = (double)(int)(rs.y - rj.y),
-                         dz = (double)(int)(rs.z - rj.z);
-            const double rsq_u = dx * dx + dy * dy + dz * dz;
-            const int tt = ONE ? 0 : ti * g.ne + (int)rj.w;
-            bool in = rsq_u < (ONE ? g.rec_in_sq[0] : cut_lds[0][tt]);
-            if (!in && rsq_u <= (ONE ? g.rec_out_sq[0] : cut_lds[1][tt])) {
-                const double4 sj = s4[j];
-                double xj0, xj1, xj2;
-                s_to_x(bd.h, shift_unit(sj.x, n0), shift_unit(sj.y, n1), shift_unit(sj.z, n2), xj0, xj1, xj2);
-                in = rsq_exact(xi0, xi1, xi2, xj0, xj1, xj2) < (ONE ? g.cut_sk_sq[0] : cut_lds[2][tt]);
-            }
+            const bool in = listed(rs, rj, j, n0, n1, n2);
             if (in) {
                 const uint32_t e = (uint32_t)j | code;
                 const int q = cnt & 3;
@@ -248,6 +270,72 @@ __global__ __launch_bounds__(kBlock) void k_build_list(int n, const double4* __r
     if ((cnt & 3) != 0 && (cnt >> 2) < maxb) list4[(size_t)(cnt >> 2) * ldl + i] = make_uint4(p0, p1, p2, p3);
     nn[i] = cnt;
     if (cnt > 4 * maxb) atomicMax(&flags[FL_OVER], cnt);
+}
+
+// The same list with 2^lg lanes per atom, for systems that would leave most of
+// the chip without work: the lanes test the candidates of a cell side by side
+// (about 14 in a metal) and the group's ballot gives each hit its place, so the
+// rows are those of k_build_list. The 16-byte blocks are written entry by entry.
+template <bool ONE>
+__global__ __launch_bounds__(kBlock) void k_build_list_group(int n, int lg, const double4* __restrict__ s4,
+                                                             const uint4* __restrict__ rec, Rec16Frame R, BoxDev bd,
+                                                             GridArgs g, const int* __restrict__ cell_rank,
+                                                             const int* __restrict__ cell_start,
+                                                             const uint4* __restrict__ order, int maxb, int ldl,
+                                                             uint32_t* __restrict__ list, int* __restrict__ nn,
+                                                             int* __restrict__ flags)
+{
+    __shared__ double cut_lds[3][kMaxElems * kMaxElems];
+    stage_cuts<ONE>(g, cut_lds);
+    const int G = 1 << lg, gl = threadIdx.x & (G - 1);
+    const int base = (threadIdx.x & 63) & ~(G - 1);  // the group's first lane of the wave
+    const int i = (int)(((long)xcd_block() * kBlock + threadIdx.x) >> lg);
+    if (i >= n) return;
+    const double4 si = s4[i];
+    const uint4 ri = rec[i];
+    const int ti = (int)si.w;
+    double xi0, xi1, xi2;
+    s_to_x(bd.h, si.x, si.y, si.z, xi0, xi1, xi2);
+    const int c0 = cell_coord(si.x, g.nc[0]), c1 = cell_coord(si.y, g.nc[1]), c2 = cell_coord(si.z, g.nc[2]);
+    const ListTest<ONE> listed{g, cut_lds, bd, s4, ti, xi0, xi1, xi2};
+    int cnt = 0;
+    auto scan = [&](int o0, int o1, int o2) {
+        const int u2 = c2 + o2, n2 = floordiv(u2, g.nc[2]), w2 = u2 - n2 * g.nc[2];
+        const int u1 = c1 + o1, n1 = floordiv(u1, g.nc[1]), w1 = u1 - n1 * g.nc[1];
+        const int u0 = c0 + o0, n0 = floordiv(u0, g.nc[0]), w0 = u0 - n0 * g.nc[0];
+        const int rank = cell_rank[w0 + g.nc[0] * (w1 + g.nc[1] * w2)];
+        const int jb = cell_start[rank], je = cell_start[rank + 1];
+        const bool self_img = (n0 | n1 | n2) == 0;
+        const uint32_t img = (uint32_t)((n0 + 2) + 5 * (n1 + 2) + 25 * (n2 + 2));
+        const uint4 sh = R.shift[img];
+        const uint4 rs = make_uint4(ri.x - sh.x, ri.y - sh.y, ri.z - sh.z, 0u);
+        for (int j0 = jb; j0 < je; j0 += G) {
+            const int j = j0 + gl;
+            const bool in =
+                j < je && !(self_img && j == i) && listed(rs, rec[j < je ? j : i], j < je ? j : i, n0, n1, n2);
+            const unsigned hits = (unsigned)(__ballot(in) >> base) & ((1u << G) - 1u);
+            const int pos = cnt + __popc(hits & ((1u << gl) - 1u));
+            if (in && (pos >> 2) < maxb)
+                list[((size_t)(pos >> 2) * ldl + i) * 4 + (pos & 3)] = (uint32_t)j | (img << kIndexBits);
+            cnt += __popc(hits);
+        }
+    };
+    if (order) {
+        const size_t w = (size_t)c0 + (size_t)g.nc[0] * (c1 + (size_t)g.nc[1] * c2);
+        const unsigned char* ob = (const unsigned char*)(order + 2 * w);
+        for (int q = 0; q < 27; ++q) {
+            const int t = ob[q];
+            scan(t % 3 - 1, t / 3 % 3 - 1, t / 9 - 1);
+        }
+    } else {
+        for (int o2 = -g.R[2]; o2 <= g.R[2]; ++o2)
+            for (int o1 = -g.R[1]; o1 <= g.R[1]; ++o1)
+                for (int o0 = -g.R[0]; o0 <= g.R[0]; ++o0) scan(o0, o1, o2);
+    }
+    if (gl == 0) {
+        nn[i] = cnt;
+        if (cnt > 4 * maxb) atomicMax(&flags[FL_OVER], cnt);
+    }
 }
 
 // ---------------- EAM ----------------
@@ -1422,6 +1510,7 @@ void MDSystem::plan_lds()
 bool MDSystem::set_lds(bool on)
 {
     use_lds_ = on && lds_ok_;
+    lds_auto_ = false;
     return use_lds_;
 }
 
@@ -1582,7 +1671,15 @@ void MDSystem::build_list()
         list_.reserve((size_t)maxn_ * ldl_);
         MAPP_HIP(hipMemsetAsync(flags_.get(), 0, sizeof(int), stream_));
         prof_.begin(K_BUILD_LIST, stream_);
-        if (t.ne == 1)
+        if (const int lg = lanes_global(); lg > 0) {
+            const int ng = (int)((((long)n_ << lg) + kXcd * kBlock - 1) / (kXcd * kBlock)) * kXcd;
+#define MAPP_BUILD(ONE) hipLaunchKernelGGL(k_build_list_group<ONE>, dim3(ng), dim3(kBlock), 0, stream_, n_, lg, \
+                                           s_.get(), rec_.get(), r16_, bd, g, cell_rank_.get(), cell_start_.get(), \
+                                           ordered_ ? cell_order_.get() : nullptr, maxn_ / 4, ldl_, list_.get(), \
+                                           nn_.get(), flags_.get())
+            if (t.ne == 1) MAPP_BUILD(true); else MAPP_BUILD(false);
+#undef MAPP_BUILD
+        } else if (t.ne == 1)
             hipLaunchKernelGGL(k_build_list<true>, dim3(nb), dim3(kBlock), 0, stream_, n_, s_.get(), rec_.get(), r16_,
                                bd, g, cell_rank_.get(), cell_start_.get(), ordered_ ? cell_order_.get() : nullptr,
                                maxn_ / 4, ldl_, list4(), nn_.get(), flags_.get());
@@ -1643,7 +1740,7 @@ void MDSystem::force_passes(const KickArgs* kick, bool records_fresh, float4* f_
         hipLaunchKernelGGL(k_make_records, dim3(grid_for(n_)), dim3(kBlock), 0, stream_, n_, x_.get(), r16_,
                            rec_.get());
     const bool one = P.ne == 1;
-    const bool lds = one && use_lds_;
+    const bool lds = one && use_lds_ && (!lds_auto_ || n_ >= kLdsMinAtoms);
     KickArgs K{};
     if (kick) {
         K = *kick;

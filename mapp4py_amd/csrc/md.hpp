@@ -13,6 +13,11 @@ namespace mapp {
 constexpr int kMaxElems = 8;
 constexpr int kIndexBits = 25;                 // neighbor entry: j in the low bits,
 constexpr uint32_t kIndexMask = (1u << kIndexBits) - 1u;  // image code in the high 7
+// Smallest one-element system whose passes hold the spline rows in LDS: below
+// it, filling 160 KB a workgroup takes longer than reading the rows from L2
+// (an NVT step at 8,788 atoms 36.8 us with LDS, 34.9 without; at 32,000 44.0
+// and 51.7)
+constexpr int kLdsMinAtoms = 12288;
 constexpr int kMinPartRows = 4096;              // see MDSystem::part_rows
 constexpr int kZeroImage = 62;                  // code of the (0,0,0) shift
 
@@ -257,6 +262,7 @@ private:
     int batch_rho_ = 8, batch_force_ = 8;
     // persistent one-element passes: LDS row windows [m_lo, m_lo + nwin)
     bool lds_ok_ = false, use_lds_ = false;
+    bool lds_auto_ = true;           // LDS passes from kLdsMinAtoms on, until set_lds has chosen
     int lds_grid_ = 0;
     int rho_m_lo_ = 0, rho_nwin_ = 0, f_m_lo_ = 0, f_nwin_ = 0;
     size_t rho_lds_bytes_ = 0, f_lds_bytes_ = 0;

@@ -330,3 +330,25 @@ def test_isolated_atoms_have_empty_rows(M, cu_pot, natoms):
         assert np.abs(f).max() == 0.0 and np.abs(FH).max() == 0.0
         assert abs(e - eo) < 1e-9 * max(1.0, abs(eo))
         np.testing.assert_array_equal(g.rho(), np.zeros(natoms))
+
+
+@pytest.mark.parametrize("cells,alloy", [((8, 9, 7), False), ((20, 21, 23), False), ((25, 26, 27), False),
+                                         ((33, 32, 34), False), ((41, 40, 41), False), ((11, 12, 13), True),
+                                         ((45, 44, 46), True)])
+def test_forces_for_every_split_of_an_atom_over_lanes(M, cells, alloy):
+    # 2^lg lanes share an atom in the passes and the list build, lg = 4 .. 0 as
+    # the system grows; a ragged last chunk, and both table families
+    p = pot.johnson_feni_fs(nr=2000, nrho=2000) if alloy else pot.johnson_cu(nr=2000, nrho=2000)
+    x, H = pot.bcc(2.86, cells) if alloy else pot.fcc(3.615, cells)
+    rng = np.random.default_rng(len(x))
+    x = np.delete(x + rng.normal(0.0, 0.05, x.shape), rng.choice(len(x), 3, replace=False), axis=0)
+    elem = ((rng.random(len(x)) < 0.2) if alloy else np.zeros(len(x))).astype(np.uint8)
+    g = M.AtomsMD(M.ForceFieldEAM.from_knots(p), H, x, elem, skin=0.5)
+    f, e, FH = g.force_calc()
+    o = O.OMD(O.OEam.from_knots(p), H, x, elem, skin=0.5)
+    fo, eo, FHo, _ = o.force()
+    # the bars of the force and energy tests above
+    assert np.abs(f - fo).max() < 1e-5
+    assert abs(e - eo) < 5e-8 * len(x)
+    assert g.half_pairs()[0].shape[0] == len(o.pairs()[0])
+    assert np.abs(FH - FHo).max() < 2e-7 * len(x)
