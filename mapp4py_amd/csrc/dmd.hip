@@ -611,13 +611,14 @@ struct NbPacked {
 };
 
 // pass 1 of site i: rho of every component (smeared r*rho_ba) and the pair
-// energy (smeared r*phi); only table functions 0 and 2 are read
+// energy (smeared r*phi); only table functions 0 and 2 are read. Lane g of the
+// 2^lg that share the site.
 template <int B, class Src, class Nb>
 __device__ inline void pass1_site(int i, const double4* __restrict__ x, const double* __restrict__ al,
                                   const double* __restrict__ cc, const int* __restrict__ el,
                                   const int* __restrict__ nn, const uint32_t* __restrict__ list, int ldl, int maxn,
                                   const DmdArgs& A, const BoxDev& bd, int energy_only, const Src& T, const Nb& nb,
-                                  double* __restrict__ E, double* __restrict__ dE, double (&acc)[2])
+                                  double* __restrict__ E, double* __restrict__ dE, double (&acc)[2], int lg, int g)
 {
     const int ks[2] = {0, 2};
     const int C = A.C;
@@ -632,7 +633,7 @@ __device__ inline void pass1_site(int i, const double4* __restrict__ x, const do
         const int ei = el[ci_idx];
         double rho = 0.0, ep = 0.0;
         const int cnt = nn[ci_idx];
-        for (int k0 = 0; k0 < cnt; k0 += B) {
+        for (int k0 = 4 * g; k0 < cnt; k0 = next_batch<B>(k0, lg)) {
             uint32_t e[B];
             double4 xj[B];
             double aj[B], cj[B];
@@ -686,16 +687,18 @@ __device__ inline void pass1_site(int i, const double4* __restrict__ x, const do
                 ep += live[b] ? 0.5 * ci * cj[b] * rp0 : 0.0;
             }
         }
+        rho = lane_sum(rho, lg);
+        acc[0] += ep;
+        if (g != 0) continue;
         double F, dF;
         femb5(A, ei, rho, F, dF);
         E[ci_idx] = F;
         dE[ci_idx] = dF;
         nb.put(ci_idx, dF, ei);
         if (!energy_only || ci != 0.0) acc[0] += ci * (F + A.mu0[ei] - 3.0 * A.kBT * log(ai));
-        acc[0] += ep;
         acc[1] += xlogx(ci);
     }
-    acc[1] += xlogx(cv);
+    if (g == 0) acc[1] += xlogx(cv);
 }
 
 // pass 2 of site i: forces on x and alpha, chemical-potential sums, virial.
@@ -712,7 +715,7 @@ __device__ inline void pass2_site(int i, const double4* __restrict__ x, const do
                                   const double* __restrict__ E,
                                   const double* __restrict__ dE, double4* __restrict__ f, double* __restrict__ fa,
                                   double* __restrict__ mu, double4* __restrict__ gu, double* __restrict__ gau,
-                                  const JState& J, double (&acc)[6])
+                                  const JState& J, double (&acc)[6], int lg, int g)
 {
     const int ks[3] = {0, 1, 2};
     const int C = A.C;
@@ -729,6 +732,7 @@ __device__ inline void pass2_site(int i, const double4* __restrict__ x, const do
         const int ci_idx = i * C + ic;
         const double ci = cc[ci_idx];
         if (ci < 0.0) {
+            if (g != 0) continue;
             fa[ci_idx] = 0.0;
             mu[ci_idx] = 0.0;
             if (UNIT) {
@@ -746,7 +750,7 @@ __device__ inline void pass2_site(int i, const double4* __restrict__ x, const do
         const double fcoef = C == 1 ? 1.0 : (c_tot == 0.0 ? (ci == 0.0 ? 1.0 : 0.0) : ci / c_tot);
         double fai = 0.0, mui = 0.0, gai = 0.0, rho = 0.0;
         const int cnt = nn[ci_idx];
-        for (int k0 = 0; k0 < cnt; k0 += B) {
+        for (int k0 = 4 * g; k0 < cnt; k0 = next_batch<B>(k0, lg)) {
             uint32_t e[B];
             double4 xj[B];
             double aj[B], cj[B], dEj[B];
@@ -843,6 +847,13 @@ __device__ inline void pass2_site(int i, const double4* __restrict__ x, const do
                 acc[5] += hf * dz * dz;
             }
         }
+        fai = lane_sum(fai, lg);
+        mui = lane_sum(mui, lg);
+        if (UNIT) {
+            gai = lane_sum(gai, lg);
+            rho = lane_sum(rho, lg);
+        }
+        if (g != 0) continue;
         fa[ci_idx] = fai + 3.0 * A.kBT * ci / ai;
         mu[ci_idx] = E[ci_idx] + mui;
         if (UNIT) {
@@ -851,13 +862,21 @@ __device__ inline void pass2_site(int i, const double4* __restrict__ x, const do
             J.ddE[ci_idx] = ddemb5(A, ei, rho);
         }
     }
-    f[i] = make_double4(fx, fy, fz, 0.0);
-    if (UNIT) gu[i] = make_double4(gx, gy, gz, 0.0);
+    fx = lane_sum(fx, lg);
+    fy = lane_sum(fy, lg);
+    fz = lane_sum(fz, lg);
+    if (g == 0) f[i] = make_double4(fx, fy, fz, 0.0);
+    if (UNIT) {
+        gx = lane_sum(gx, lg);
+        gy = lane_sum(gy, lg);
+        gz = lane_sum(gz, lg);
+        if (g == 0) gu[i] = make_double4(gx, gy, gz, 0.0);
+    }
 }
 
-// the batched passes over the global rows, one site per thread
+// the batched passes over the global rows, 2^lg lanes per site
 template <int B, bool F32>
-__global__ __launch_bounds__(kBlock) void k_dmd_pass1q(int n, const double4* __restrict__ x, const double* __restrict__ al,
+__global__ __launch_bounds__(kBlock) void k_dmd_pass1q(int n, int lg, const double4* __restrict__ x, const double* __restrict__ al,
                                                        const double* __restrict__ cc, const int* __restrict__ el,
                                                        const int* __restrict__ nn, const uint32_t* __restrict__ list,
                                                        int ldl, int maxn, DmdArgs A, BoxDev bd, int energy_only,
@@ -865,16 +884,16 @@ __global__ __launch_bounds__(kBlock) void k_dmd_pass1q(int n, const double4* __r
                                                        double* __restrict__ part)
 {
     const int blk = xcd_block();
-    const int i = blk * kBlock + threadIdx.x;
+    const int i = (int)(((long)blk * kBlock + threadIdx.x) >> lg), g = threadIdx.x & ((1 << lg) - 1);
     double acc[2] = {0.0, 0.0};  // free energy without the kT S term, S
     if (i < n)
         pass1_site<B>(i, x, al, cc, el, nn, list, ldl, maxn, A, bd, energy_only, RowsGlobal<F32>{drows<F32>(A), A.nr},
-                      NbPlain{al, cc, el, dE}, E, dE, acc);
+                      NbPlain{al, cc, el, dE}, E, dE, acc, lg, g);
     block_sum_store<2>(acc, part + (size_t)blk * kPartW);
 }
 
 template <int B, bool UNIT, bool F32>
-__global__ __launch_bounds__(kBlock) void k_dmd_pass2q(int n, const double4* __restrict__ x, const double* __restrict__ al,
+__global__ __launch_bounds__(kBlock) void k_dmd_pass2q(int n, int lg, const double4* __restrict__ x, const double* __restrict__ al,
                                                        const double* __restrict__ cc, const int* __restrict__ el,
                                                        const int* __restrict__ nn, const uint32_t* __restrict__ list,
                                                        int ldl, int maxn, DmdArgs A, BoxDev bd,
@@ -884,24 +903,23 @@ __global__ __launch_bounds__(kBlock) void k_dmd_pass2q(int n, const double4* __r
                                                        double4* __restrict__ gu, double* __restrict__ gau, JState J)
 {
     const int blk = xcd_block();
-    const int i = blk * kBlock + threadIdx.x;
+    const int i = (int)(((long)blk * kBlock + threadIdx.x) >> lg), g = threadIdx.x & ((1 << lg) - 1);
     double acc[6] = {0, 0, 0, 0, 0, 0};
     if (i < n)
         pass2_site<B, UNIT>(i, x, al, cc, el, nn, list, ldl, maxn, A, bd, RowsGlobal<F32>{drows<F32>(A), A.nr},
-                            NbPlain{al, cc, el, dE}, E, dE, f, fa, mu, gu, gau, J, acc);
+                            NbPlain{al, cc, el, dE}, E, dE, f, fa, mu, gu, gau, J, acc, lg, g);
     block_sum_store<6>(acc, part + (size_t)blk * kPartW);
 }
 
 // Persistent passes with the FP32 knots in LDS: one workgroup of NT threads
-// per CU loads the knot window once and walks chunks of NT sites. The chunks
+// per CU loads the knot window once and walks chunks of NT / 2^lg sites. The chunks
 // form 8 contiguous ranges, one per XCD, and the workgroups of an XCD stride
 // through its range side by side (neighbor halos shared in that XCD's L2).
-template <int NT>
 struct SiteWalk {
     int c, end, step;
-    __device__ explicit SiteWalk(int n)
+    __device__ SiteWalk(int n, int size)
     {
-        const int nchunks = (n + NT - 1) / NT;
+        const int nchunks = (n + size - 1) / size;
         const int per = (nchunks + kXcd - 1) / kXcd;
         const int xcd = (int)blockIdx.x % kXcd;
         c = xcd * per + (int)blockIdx.x / kXcd;
@@ -931,7 +949,7 @@ __global__ __launch_bounds__(kBlock) void k_pack_ac(int nc, const double* __rest
 }
 
 template <int B, int NT>
-__global__ __launch_bounds__(NT) void k_dmd_pass1k(int n, const double4* __restrict__ x, const double* __restrict__ al,
+__global__ __launch_bounds__(NT) void k_dmd_pass1k(int n, int lg, const double4* __restrict__ x, const double* __restrict__ al,
                                                    const double* __restrict__ cc, const int* __restrict__ el,
                                                    const int* __restrict__ nn, const uint32_t* __restrict__ list,
                                                    int ldl, int maxn, DmdArgs A, BoxDev bd, KnotArgs K,
@@ -944,15 +962,16 @@ __global__ __launch_bounds__(NT) void k_dmd_pass1k(int n, const double4* __restr
     const KnotsLds T = load_knots<NT>(K, knot_win, knot_fn);
     const NbPacked nb{ac, el, ed};
     double acc[2] = {0.0, 0.0};
-    for (SiteWalk<NT> w(n); w.c < w.end; w.c += w.step) {
-        const int i = w.c * NT + (int)threadIdx.x;
-        if (i < n) pass1_site<B>(i, x, al, cc, el, nn, list, ldl, maxn, A, bd, energy_only, T, nb, E, dE, acc);
+    const int size = NT >> lg, g = threadIdx.x & ((1 << lg) - 1);
+    for (SiteWalk w(n, size); w.c < w.end; w.c += w.step) {
+        const int i = w.c * size + (int)(threadIdx.x >> lg);
+        if (i < n) pass1_site<B>(i, x, al, cc, el, nn, list, ldl, maxn, A, bd, energy_only, T, nb, E, dE, acc, lg, g);
     }
     block_sum_store<2, NT>(acc, part + (size_t)blockIdx.x * kPartW);
 }
 
 template <int B, int NT>
-__global__ __launch_bounds__(NT) void k_dmd_pass2k(int n, const double4* __restrict__ x, const double* __restrict__ al,
+__global__ __launch_bounds__(NT) void k_dmd_pass2k(int n, int lg, const double4* __restrict__ x, const double* __restrict__ al,
                                                    const double* __restrict__ cc, const int* __restrict__ el,
                                                    const int* __restrict__ nn, const uint32_t* __restrict__ list,
                                                    int ldl, int maxn, DmdArgs A, BoxDev bd, KnotArgs K,
@@ -966,11 +985,12 @@ __global__ __launch_bounds__(NT) void k_dmd_pass2k(int n, const double4* __restr
     const KnotsLds T = load_knots<NT>(K, knot_win, knot_fn);
     const NbPacked nb{ac, el, ed};
     double acc[6] = {0, 0, 0, 0, 0, 0};
-    for (SiteWalk<NT> w(n); w.c < w.end; w.c += w.step) {
-        const int i = w.c * NT + (int)threadIdx.x;
+    const int size = NT >> lg, g = threadIdx.x & ((1 << lg) - 1);
+    for (SiteWalk w(n, size); w.c < w.end; w.c += w.step) {
+        const int i = w.c * size + (int)(threadIdx.x >> lg);
         if (i < n)
             pass2_site<B, false>(i, x, al, cc, el, nn, list, ldl, maxn, A, bd, T, nb, E, dE, f, fa, mu, nullptr,
-                                 nullptr, JState{}, acc);
+                                 nullptr, JState{}, acc, lg, g);
     }
     block_sum_store<6, NT>(acc, part + (size_t)blockIdx.x * kPartW);
 }
@@ -1000,7 +1020,7 @@ __device__ inline void exchange_q(double gamma_i, double gamma_j, double mu_ji, 
 // One thread per component; the owner sums every exchange of its component
 // from its own side (the rate of a pair seen from the other side is minus
 // this one: the barrier there is Q - mu_ji). Partial max |c_d| per workgroup.
-__global__ __launch_bounds__(kBlock) void k_dmd_cd(int nc, const double4* __restrict__ x, const double* __restrict__ al,
+__global__ __launch_bounds__(kBlock) void k_dmd_cd(int nc, int lg, const double4* __restrict__ x, const double* __restrict__ al,
                                                    const double* __restrict__ cc, const int* __restrict__ el,
                                                    const int* __restrict__ nn, const uint32_t* __restrict__ list,
                                                    int ldl, int C, BoxDev bd, CdArgs P,
@@ -1010,7 +1030,7 @@ __global__ __launch_bounds__(kBlock) void k_dmd_cd(int nc, const double4* __rest
 #pragma clang fp contract(off)
     __shared__ double sh[kBlock];
     const int blk = xcd_block();
-    const int ic = blk * kBlock + threadIdx.x;
+    const int ic = (int)(((long)blk * kBlock + threadIdx.x) >> lg), g = threadIdx.x & ((1 << lg) - 1);
     double dci = 0.0;
     if (ic < nc) {
         const double ci = cc[ic];
@@ -1025,7 +1045,7 @@ __global__ __launch_bounds__(kBlock) void k_dmd_cd(int nc, const double4* __rest
             }
             const double zeta = P.zeta[ei], c1 = P.c1[ei], rsq_crd = P.rsq_crd[ei];
             const int cnt = nn[ic];
-            for (int k = 0; k < cnt; ++k) {
+            for (int k = g; k < cnt; k += 1 << lg) {
                 const uint32_t e = list[(size_t)k * ldl + ic];
                 const int jc = (int)(e & kIndexMask);
                 if (el[jc] != ei) continue;
@@ -1049,7 +1069,8 @@ __global__ __launch_bounds__(kBlock) void k_dmd_cd(int nc, const double4* __rest
                                 cc[jc] * cv_i * exp(0.5 * mu_ji) / (alpha_sq_j * alpha_j));
             }
         }
-        cd[ic] = dci;
+        dci = lane_sum(dci, lg);
+        if (g == 0) cd[ic] = dci;
     }
     sh[threadIdx.x] = fabs(dci);
     __syncthreads();
@@ -1176,15 +1197,18 @@ __global__ __launch_bounds__(kBlock) void k_dmd_jrp(int n, const double4* __rest
 // the second list with the exchange coefficients of the state. Each
 // component keeps its own exchanges; seen from j a term is minus this one
 // (coef0 and M0 are symmetric in i and j, d_i and d_j trade places).
-__global__ __launch_bounds__(kBlock) void k_dmd_jex(int nc, const double4* __restrict__ x, const double* __restrict__ al,
+__global__ __launch_bounds__(kBlock) void k_dmd_jex(int nc, int lg, const double4* __restrict__ x, const double* __restrict__ al,
                                                     const double* __restrict__ cc, const int* __restrict__ el,
                                                     const int* __restrict__ nn, const uint32_t* __restrict__ list,
                                                     int ldl, int C, BoxDev bd, CdArgs P,
                                                     const double* __restrict__ mu, JState J)
 {
 #pragma clang fp contract(off)
-    const int ic = xcd_block() * kBlock + threadIdx.x;
+    const int ic = (int)(((long)xcd_block() * kBlock + threadIdx.x) >> lg);
     if (ic >= nc) return;
+    // a group's lanes look at neighboring entries; its ballot gives each
+    // exchange its place in the second list
+    const int G = 1 << lg, g = threadIdx.x & (G - 1), base = (threadIdx.x & 63) & ~(G - 1);
     const double ci = cc[ic];
     double S0 = 0.0, S1 = 0.0, S2 = 0.0;
     int m = 0;
@@ -1199,14 +1223,22 @@ __global__ __launch_bounds__(kBlock) void k_dmd_jex(int nc, const double4* __res
         }
         const double zeta = P.zeta[ei], c1 = P.c1[ei], rsq_crd = P.rsq_crd[ei];
         const int cnt = nn[ic];
-        for (int k = 0; k < cnt; ++k) {
-            const uint32_t e = list[(size_t)k * ldl + ic];
+        for (int k0 = 0; k0 < cnt; k0 += G) {
+            const int k = k0 + g;
+            const uint32_t e = list[(size_t)(k < cnt ? k : cnt - 1) * ldl + ic];
             const int jc = (int)(e & kIndexMask);
-            if (el[jc] != ei) continue;
-            double dx, dy, dz;
-            dpair_dx(xi, x[jc / C], e >> kIndexBits, bd.h, dx, dy, dz);
-            const double rsq = dx * dx + (dy * dy + dz * dz);
-            if (rsq >= rsq_crd) continue;
+            bool in = k < cnt && el[jc] == ei;
+            double rsq = 0.0;
+            if (in) {
+                double dx, dy, dz;
+                dpair_dx(xi, x[jc / C], e >> kIndexBits, bd.h, dx, dy, dz);
+                rsq = dx * dx + (dy * dy + dz * dz);
+                in = rsq < rsq_crd;
+            }
+            const unsigned hits = (unsigned)(__ballot(in) >> base) & ((1u << G) - 1u);
+            const size_t slot = (size_t)(m + __popc(hits & ((1u << g) - 1u))) * ldl + ic;
+            m += __popc(hits);
+            if (!in) continue;
             const double alpha_j = al[jc], alpha_sq_j = alpha_j * alpha_j;
             const double gamma_i = rsq / (zeta * alpha_sq_i), gamma_j = rsq / (zeta * alpha_sq_j);
             const double mu_ji = P.beta * (mu[jc] - mu_i);
@@ -1224,7 +1256,6 @@ __global__ __launch_bounds__(kBlock) void k_dmd_jex(int nc, const double4* __res
             const double d_i = exp(-0.5 * mu_ji) / (alpha_sq_i * alpha_i);
             const double d_j = exp(0.5 * mu_ji) / (alpha_sq_j * alpha_j);
             const double M0 = P.beta * (theta_i * ci * cv_j * d_i - theta_j * cj * cv_i * d_j);
-            const size_t slot = (size_t)m * ldl + ic;
             J.idx2[slot] = (uint32_t)jc;
             J.f0[slot] = coef0 * M0;
             J.f1[slot] = coef0 * d_i * ci;
@@ -1232,9 +1263,12 @@ __global__ __launch_bounds__(kBlock) void k_dmd_jex(int nc, const double4* __res
             S0 += coef0 * M0;
             S1 += coef0 * d_i * cv_j;
             S2 += coef0 * d_j * cj;
-            ++m;
         }
     }
+    S0 = lane_sum(S0, lg);
+    S1 = lane_sum(S1, lg);
+    S2 = lane_sum(S2, lg);
+    if (g != 0) return;
     J.cnt2[ic] = m;
     J.S[(size_t)ic * 3] = S0;
     J.S[(size_t)ic * 3 + 1] = S1;
@@ -1245,19 +1279,22 @@ __global__ __launch_bounds__(kBlock) void k_dmd_jex(int nc, const double4* __res
 // of F'(rho_i), times c_i); every component sums its own list (the
 // reference's half list adds the j side of each pair in the same loop). The
 // thread of a site's first component also writes xs of the site.
-__global__ __launch_bounds__(kBlock) void k_dmd_ja1(int nc, int C, const double* __restrict__ cc, int ldl, JState J,
+__global__ __launch_bounds__(kBlock) void k_dmd_ja1(int nc, int lg, int C, const double* __restrict__ cc, int ldl, JState J,
                                                     const double* __restrict__ xv, double* __restrict__ a1,
                                                     double* __restrict__ xs)
 {
-    const int ic = xcd_block() * kBlock + threadIdx.x;
+    const int ic = (int)(((long)xcd_block() * kBlock + threadIdx.x) >> lg), g = threadIdx.x & ((1 << lg) - 1);
     if (ic >= nc) return;
     const double ci = cc[ic];
     double s = 0.0;
     const int cnt = J.cnt[ic];
-    for (int k = 0; k < cnt; ++k) {
+#pragma unroll 4
+    for (int k = g; k < cnt; k += 1 << lg) {
         const size_t slot = (size_t)k * ldl + ic;
         s += J.r2[slot] * xv[J.idx[slot]];
     }
+    s = lane_sum(s, lg);
+    if (g != 0) return;
     a1[ic] = ci >= 0.0 ? s * (ci * J.ddE[ic]) : 0.0;
     if (ic % C == 0) {
         double t = 0.0;
@@ -1269,19 +1306,21 @@ __global__ __launch_bounds__(kBlock) void k_dmd_ja1(int nc, int C, const double*
 
 // product, second sum: b0_i = sum_j rho_{i->j} A1_j + t0 x_j, the change of
 // the chemical potential mu_i
-__global__ __launch_bounds__(kBlock) void k_dmd_jb0(int nc, int ldl, JState J, const double* __restrict__ a1,
+__global__ __launch_bounds__(kBlock) void k_dmd_jb0(int nc, int lg, int ldl, JState J, const double* __restrict__ a1,
                                                     const double* __restrict__ xv, double* __restrict__ b0)
 {
-    const int ic = xcd_block() * kBlock + threadIdx.x;
+    const int ic = (int)(((long)xcd_block() * kBlock + threadIdx.x) >> lg), g = threadIdx.x & ((1 << lg) - 1);
     if (ic >= nc) return;
     double s = 0.0;
     const int cnt = J.cnt[ic];
-    for (int k = 0; k < cnt; ++k) {
+#pragma unroll 4
+    for (int k = g; k < cnt; k += 1 << lg) {
         const size_t slot = (size_t)k * ldl + ic;
         const uint32_t jc = J.idx[slot];
         s += J.r1[slot] * a1[jc] + J.t0[slot] * xv[jc];
     }
-    b0[ic] = s;
+    s = lane_sum(s, lg);
+    if (g == 0) b0[ic] = s;
 }
 
 // product over the second list (src/ff_eam_dmd.cpp:1536-1572)
@@ -2233,7 +2272,7 @@ DMDSystem::DMDSystem(std::shared_ptr<EamForceField> ff, int nsites, int c_dim, i
     keys_.reserve(n_); keys_alt_.reserve(n_); vals_.reserve(n_); vals_alt_.reserve(n_);
     nn_.reserve(nc_);
     flags_.reserve(4);
-    part_.reserve((size_t)2 * grid_for(std::max(n_, nc_)) * kPartW + 64);
+    part_.reserve((size_t)2 * part_rows() * kPartW + 64);
     red_.reserve(64);
     red2_.reserve(256 * kPartW);
     std::vector<double4> xh(n_);
@@ -2469,13 +2508,53 @@ void DMDSystem::stage_surrogate()
 constexpr int knot_nt1(int B) { return B == 4 ? 512 : 1024; }
 constexpr int kKnotNT2 = 512;
 
+// log2 of the lanes that share a row of n sites or components in the passes
+// over global tables: as many as keep `threads` threads in flight. The FP64
+// passes hold about two waves a SIMD, the list walks eight.
+int DMDSystem::lanes(int n, int threads)
+{
+    int lg = 0;
+    while (lg < 4 && ((long)n << (lg + 1)) <= threads) ++lg;
+    return lg;
+}
+// rows of half the partial-sum buffer
+int DMDSystem::part_rows() const
+{
+    return std::max(grid_for(std::max(n_, nc_)), (std::max(kPassThreads, kWalkThreads) / kBlock + kXcd));
+}
+
+// the same for the LDS passes of nt threads a workgroup: the fewest rounds of
+// 4-entry batches over the CUs, with the site's own work as one more
+int DMDSystem::lanes_knots(int nt) const
+{
+    const int batches = (int)((maxn_ - 16) / 1.25 / 4.0) + 1;  // a component's expected row
+    int best = 0;
+    long least = 0;
+    for (int lg = 0; lg <= 3; ++lg) {
+        const int size = nt >> lg;
+        const long chunks = (n_ + size - 1) / size;
+        const long cost = ((chunks + knot_grid_ - 1) / knot_grid_) * (((batches - 1) >> lg) + (lg ? 3 : 2));
+        if (lg == 0 || cost < least) {
+            least = cost;
+            best = lg;
+        }
+    }
+    return best;
+}
+// workgroups of the LDS passes: at most one per CU, one per chunk
+int DMDSystem::knot_blocks(int nt, int lg) const
+{
+    const int size = nt >> lg, chunks = (n_ + size - 1) / size;
+    return std::min(knot_grid_, (chunks + kXcd - 1) / kXcd * kXcd);
+}
+
 void DMDSystem::pass1(bool energy_only, int f32)
 {
     BoxDev bd;
     std::memcpy(bd.h, box_.h, sizeof bd.h);
     std::memcpy(bd.b, box_.b, sizeof bd.b);
     if (f32 == 1 && knots_ok_ && !surr_ && batch_ != 1) {
-        const int nb = std::min(knot_grid_, grid_for(n_));
+        const int nt = batch_ == 4 ? knot_nt1(4) : knot_nt1(2), lg = lanes_knots(nt), nb = knot_blocks(nt, lg);
         ac_.reserve(nc_);
         ed_.reserve(nc_);
         prof_.begin(energy_only ? K_DMD_ENERGY : K_DMD_PASS1, stream_);
@@ -2483,11 +2562,11 @@ void DMDSystem::pass1(bool energy_only, int f32)
                            c_.get(), ac_.get());
         if (batch_ == 4)
             hipLaunchKernelGGL((k_dmd_pass1k<4, knot_nt1(4)>), dim3(nb), dim3(knot_nt1(4)), knot_lds_, stream_, n_,
-                               x_.get(), al_.get(), c_.get(), el_.get(), nn_.get(), list_.get(), ldl_, maxn_, A_, bd,
+                               lg, x_.get(), al_.get(), c_.get(), el_.get(), nn_.get(), list_.get(), ldl_, maxn_, A_, bd,
                                kn_, ac_.get(), ed_.get(), energy_only ? 1 : 0, E_.get(), dE_.get(), part_.get());
         else
             hipLaunchKernelGGL((k_dmd_pass1k<2, knot_nt1(2)>), dim3(nb), dim3(knot_nt1(2)), knot_lds_, stream_, n_,
-                               x_.get(), al_.get(), c_.get(), el_.get(), nn_.get(), list_.get(), ldl_, maxn_, A_, bd,
+                               lg, x_.get(), al_.get(), c_.get(), el_.get(), nn_.get(), list_.get(), ldl_, maxn_, A_, bd,
                                kn_, ac_.get(), ed_.get(), energy_only ? 1 : 0, E_.get(), dE_.get(), part_.get());
         prof_.end(stream_);
         reduce_rows(part_.get(), nb, 2, red_.get());
@@ -2495,7 +2574,9 @@ void DMDSystem::pass1(bool energy_only, int f32)
         return;
     }
     ed_ver_ = -1;
-    const int nb = grid_for(n_);
+    // the per-pair loops (surrogate, batch 1) keep one thread per site
+    const int lg = surr_ || batch_ == 1 ? 0 : lanes(n_, kPassThreads);
+    const int nb = grid_lanes(n_, lg);
     SurrogateArgs S{};
     if (surr_) {
         stage_surrogate();
@@ -2511,7 +2592,7 @@ void DMDSystem::pass1(bool energy_only, int f32)
                            el_.get(), nn_.get(), list_.get(), ldl_, A_, bd, S, energy_only ? 1 : 0, E_.get(),
                            dE_.get(), part_.get());
     else {
-#define MAPP_P1(B, F) hipLaunchKernelGGL((k_dmd_pass1q<B, F>), dim3(nb), dim3(kBlock), 0, stream_, n_, x_.get(), \
+#define MAPP_P1(B, F) hipLaunchKernelGGL((k_dmd_pass1q<B, F>), dim3(nb), dim3(kBlock), 0, stream_, n_, lg, x_.get(), \
                                          al_.get(), c_.get(), el_.get(), nn_.get(), list_.get(), ldl_, maxn_, A_, bd, \
                                          energy_only ? 1 : 0, E_.get(), dE_.get(), part_.get())
         if (batch_ == 2) {
@@ -2527,17 +2608,18 @@ void DMDSystem::pass1(bool energy_only, int f32)
 
 void DMDSystem::pass2(bool unit, int f32)
 {
-    const int nb = grid_for(n_);
+    const int lg = surr_ || (batch_ == 1 && !unit) ? 0 : lanes(n_, kPassThreads);
+    const int nb = grid_lanes(n_, lg);
     BoxDev bd;
     std::memcpy(bd.h, box_.h, sizeof bd.h);
     std::memcpy(bd.b, box_.b, sizeof bd.b);
-    double* p2 = part_.get() + (size_t)nb * kPartW;
+    double* p2 = part_.get() + (size_t)part_rows() * kPartW;
     if (f32 == 1 && knots_ok_ && !surr_ && !unit && batch_ != 1) {
         // the packed records of pass 1 of this state (pass 2 follows pass 1)
         MAPP_REQUIRE(ed_ver_ == ver_, ERR_STATE, "the FP32-knot pass 2 needs pass 1 of the same state");
-        const int nbk = std::min(knot_grid_, nb);
+        const int lgk = lanes_knots(kKnotNT2), nbk = knot_blocks(kKnotNT2, lgk);
         prof_.begin(K_DMD_PASS2, stream_);
-        hipLaunchKernelGGL((k_dmd_pass2k<2, kKnotNT2>), dim3(nbk), dim3(kKnotNT2), knot_lds_, stream_, n_, x_.get(),
+        hipLaunchKernelGGL((k_dmd_pass2k<2, kKnotNT2>), dim3(nbk), dim3(kKnotNT2), knot_lds_, stream_, n_, lgk, x_.get(),
                            al_.get(), c_.get(), el_.get(), nn_.get(), list_.get(), ldl_, maxn_, A_, bd, kn_, ac_.get(),
                            ed_.get(), E_.get(), dE_.get(), f_.get(), fa_.get(), mu_.get(), p2);
         prof_.end(stream_);
@@ -2555,7 +2637,7 @@ void DMDSystem::pass2(bool unit, int f32)
         gu_.reserve(n_);
         gau_.reserve(nc_);
         j_reserve();
-        hipLaunchKernelGGL((k_dmd_pass2q<4, true, false>), dim3(nb), dim3(kBlock), 0, stream_, n_, x_.get(), al_.get(),
+        hipLaunchKernelGGL((k_dmd_pass2q<4, true, false>), dim3(nb), dim3(kBlock), 0, stream_, n_, lg, x_.get(), al_.get(),
                            c_.get(), el_.get(), nn_.get(), list_.get(), ldl_, maxn_, A_, bd, E_.get(), dE_.get(),
                            f_.get(), fa_.get(), mu_.get(), p2, gu_.get(), gau_.get(), jstate());
         gu_ver_ = ver_;
@@ -2565,7 +2647,7 @@ void DMDSystem::pass2(bool unit, int f32)
                            el_.get(), nn_.get(), list_.get(), ldl_, A_, bd, S, E_.get(), dE_.get(), f_.get(),
                            fa_.get(), mu_.get(), p2);
     else {
-#define MAPP_P2(B, F) hipLaunchKernelGGL((k_dmd_pass2q<B, false, F>), dim3(nb), dim3(kBlock), 0, stream_, n_, \
+#define MAPP_P2(B, F) hipLaunchKernelGGL((k_dmd_pass2q<B, false, F>), dim3(nb), dim3(kBlock), 0, stream_, n_, lg, \
                                          x_.get(), al_.get(), c_.get(), el_.get(), nn_.get(), list_.get(), ldl_, maxn_, \
                                          A_, bd, E_.get(), dE_.get(), f_.get(), fa_.get(), mu_.get(), p2, nullptr, \
                                          nullptr, JState{})
@@ -2684,9 +2766,9 @@ double DMDSystem::c_d(const double* r_crd, const double* zeta, double* c_d_host)
     BoxDev bd;
     std::memcpy(bd.h, box_.h, sizeof bd.h);
     std::memcpy(bd.b, box_.b, sizeof bd.b);
-    const int nb = grid_for(nc_);
+    const int lg = lanes(nc_, kWalkThreads), nb = grid_lanes(nc_, lg);
     prof_.begin(K_DMD_CD, stream_);
-    hipLaunchKernelGGL(k_dmd_cd, dim3(nb), dim3(kBlock), 0, stream_, nc_, x_.get(), al_.get(), c_.get(), el_.get(),
+    hipLaunchKernelGGL(k_dmd_cd, dim3(nb), dim3(kBlock), 0, stream_, nc_, lg, x_.get(), al_.get(), c_.get(), el_.get(),
                        nn_.get(), list_.get(), ldl_, C_, bd, P, mu_.get(), cd_.get(), part_.get());
     hipLaunchKernelGGL(k_extrema_rows, dim3(1), dim3(kBlock), 0, stream_, nb, 1, 0, part_.get(), red_.get() + 40);
     prof_.end(stream_);
@@ -2744,7 +2826,8 @@ void DMDSystem::J_prepare()
     if (jslot_ver_ != ver_)  // the slot values come with c_d's second pass; else a pass of their own
         hipLaunchKernelGGL(k_dmd_jrp<4>, dim3(grid_for(n_)), dim3(kBlock), 0, stream_, n_, x_.get(), al_.get(),
                            c_.get(), el_.get(), nn_.get(), list_.get(), ldl_, maxn_, A_, bd, jdE_.get(), jstate());
-    hipLaunchKernelGGL(k_dmd_jex, dim3(grid_for(nc_)), dim3(kBlock), 0, stream_, nc_, x_.get(), al_.get(), c_.get(),
+    const int lg = lanes(nc_, kWalkThreads);
+    hipLaunchKernelGGL(k_dmd_jex, dim3(grid_lanes(nc_, lg)), dim3(kBlock), 0, stream_, nc_, lg, x_.get(), al_.get(), c_.get(),
                        el_.get(), nn_.get(), list_.get(), ldl_, C_, bd, jP_, jmu_.get(), jstate());
     prof_.end(stream_);
     jrp_ver_ = ver_;
@@ -2787,9 +2870,10 @@ void DMDSystem::J_dev(const double* x, double* ax)
     const int nbc = grid_for(nc_);
     const JState js = jstate();
     prof_.begin(K_DMD_J, stream_);
-    hipLaunchKernelGGL(k_dmd_ja1, dim3(nbc), dim3(kBlock), 0, stream_, nc_, C_, c_.get(), ldl_, js, x, ja1_.get(),
+    const int lg = lanes(nc_, kWalkThreads), nbl = grid_lanes(nc_, lg);
+    hipLaunchKernelGGL(k_dmd_ja1, dim3(nbl), dim3(kBlock), 0, stream_, nc_, lg, C_, c_.get(), ldl_, js, x, ja1_.get(),
                        jxs_.get());
-    hipLaunchKernelGGL(k_dmd_jb0, dim3(nbc), dim3(kBlock), 0, stream_, nc_, ldl_, js, ja1_.get(), x, jb0_.get());
+    hipLaunchKernelGGL(k_dmd_jb0, dim3(nbl), dim3(kBlock), 0, stream_, nc_, lg, ldl_, js, ja1_.get(), x, jb0_.get());
     hipLaunchKernelGGL(k_dmd_jax, dim3(nbc), dim3(kBlock), 0, stream_, nc_, C_, ldl_, js, jb0_.get(), x, jxs_.get(),
                        ax);
     prof_.end(stream_);

@@ -243,6 +243,12 @@ private:
     bool knots_ok_ = false;
     size_t knot_lds_ = 0;
     int knot_grid_ = 0;
+    // lanes that share a row (log2), and the threads to fill
+    static constexpr int kPassThreads = 262144, kWalkThreads = 524288;
+    static int lanes(int n, int threads);
+    int part_rows() const;
+    int lanes_knots(int nt) const;
+    int knot_blocks(int nt, int lg) const;
     // their passes' packed neighbor records: (alpha, c), and (F', element)
     // from pass 1 of state ed_ver_
     DevBuf<double2> ac_, ed_;

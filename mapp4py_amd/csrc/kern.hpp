@@ -119,6 +119,28 @@ __global__ __launch_bounds__(kBlock) void k_reduce_rows(int nrows, int ncols, co
 
 
 
+// Lanes sharing an atom (or a site): 2^lg neighboring lanes take the batches
+// of its row in turn and meet in a butterfly, so that a small system still
+// fills the chip (one lane an atom leaves most CUs without work below 262,144
+// atoms). Every lane of the group ends with the same sum.
+template <class T>
+__device__ inline T lane_sum(T v, int lg)
+{
+    for (int o = 1; o < (1 << lg); o <<= 1) v += __shfl_xor(v, o, 64);
+    return v;
+}
+
+// The lanes take the entries in blocks of 4 whatever the batch length B is, so
+// the sums do not depend on it: entry after k0's batch of a lane.
+template <int B>
+__device__ inline int next_batch(int k0, int lg)
+{
+    return k0 + B + (B >= 4 || ((k0 + B) & 3) == 0 ? (4 << lg) - 4 : 0);
+}
+
+// workgroups of kBlock threads for n items of 2^lg lanes each
+inline int grid_lanes(int n, int lg) { return (int)((((long)n << lg) + kXcd * kBlock - 1) / (kXcd * kBlock)) * kXcd; }
+
 __device__ inline int cell_coord(double s, int nc)
 {
     int c = (int)(s * (double)nc);

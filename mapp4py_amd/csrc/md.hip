@@ -489,25 +489,6 @@ __global__ __launch_bounds__(kBlock) void k_make_records(int n, const double4* _
                         (unsigned)__double2ll_rn(xi.z * R.inv_q), (unsigned)(int)xi.w);
 }
 
-// Lanes sharing an atom: 2^lg neighboring lanes take the batches of its row
-// in turn and meet in a butterfly, so that a small system still fills the
-// chip (one lane an atom leaves most CUs without work below 262,144 atoms).
-// Every lane of the group ends with the same sum.
-template <class T>
-__device__ inline T lane_sum(T v, int lg)
-{
-    for (int o = 1; o < (1 << lg); o <<= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
-
-// The lanes take the entries in blocks of 4 whatever the batch length B is, so
-// the sums do not depend on it: entry after k0's batch of a lane.
-template <int B>
-__device__ inline int next_batch(int k0, int lg)
-{
-    return k0 + B + (B >= 4 || ((k0 + B) & 3) == 0 ? (4 << lg) - 4 : 0);
-}
-
 // pass 1 per atom: rho_i = sum_j rho_{j->i}(r_ij), an FP64 sum of FP32 spline
 // values, over the batches of lane g of the 2^lg that share the atom. Tab
 // supplies the spline rows (global table or an LDS window).
@@ -1672,7 +1653,7 @@ void MDSystem::build_list()
         MAPP_HIP(hipMemsetAsync(flags_.get(), 0, sizeof(int), stream_));
         prof_.begin(K_BUILD_LIST, stream_);
         if (const int lg = lanes_global(); lg > 0) {
-            const int ng = (int)((((long)n_ << lg) + kXcd * kBlock - 1) / (kXcd * kBlock)) * kXcd;
+            const int ng = grid_lanes(n_, lg);
 #define MAPP_BUILD(ONE) hipLaunchKernelGGL(k_build_list_group<ONE>, dim3(ng), dim3(kBlock), 0, stream_, n_, lg, \
                                            s_.get(), rec_.get(), r16_, bd, g, cell_rank_.get(), cell_start_.get(), \
                                            ordered_ ? cell_order_.get() : nullptr, maxn_ / 4, ldl_, list_.get(), \
@@ -1787,7 +1768,7 @@ void MDSystem::force_passes(const KickArgs* kick, bool records_fresh, float4* f_
         return;
     }
     const int lg = lanes_global();
-    const int nb = (int)((((long)n_ << lg) + kXcd * kBlock - 1) / (kXcd * kBlock)) * kXcd;
+    const int nb = grid_lanes(n_, lg);
     const int br = lg && batch_rho_ > 4 ? 4 : batch_rho_, bf = lg && batch_force_ > 4 ? 4 : batch_force_;
 #define MAPP_RHO(B, ONE) hipLaunchKernelGGL((k_eam_rho<B, ONE>), dim3(nb), dim3(kBlock), 0, stream_, n_, lg, stop, \
                                             rec_.get(), nn_.get(), list4(), ldl_, maxb, P, r16_, ro, xr_.get(), \
