@@ -192,6 +192,7 @@ __device__ inline void dpair_dx(const double4& xi, const double4& xj, uint32_t c
 // surrogate staging must take identical decisions pair by pair.
 struct PairGeo {
     double dx, dy, dz, r, a;
+    double rinv, ainv;
     bool live;
 };
 
@@ -201,8 +202,10 @@ __device__ inline PairGeo pair_geo(const double4& xi, const double4& xj, uint32_
 #pragma clang fp contract(off)
     PairGeo g;
     dpair_dx(xi, xj, code, h, g.dx, g.dy, g.dz);
-    g.r = sqrt(g.dx * g.dx + g.dy * g.dy + g.dz * g.dz);
-    g.a = sqrt(ai * ai + aj * aj);
+    // both roots come with their reciprocals (about 50 cycles; a correctly
+    // rounded root takes 88 and a division 68)
+    root_inv(g.dx * g.dx + g.dy * g.dy + g.dz * g.dz, g.r, g.rinv);
+    root_inv(ai * ai + aj * aj, g.a, g.ainv);
     g.live = g.r - g.a * xmax < cut;
     return g;
 }
@@ -464,7 +467,7 @@ __device__ inline int dknot(const DmdArgs& A, double u, double& p)
 // the offset p in [0, 1] contributes to every function of the interval, and
 // eval(c, basis) is the interval's cubic there. Acc1 and Acc2 are the types
 // in which passes 1 and 2 sum the Hermite points of one pair into its
-// moments, and recip is the reciprocal of a pair's distance and width.
+// moments.
 
 // coefficient rows [ne*ne][nr][3] in global memory, FP64 or FP32
 template <bool F32>
@@ -488,31 +491,39 @@ struct RowsGlobal {
     using Basis = double;
     __device__ static Basis basis(double p) { return p; }
     __device__ static double eval(const Row& c, double p) { return hv(c, p); }
-    __device__ static double recip(double v) { return 1.0 / v; }
 };
 
-// FP32 knots. Every table function is the Hermite cubic of its interval's
-// two knot values and slopes per unit offset (c2 = 3 dy - 2 s0 - s1,
-// c3 = s0 + s1 - 2 dy, as the spline builder makes them), so one (value,
-// slope) pair per knot holds a function in 8 bytes per knot, and an interval
-// is two adjacent pairs. Only the distinct functions are kept: fn maps
-// (element pair, function) to one of them. The top nwin knots of every
-// distinct function sit in LDS; intervals below m_lo read the global copy.
-// A random 16-byte row from L2 costs the vector cache one tag lookup per
-// lane; from LDS a few bank cycles. The cubic is evaluated in the Hermite
-// basis, y0 + (y1 - y0) h1 + s0 h2 + s1 h3, with h1..h3 of the offset shared
-// by the three functions. Pass 2 sums one pair's Hermite points in FP32;
-// pass 1, whose pair terms make the free energy, and both passes' sums over
-// pairs stay FP64.
+// Knots. Every table function is the Hermite cubic of its interval's two knot
+// values and slopes per unit offset (c2 = 3 dy - 2 s0 - s1, c3 = s0 + s1 -
+// 2 dy, as the spline builder makes them), so one (value, slope) pair per knot
+// holds a function in 8 bytes per knot (FP32) or 16 (FP64), and an interval is
+// two adjacent pairs. Only the distinct functions are kept: fn maps (element
+// pair, function) to one of them. The top nwin knots of every distinct
+// function sit in LDS; intervals below m_lo read the global copy. A random row
+// from L2 costs the vector cache one tag lookup per lane and load; from LDS a
+// few bank cycles, and where a part of a wave's lanes falls below the window
+// only those lanes are looked up. The cubic is evaluated in the Hermite basis,
+// y0 + (y1 - y0) h1 + s0 h2 + s1 h3, with h1..h3 of the offset shared by the
+// three functions. FP32: pass 2 sums one pair's Hermite points in FP32; pass 1,
+// whose pair terms make the free energy, and both passes' sums over pairs stay
+// FP64. FP64: 5 functions of 5,000 knots leave 1,996 knots in LDS (r > 3.3 A of
+// 5.5); the cubic from knots differs from the coefficient row's by rounding.
+template <class F>
+struct Pair2 {
+    F x, y;
+};
+template <class F>
 struct KnotsLds {
-    using Row = float4;  // y0, s0, y1, s1
-    const float2* glob;  // [nf][nr]
-    const float2* win;   // [nf][nwin], LDS
-    const int* fn;       // [ne*ne*3], LDS
+    struct Row {
+        F y0, s0, y1, s1;
+    };
+    const Pair2<F>* glob;  // [nf][nr]
+    const Pair2<F>* win;   // [nf][nwin], LDS
+    const int* fn;         // [ne*ne*3], LDS
     int nr, nwin, m_lo;
     template <int B, int K>
     __device__ void fetch(const int (&ks)[K], const int (&tt)[B], const int (&m)[B], const bool (&live)[B],
-                          float4 (&c)[B][K]) const
+                          Row (&c)[B][K]) const
     {
         bool low[B], any = false;
 #pragma unroll
@@ -523,9 +534,9 @@ struct KnotsLds {
             const int r = live[b] && !low[b] ? m[b] - m_lo : 0;
 #pragma unroll
             for (int j = 0; j < K; ++j) {
-                const float2* q = win + fn[tt[b] * 3 + ks[j]] * nwin + r;
-                const float2 a = q[0], d = q[1];
-                c[b][j] = make_float4(a.x, a.y, d.x, d.y);
+                const Pair2<F>* q = win + fn[tt[b] * 3 + ks[j]] * nwin + r;
+                const Pair2<F> a = q[0], d = q[1];
+                c[b][j] = Row{a.x, a.y, d.x, d.y};
             }
         }
         if (__ballot(any) != 0ull) {
@@ -534,32 +545,25 @@ struct KnotsLds {
                 if (low[b])
 #pragma unroll
                     for (int j = 0; j < K; ++j) {
-                        const float2* q = glob + (size_t)fn[tt[b] * 3 + ks[j]] * nr + m[b];
-                        const float2 a = q[0], d = q[1];
-                        c[b][j] = make_float4(a.x, a.y, d.x, d.y);
+                        const Pair2<F>* q = glob + (size_t)fn[tt[b] * 3 + ks[j]] * nr + m[b];
+                        const Pair2<F> a = q[0], d = q[1];
+                        c[b][j] = Row{a.x, a.y, d.x, d.y};
                     }
         }
     }
     using Acc1 = double;
-    using Acc2 = float;
+    using Acc2 = F;
     struct Basis {
-        float h1, h2, h3;
+        F h1, h2, h3;
     };
     __device__ static Basis basis(double p)
     {
-        const float q = (float)p, q1 = 1.0f - q, q2 = q * q;
-        return Basis{q2 * (3.0f - 2.0f * q), q * q1 * q1, -q2 * q1};
+        const F q = (F)p, q1 = (F)1 - q, q2 = q * q;
+        return Basis{q2 * ((F)3 - (F)2 * q), q * q1 * q1, -q2 * q1};
     }
-    __device__ static float eval(const float4& c, const Basis& h)
+    __device__ static F eval(const Row& c, const Basis& h)
     {
-        return c.x + (c.z - c.x) * h.h1 + c.y * h.h2 + c.w * h.h3;
-    }
-    // the hardware reciprocal and one Newton step (squares its relative
-    // error), in place of the correctly rounded division
-    __device__ static double recip(double v)
-    {
-        const double y = __builtin_amdgcn_rcp(v);
-        return fma(fma(-v, y, 1.0), y, y);
+        return c.y0 + (c.y1 - c.y0) * h.h1 + c.s0 * h.h2 + c.s1 * h.h3;
     }
 };
 
@@ -681,7 +685,7 @@ __device__ inline void pass1_site(int i, const double4* __restrict__ x, const do
             }
 #pragma unroll
             for (int b = 0; b < B; ++b) {
-                const double rinv = Src::recip(pg[b].r);
+                const double rinv = pg[b].rinv;
                 const double rp0 = kPiInSq * rinv * (double)H0[b], rp2 = kPiInSq * rinv * (double)H2[b];
                 rho += live[b] ? cj[b] * rp2 : 0.0;
                 ep += live[b] ? 0.5 * ci * cj[b] * rp0 : 0.0;
@@ -805,7 +809,7 @@ __device__ inline void pass2_site(int i, const double4* __restrict__ x, const do
             }
 #pragma unroll
             for (int b = 0; b < B; ++b) {
-                const double rinv = Src::recip(pg[b].r), ainv = Src::recip(pg[b].a);
+                const double rinv = pg[b].rinv, ainv = pg[b].ainv;
                 double rp[3], drr[3], dal[3];
 #pragma unroll
                 for (int k = 0; k < 3; ++k) {
@@ -928,16 +932,25 @@ struct SiteWalk {
     }
 };
 
-template <int NT>
-__device__ inline KnotsLds load_knots(const KnotArgs& K, float2* win, int* fn)
+// the knots of table type F, and the window in the workgroup's LDS
+extern __shared__ __align__(16) unsigned char knot_lds[];
+template <class F, int NT>
+__device__ inline KnotsLds<F> load_knots(const KnotArgs& K, int* fn)
 {
-    for (int r = threadIdx.x; r < K.nf * K.nwin; r += NT) {
-        const int q = r / K.nwin;
-        win[r] = K.glob[(size_t)q * K.nr + K.m_lo + (r - q * K.nwin)];
-    }
+    const Pair2<F>* glob = static_cast<const Pair2<F>*>(K.glob);
+    Pair2<F>* win = reinterpret_cast<Pair2<F>*>(knot_lds);
+    for (int q = 0; q < K.nf; ++q)
+        for (int r0 = threadIdx.x; r0 < K.nwin; r0 += 4 * NT) {
+            Pair2<F> t[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) t[u] = glob[(size_t)q * K.nr + K.m_lo + min(r0 + u * NT, K.nwin - 1)];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (r0 + u * NT < K.nwin) win[q * K.nwin + r0 + u * NT] = t[u];
+        }
     for (int t = threadIdx.x; t < K.nfn; t += NT) fn[t] = K.fn[t];
     __syncthreads();
-    return KnotsLds{K.glob, win, fn, K.nr, K.nwin, K.m_lo};
+    return KnotsLds<F>{glob, win, fn, K.nr, K.nwin, K.m_lo};
 }
 
 // (alpha, c) of every component in one record for the LDS passes
@@ -948,7 +961,7 @@ __global__ __launch_bounds__(kBlock) void k_pack_ac(int nc, const double* __rest
     if (k < nc) ac[k] = make_double2(al[k], cc[k]);
 }
 
-template <int B, int NT>
+template <class F, int B, int NT>
 __global__ __launch_bounds__(NT) void k_dmd_pass1k(int n, int lg, const double4* __restrict__ x, const double* __restrict__ al,
                                                    const double* __restrict__ cc, const int* __restrict__ el,
                                                    const int* __restrict__ nn, const uint32_t* __restrict__ list,
@@ -957,9 +970,8 @@ __global__ __launch_bounds__(NT) void k_dmd_pass1k(int n, int lg, const double4*
                                                    int energy_only, double* __restrict__ E, double* __restrict__ dE,
                                                    double* __restrict__ part)
 {
-    extern __shared__ float2 knot_win[];
     __shared__ int knot_fn[kMaxElems * kMaxElems * 3];
-    const KnotsLds T = load_knots<NT>(K, knot_win, knot_fn);
+    const KnotsLds<F> T = load_knots<F, NT>(K, knot_fn);
     const NbPacked nb{ac, el, ed};
     double acc[2] = {0.0, 0.0};
     const int size = NT >> lg, g = threadIdx.x & ((1 << lg) - 1);
@@ -970,7 +982,7 @@ __global__ __launch_bounds__(NT) void k_dmd_pass1k(int n, int lg, const double4*
     block_sum_store<2, NT>(acc, part + (size_t)blockIdx.x * kPartW);
 }
 
-template <int B, int NT>
+template <class F, int B, int NT, bool UNIT>
 __global__ __launch_bounds__(NT) void k_dmd_pass2k(int n, int lg, const double4* __restrict__ x, const double* __restrict__ al,
                                                    const double* __restrict__ cc, const int* __restrict__ el,
                                                    const int* __restrict__ nn, const uint32_t* __restrict__ list,
@@ -978,19 +990,19 @@ __global__ __launch_bounds__(NT) void k_dmd_pass2k(int n, int lg, const double4*
                                                    const double2* __restrict__ ac, double2* __restrict__ ed,
                                                    const double* __restrict__ E, const double* __restrict__ dE,
                                                    double4* __restrict__ f, double* __restrict__ fa,
-                                                   double* __restrict__ mu, double* __restrict__ part)
+                                                   double* __restrict__ mu, double* __restrict__ part,
+                                                   double4* __restrict__ gu, double* __restrict__ gau, JState J)
 {
-    extern __shared__ float2 knot_win[];
     __shared__ int knot_fn[kMaxElems * kMaxElems * 3];
-    const KnotsLds T = load_knots<NT>(K, knot_win, knot_fn);
+    const KnotsLds<F> T = load_knots<F, NT>(K, knot_fn);
     const NbPacked nb{ac, el, ed};
     double acc[6] = {0, 0, 0, 0, 0, 0};
     const int size = NT >> lg, g = threadIdx.x & ((1 << lg) - 1);
     for (SiteWalk w(n, size); w.c < w.end; w.c += w.step) {
         const int i = w.c * size + (int)(threadIdx.x >> lg);
         if (i < n)
-            pass2_site<B, false>(i, x, al, cc, el, nn, list, ldl, maxn, A, bd, T, nb, E, dE, f, fa, mu, nullptr,
-                                 nullptr, JState{}, acc, lg, g);
+            pass2_site<B, UNIT>(i, x, al, cc, el, nn, list, ldl, maxn, A, bd, T, nb, E, dE, f, fa, mu, gu, gau, J, acc,
+                                lg, g);
     }
     block_sum_store<6, NT>(acc, part + (size_t)blockIdx.x * kPartW);
 }
@@ -1169,7 +1181,7 @@ __global__ __launch_bounds__(kBlock) void k_dmd_jrp(int n, const double4* __rest
             for (int b = 0; b < B; ++b) {
                 if (k0 + b >= cnt) continue;
                 const int jc = (int)(e[b] & kIndexMask);
-                const double rinv = 1.0 / pg[b].r;
+                const double rinv = pg[b].rinv;
                 const double v0 = live[b] ? kPiInSq * rinv * H[b][0] : 0.0;
                 const double v1 = live[b] ? kPiInSq * rinv * H[b][1] : 0.0;
                 const double v2 = live[b] ? kPiInSq * rinv * H[b][2] : 0.0;
@@ -1280,7 +1292,7 @@ __global__ __launch_bounds__(kBlock) void k_dmd_jex(int nc, int lg, const double
 // reference's half list adds the j side of each pair in the same loop). The
 // thread of a site's first component also writes xs of the site.
 __global__ __launch_bounds__(kBlock) void k_dmd_ja1(int nc, int lg, int C, const double* __restrict__ cc, int ldl, JState J,
-                                                    const double* __restrict__ xv, double* __restrict__ a1,
+                                                    const double* __restrict__ xv, double2* __restrict__ a1x,
                                                     double* __restrict__ xs)
 {
     const int ic = (int)(((long)xcd_block() * kBlock + threadIdx.x) >> lg), g = threadIdx.x & ((1 << lg) - 1);
@@ -1295,7 +1307,8 @@ __global__ __launch_bounds__(kBlock) void k_dmd_ja1(int nc, int lg, int C, const
     }
     s = lane_sum(s, lg);
     if (g != 0) return;
-    a1[ic] = ci >= 0.0 ? s * (ci * J.ddE[ic]) : 0.0;
+    // A1 and x in one record: the second sum gathers both at once
+    a1x[ic] = make_double2(ci >= 0.0 ? s * (ci * J.ddE[ic]) : 0.0, xv[ic]);
     if (ic % C == 0) {
         double t = 0.0;
         for (int q = 0; q < C; ++q)
@@ -1306,8 +1319,8 @@ __global__ __launch_bounds__(kBlock) void k_dmd_ja1(int nc, int lg, int C, const
 
 // product, second sum: b0_i = sum_j rho_{i->j} A1_j + t0 x_j, the change of
 // the chemical potential mu_i
-__global__ __launch_bounds__(kBlock) void k_dmd_jb0(int nc, int lg, int ldl, JState J, const double* __restrict__ a1,
-                                                    const double* __restrict__ xv, double* __restrict__ b0)
+__global__ __launch_bounds__(kBlock) void k_dmd_jb0(int nc, int lg, int ldl, JState J, const double2* __restrict__ a1x,
+                                                    double* __restrict__ b0)
 {
     const int ic = (int)(((long)xcd_block() * kBlock + threadIdx.x) >> lg), g = threadIdx.x & ((1 << lg) - 1);
     if (ic >= nc) return;
@@ -1316,8 +1329,8 @@ __global__ __launch_bounds__(kBlock) void k_dmd_jb0(int nc, int lg, int ldl, JSt
 #pragma unroll 4
     for (int k = g; k < cnt; k += 1 << lg) {
         const size_t slot = (size_t)k * ldl + ic;
-        const uint32_t jc = J.idx[slot];
-        s += J.r1[slot] * a1[jc] + J.t0[slot] * xv[jc];
+        const double2 v = a1x[J.idx[slot]];
+        s += J.r1[slot] * v.x + J.t0[slot] * v.y;
     }
     s = lane_sum(s, lg);
     if (g == 0) b0[ic] = s;
@@ -2505,7 +2518,6 @@ void DMDSystem::stage_surrogate()
 // workgroup, and 262,144 sites over 256 x 768 threads leave a third of the
 // workgroups a second chunk (measured 1.49 against 1.13 ms); one entry in
 // 1024 threads measured 1.42 ms, four entries spill.
-constexpr int knot_nt1(int B) { return B == 4 ? 512 : 1024; }
 constexpr int kKnotNT2 = 512;
 
 // log2 of the lanes that share a row of n sites or components in the passes
@@ -2522,6 +2534,9 @@ int DMDSystem::part_rows() const
 {
     return std::max(grid_for(std::max(n_, nc_)), (std::max(kPassThreads, kWalkThreads) / kBlock + kXcd));
 }
+
+// the batched passes from knots in LDS: FP32 (mode 1) or FP64 (mode 0)
+bool DMDSystem::use_knots(int f32) const { return f32 != 2 && knots_ok_ && !surr_ && batch_ != 1; }
 
 // the same for the LDS passes of nt threads a workgroup: the fewest rounds of
 // 4-entry batches over the CUs, with the site's own work as one more
@@ -2553,21 +2568,23 @@ void DMDSystem::pass1(bool energy_only, int f32)
     BoxDev bd;
     std::memcpy(bd.h, box_.h, sizeof bd.h);
     std::memcpy(bd.b, box_.b, sizeof bd.b);
-    if (f32 == 1 && knots_ok_ && !surr_ && batch_ != 1) {
-        const int nt = batch_ == 4 ? knot_nt1(4) : knot_nt1(2), lg = lanes_knots(nt), nb = knot_blocks(nt, lg);
+    if (use_knots(f32)) {
+        const int nt = batch_ == 4 || f32 == 0 ? 512 : 1024, lg = lanes_knots(nt), nb = knot_blocks(nt, lg);
         ac_.reserve(nc_);
         ed_.reserve(nc_);
         prof_.begin(energy_only ? K_DMD_ENERGY : K_DMD_PASS1, stream_);
         hipLaunchKernelGGL(k_pack_ac, dim3((nc_ + kBlock - 1) / kBlock), dim3(kBlock), 0, stream_, nc_, al_.get(),
                            c_.get(), ac_.get());
-        if (batch_ == 4)
-            hipLaunchKernelGGL((k_dmd_pass1k<4, knot_nt1(4)>), dim3(nb), dim3(knot_nt1(4)), knot_lds_, stream_, n_,
-                               lg, x_.get(), al_.get(), c_.get(), el_.get(), nn_.get(), list_.get(), ldl_, maxn_, A_, bd,
-                               kn_, ac_.get(), ed_.get(), energy_only ? 1 : 0, E_.get(), dE_.get(), part_.get());
-        else
-            hipLaunchKernelGGL((k_dmd_pass1k<2, knot_nt1(2)>), dim3(nb), dim3(knot_nt1(2)), knot_lds_, stream_, n_,
-                               lg, x_.get(), al_.get(), c_.get(), el_.get(), nn_.get(), list_.get(), ldl_, maxn_, A_, bd,
-                               kn_, ac_.get(), ed_.get(), energy_only ? 1 : 0, E_.get(), dE_.get(), part_.get());
+#define MAPP_P1(F, B, NT) hipLaunchKernelGGL((k_dmd_pass1k<F, B, NT>), dim3(nb), dim3(NT), kn_[f32 == 0].lds, stream_, \
+                                             n_, lg, x_.get(), al_.get(), c_.get(), el_.get(), nn_.get(), list_.get(), \
+                                             ldl_, maxn_, A_, bd, kn_[f32 == 0], ac_.get(), ed_.get(), \
+                                             energy_only ? 1 : 0, E_.get(), dE_.get(), part_.get())
+        if (f32 == 0) {
+            if (batch_ == 4) MAPP_P1(double, 4, 512); else MAPP_P1(double, 2, 512);
+        } else {
+            if (batch_ == 4) MAPP_P1(float, 4, 512); else MAPP_P1(float, 2, 1024);
+        }
+#undef MAPP_P1
         prof_.end(stream_);
         reduce_rows(part_.get(), nb, 2, red_.get());
         ed_ver_ = ver_;
@@ -2614,14 +2631,28 @@ void DMDSystem::pass2(bool unit, int f32)
     std::memcpy(bd.h, box_.h, sizeof bd.h);
     std::memcpy(bd.b, box_.b, sizeof bd.b);
     double* p2 = part_.get() + (size_t)part_rows() * kPartW;
-    if (f32 == 1 && knots_ok_ && !surr_ && !unit && batch_ != 1) {
+    if (unit) {
+        gu_.reserve(n_);
+        gau_.reserve(nc_);
+        j_reserve();
+        gu_ver_ = ver_;
+        jslot_ver_ = ver_;
+    }
+    if (use_knots(f32) && !(unit && f32 == 1)) {
         // the packed records of pass 1 of this state (pass 2 follows pass 1)
-        MAPP_REQUIRE(ed_ver_ == ver_, ERR_STATE, "the FP32-knot pass 2 needs pass 1 of the same state");
+        MAPP_REQUIRE(ed_ver_ == ver_, ERR_STATE, "the knot passes' pass 2 needs pass 1 of the same state");
         const int lgk = lanes_knots(kKnotNT2), nbk = knot_blocks(kKnotNT2, lgk);
         prof_.begin(K_DMD_PASS2, stream_);
-        hipLaunchKernelGGL((k_dmd_pass2k<2, kKnotNT2>), dim3(nbk), dim3(kKnotNT2), knot_lds_, stream_, n_, lgk, x_.get(),
-                           al_.get(), c_.get(), el_.get(), nn_.get(), list_.get(), ldl_, maxn_, A_, bd, kn_, ac_.get(),
-                           ed_.get(), E_.get(), dE_.get(), f_.get(), fa_.get(), mu_.get(), p2);
+#define MAPP_P2(F, UNIT) hipLaunchKernelGGL((k_dmd_pass2k<F, 2, kKnotNT2, UNIT>), dim3(nbk), dim3(kKnotNT2), \
+                                            kn_[f32 == 0].lds, stream_, n_, lgk, x_.get(), al_.get(), c_.get(), \
+                                            el_.get(), nn_.get(), list_.get(), ldl_, maxn_, A_, bd, kn_[f32 == 0], \
+                                            ac_.get(), ed_.get(), E_.get(), dE_.get(), f_.get(), fa_.get(), mu_.get(), \
+                                            p2, unit ? gu_.get() : nullptr, unit ? gau_.get() : nullptr, \
+                                            unit ? jstate() : JState{})
+        if (f32 == 1) MAPP_P2(float, false);
+        else if (unit) MAPP_P2(double, true);
+        else MAPP_P2(double, false);
+#undef MAPP_P2
         prof_.end(stream_);
         reduce_rows(p2, nbk, 6, red_.get() + 8);
         return;
@@ -2634,14 +2665,9 @@ void DMDSystem::pass2(bool unit, int f32)
                            el_.get(), nn_.get(), list_.get(), ldl_, A_, bd, S, E_.get(), dE_.get(), f_.get(),
                            fa_.get(), mu_.get(), p2);
     else if (unit) {
-        gu_.reserve(n_);
-        gau_.reserve(nc_);
-        j_reserve();
         hipLaunchKernelGGL((k_dmd_pass2q<4, true, false>), dim3(nb), dim3(kBlock), 0, stream_, n_, lg, x_.get(), al_.get(),
                            c_.get(), el_.get(), nn_.get(), list_.get(), ldl_, maxn_, A_, bd, E_.get(), dE_.get(),
                            f_.get(), fa_.get(), mu_.get(), p2, gu_.get(), gau_.get(), jstate());
-        gu_ver_ = ver_;
-        jslot_ver_ = ver_;
     } else if (batch_ == 1)
         hipLaunchKernelGGL(k_dmd_pass2<false>, dim3(nb), dim3(kBlock), 0, stream_, n_, x_.get(), al_.get(), c_.get(),
                            el_.get(), nn_.get(), list_.get(), ldl_, A_, bd, S, E_.get(), dE_.get(), f_.get(),
@@ -2668,9 +2694,9 @@ void DMDSystem::set_f32(int mode)
     f32_ = mode;
 }
 
-// FP32 knots for the LDS passes. Each table function's interval cubic must
+// FP32 and FP64 knots for the LDS passes. Each table function's interval cubic must
 // be the Hermite cubic of its two knots' values and slopes (what the spline
-// builder makes); a table that is not stays on the FP32 rows. Equal functions
+// builder makes); a table that is not stays on the rows. Equal functions
 // (the density of one element seen from every pair of an eam/alloy table)
 // are kept once, and the window is the top knots that fit the workgroup LDS
 // beside the passes' static arrays.
@@ -2704,23 +2730,36 @@ void DMDSystem::plan_knots()
     MAPP_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
     // room for the passes' static LDS: the slot map and the block reduction
     const long budget = (long)lds_max - 4096;
-    const int nwin = (int)std::min<long>(nr, budget / (8L * nf));
-    if (nwin < 2 || ncu < 1) return;
-    std::vector<float2> g((size_t)nf * nr);
-    for (int q = 0; q < nf; ++q)
-        for (int m = 0; m < nr; ++m)
-            g[(size_t)q * nr + m] = make_float2((float)uniq[q][2 * (size_t)m], (float)uniq[q][2 * (size_t)m + 1]);
-    knots_.reserve(g.size());
-    MAPP_HIP(hipMemcpy(knots_.get(), g.data(), g.size() * sizeof(float2), hipMemcpyHostToDevice));
+    if (ncu < 1) return;
     knot_fn_.reserve(fn.size());
     MAPP_HIP(hipMemcpy(knot_fn_.get(), fn.data(), fn.size() * sizeof(int), hipMemcpyHostToDevice));
-    kn_ = KnotArgs{knots_.get(), knot_fn_.get(), nf, nr, nwin, nr - nwin, (int)fn.size()};
-    knot_lds_ = (size_t)nf * nwin * sizeof(float2);
+    for (int f64 = 0; f64 < 2; ++f64) {
+        const long bytes = f64 ? 16 : 8;
+        const int nwin = (int)std::min<long>(nr, budget / (bytes * nf));
+        if (nwin < 2) return;
+        std::vector<unsigned char> g((size_t)nf * nr * bytes);
+        for (int q = 0; q < nf; ++q)
+            for (int m = 0; m < 2 * nr; ++m) {
+                const double v = uniq[q][m];
+                const float vf = (float)v;
+                std::memcpy(&g[((size_t)q * nr * 2 + m) * (bytes / 2)], f64 ? (const void*)&v : (const void*)&vf, bytes / 2);
+            }
+        knots_[f64].reserve(g.size());
+        MAPP_HIP(hipMemcpy(knots_[f64].get(), g.data(), g.size(), hipMemcpyHostToDevice));
+        kn_[f64] = KnotArgs{knots_[f64].get(), knot_fn_.get(), nf, nr, nwin, nr - nwin, (int)fn.size(),
+                            (size_t)nf * nwin * bytes};
+    }
     knot_grid_ = std::max(1, ncu / kXcd) * kXcd;
-    const void* fns[] = {(const void*)k_dmd_pass1k<2, knot_nt1(2)>, (const void*)k_dmd_pass1k<4, knot_nt1(4)>,
-                         (const void*)k_dmd_pass2k<2, kKnotNT2>};
-    for (const void* f : fns)
-        if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)knot_lds_) != hipSuccess) {
+    const std::pair<const void*, int> fns[] = {{(const void*)k_dmd_pass1k<float, 2, 1024>, 0},
+                                               {(const void*)k_dmd_pass1k<float, 4, 512>, 0},
+                                               {(const void*)k_dmd_pass1k<double, 2, 512>, 1},
+                                               {(const void*)k_dmd_pass1k<double, 4, 512>, 1},
+                                               {(const void*)k_dmd_pass2k<float, 2, kKnotNT2, false>, 0},
+                                               {(const void*)k_dmd_pass2k<double, 2, kKnotNT2, false>, 1},
+                                               {(const void*)k_dmd_pass2k<double, 2, kKnotNT2, true>, 1}};
+    for (const auto& f : fns)
+        if (hipFuncSetAttribute(f.first, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kn_[f.second].lds) !=
+            hipSuccess) {
             (void)hipGetLastError();
             return;
         }
@@ -2873,7 +2912,7 @@ void DMDSystem::J_dev(const double* x, double* ax)
     const int lg = lanes(nc_, kWalkThreads), nbl = grid_lanes(nc_, lg);
     hipLaunchKernelGGL(k_dmd_ja1, dim3(nbl), dim3(kBlock), 0, stream_, nc_, lg, C_, c_.get(), ldl_, js, x, ja1_.get(),
                        jxs_.get());
-    hipLaunchKernelGGL(k_dmd_jb0, dim3(nbl), dim3(kBlock), 0, stream_, nc_, lg, ldl_, js, ja1_.get(), x, jb0_.get());
+    hipLaunchKernelGGL(k_dmd_jb0, dim3(nbl), dim3(kBlock), 0, stream_, nc_, lg, ldl_, js, ja1_.get(), jb0_.get());
     hipLaunchKernelGGL(k_dmd_jax, dim3(nbc), dim3(kBlock), 0, stream_, nc_, C_, ldl_, js, jb0_.get(), x, jxs_.get(),
                        ax);
     prof_.end(stream_);

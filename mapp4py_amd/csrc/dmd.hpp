@@ -26,14 +26,15 @@ struct DmdArgs {
     const double* F5;    // [ne][nrho][5], quartic embedding
 };
 
-// FP32 knots of the LDS passes: the distinct table functions as (value,
+// Knots of the LDS passes: the distinct table functions as (value,
 // slope per unit offset) pairs [nf][nr], the distinct function of each
 // (element pair, function) slot [nfn = ne*ne*3], and the knot window
 // m_lo .. nr-1 (nwin knots per function) the workgroups hold in LDS
 struct KnotArgs {
-    const float2* glob;
+    const void* glob;  // (value, slope) pairs, FP32 or FP64
     const int* fn;
     int nf, nr, nwin, m_lo, nfn;
+    size_t lds;        // bytes of the window
 };
 
 
@@ -92,7 +93,7 @@ public:
     int f32() const { return f32_; }
     // whether mode 1 holds the knots in LDS, and the window's first knot
     bool knots_in_lds() const { return knots_ok_; }
-    int knot_window_first() const { return kn_.m_lo; }
+    int knot_window_first() const { return kn_[0].m_lo; }
     ~DMDSystem();
 
     int nsites() const { return n_; }
@@ -213,7 +214,8 @@ private:
     DevBuf<uint32_t> jidx_, jidx2_;   // list entries / second list, slot-major
     DevBuf<double> jr2_, jr1_, jt0_, jf0_, jf1_, jf2_, jS_;
     DevBuf<int> jcnt_, jcnt2_;
-    DevBuf<double> jx_, ja1_, jb0_, jax_, jxs_;
+    DevBuf<double> jx_, jb0_, jax_, jxs_;
+    DevBuf<double2> ja1_;  // A1 and x of a product
     // implicit-step vectors (slot order) and the Krylov basis [m+1][nc]
     DevBuf<double> nt_a_, nt_F_, nt_del_, nt_c0_, nt_red_;
     GmresWork nt_gm_;
@@ -237,16 +239,16 @@ private:
     int batch_ = 4;                  // quadrature pass batch: 1 (per-pair loop), 2 or 4 list entries
     int f32_ = 0;                    // table mode of derivative / value (set_f32)
     // FP32 knots and their LDS window (plan_knots)
-    DevBuf<float2> knots_;
+    DevBuf<unsigned char> knots_[2];  // FP32, FP64
     DevBuf<int> knot_fn_;
-    KnotArgs kn_{};
+    KnotArgs kn_[2] = {};
     bool knots_ok_ = false;
-    size_t knot_lds_ = 0;
     int knot_grid_ = 0;
     // lanes that share a row (log2), and the threads to fill
     static constexpr int kPassThreads = 262144, kWalkThreads = 524288;
     static int lanes(int n, int threads);
     int part_rows() const;
+    bool use_knots(int f32) const;
     int lanes_knots(int nt) const;
     int knot_blocks(int nt, int lg) const;
     // their passes' packed neighbor records: (alpha, c), and (F', element)

@@ -158,6 +158,18 @@ __device__ inline double root64(double rsq)
     return fma(e, (double)(0.5f / rf), r0);
 }
 
+// r = sqrt(x) and 1 / r to an ulp or so: the hardware's reciprocal root
+// (about 24 bits), one third-order step for the inverse, one for the root
+__device__ inline void root_inv(double x, double& r, double& r_inv)
+{
+    double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-(x * y), y, 1.0);
+    y = fma(y * e, fma(0.375, e, 0.5), y);
+    const double t = x * y;
+    r = fma(fma(-t, t, x), 0.5 * y, t);
+    r_inv = y;
+}
+
 inline uint32_t morton3(uint32_t a, uint32_t b, uint32_t c)
 {
     auto spread = [](uint32_t v) {

@@ -59,18 +59,6 @@ __device__ inline void spline_at(double v, double inv, int n, int& m, double& p)
     m = mm;
 }
 
-// r = sqrt(x) and 1 / r to an ulp or so: the hardware's reciprocal root
-// (about 24 bits), one third-order step for the inverse, one for the root
-__device__ inline void root_inv(double x, double& r, double& r_inv)
-{
-    double y = __builtin_amdgcn_rsq(x);
-    const double e = fma(-(x * y), y, 1.0);
-    y = fma(y * e, fma(0.375, e, 0.5), y);
-    const double t = x * y;
-    r = fma(fma(-t, t, x), 0.5 * y, t);
-    r_inv = y;
-}
-
 __device__ inline int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
 __device__ inline double uni(double v)
 {
