@@ -154,6 +154,8 @@ __global__ __launch_bounds__(kBlock) void k_cell_order(int ncells, GridArgs g, c
 // each, exact integer separations. Only a pair within the quantisation band
 // of the cut-off (a few 1e-8 A wide) is decided by the FP64 predicate on s,
 // so the neighbor set is that of the predicate for every pair.
+// eord: the list of the alloy passes, its columns in element order (column c is
+// slot eord[c]) and the neighbor's element in each entry.
 // ONE: a single element, so the cut-offs are kernel-argument scalars; with
 // several, the element pairs' cut-offs are read from LDS (an indexed
 // kernel-argument array would cost a memory round trip per candidate).
@@ -202,12 +204,13 @@ __global__ __launch_bounds__(kBlock) void k_build_list(int n, const double4* __r
                                                        const int* __restrict__ cell_start,
                                                        const uint4* __restrict__ order, int maxb, int ldl,
                                                        uint4* __restrict__ list4, int* __restrict__ nn,
-                                                       int* __restrict__ flags)
+                                                       int* __restrict__ flags, const int* __restrict__ eord)
 {
     __shared__ double cut_lds[3][kMaxElems * kMaxElems];
     stage_cuts<ONE>(g, cut_lds);
-    const int i = xcd_block() * kBlock + threadIdx.x;
-    if (i >= n) return;
+    const int col = xcd_block() * kBlock + threadIdx.x;
+    if (col >= n) return;
+    const int i = !ONE && eord ? eord[col] : col;
     const double4 si = s4[i];
     const uint4 ri = rec[i];
     const int ti = (int)si.w;
@@ -237,14 +240,14 @@ __global__ __launch_bounds__(kBlock) void k_build_list(int n, const double4* __r
             if (self_img && j == i) continue;
             const bool in = listed(rs, rj, j, n0, n1, n2);
             if (in) {
-                const uint32_t e = (uint32_t)j | code;
+                const uint32_t e = (uint32_t)j | code | (!ONE && eord ? rj.w << kElemShift : 0u);
                 const int q = cnt & 3;
                 p0 = q == 0 ? e : p0;
                 p1 = q == 1 ? e : p1;
                 p2 = q == 2 ? e : p2;
                 p3 = q == 3 ? e : p3;
                 ++cnt;
-                if (q == 3 && (cnt >> 2) <= maxb) list4[(size_t)((cnt >> 2) - 1) * ldl + i] = make_uint4(p0, p1, p2, p3);
+                if (q == 3 && (cnt >> 2) <= maxb) list4[(size_t)((cnt >> 2) - 1) * ldl + col] = make_uint4(p0, p1, p2, p3);
             }
         }
     };
@@ -267,7 +270,7 @@ __global__ __launch_bounds__(kBlock) void k_build_list(int n, const double4* __r
                 for (int o0 = -g.R[0]; o0 <= g.R[0]; ++o0) scan(o0, o1, o2);
     }
     // the last, partly filled block (its entries past cnt are never read)
-    if ((cnt & 3) != 0 && (cnt >> 2) < maxb) list4[(size_t)(cnt >> 2) * ldl + i] = make_uint4(p0, p1, p2, p3);
+    if ((cnt & 3) != 0 && (cnt >> 2) < maxb) list4[(size_t)(cnt >> 2) * ldl + col] = make_uint4(p0, p1, p2, p3);
     nn[i] = cnt;
     if (cnt > 4 * maxb) atomicMax(&flags[FL_OVER], cnt);
 }
@@ -283,14 +286,15 @@ __global__ __launch_bounds__(kBlock) void k_build_list_group(int n, int lg, cons
                                                              const int* __restrict__ cell_start,
                                                              const uint4* __restrict__ order, int maxb, int ldl,
                                                              uint32_t* __restrict__ list, int* __restrict__ nn,
-                                                             int* __restrict__ flags)
+                                                             int* __restrict__ flags, const int* __restrict__ eord)
 {
     __shared__ double cut_lds[3][kMaxElems * kMaxElems];
     stage_cuts<ONE>(g, cut_lds);
     const int G = 1 << lg, gl = threadIdx.x & (G - 1);
     const int base = (threadIdx.x & 63) & ~(G - 1);  // the group's first lane of the wave
-    const int i = (int)(((long)xcd_block() * kBlock + threadIdx.x) >> lg);
-    if (i >= n) return;
+    const int col = (int)(((long)xcd_block() * kBlock + threadIdx.x) >> lg);
+    if (col >= n) return;
+    const int i = !ONE && eord ? eord[col] : col;
     const double4 si = s4[i];
     const uint4 ri = rec[i];
     const int ti = (int)si.w;
@@ -311,12 +315,13 @@ __global__ __launch_bounds__(kBlock) void k_build_list_group(int n, int lg, cons
         const uint4 rs = make_uint4(ri.x - sh.x, ri.y - sh.y, ri.z - sh.z, 0u);
         for (int j0 = jb; j0 < je; j0 += G) {
             const int j = j0 + gl;
-            const bool in =
-                j < je && !(self_img && j == i) && listed(rs, rec[j < je ? j : i], j < je ? j : i, n0, n1, n2);
+            const uint4 rj = rec[j < je ? j : i];
+            const bool in = j < je && !(self_img && j == i) && listed(rs, rj, j < je ? j : i, n0, n1, n2);
             const unsigned hits = (unsigned)(__ballot(in) >> base) & ((1u << G) - 1u);
             const int pos = cnt + __popc(hits & ((1u << gl) - 1u));
             if (in && (pos >> 2) < maxb)
-                list[((size_t)(pos >> 2) * ldl + i) * 4 + (pos & 3)] = (uint32_t)j | (img << kIndexBits);
+                list[((size_t)(pos >> 2) * ldl + col) * 4 + (pos & 3)] =
+                    (uint32_t)j | (img << kIndexBits) | (!ONE && eord ? rj.w << kElemShift : 0u);
             cnt += __popc(hits);
         }
     };
@@ -392,16 +397,19 @@ __device__ inline void embed(const EamArgs& P, int t, double rho, double& F, dou
 // arithmetic is kept to what the result needs (FP32 splines and reciprocal
 // root, FP64 where a sum or the spline abscissa needs it).
 
-// entries k0 .. k0+G-1 of slot i, G = 1, 2 or a multiple of 4 and k0 a
+__device__ inline uint32_t self_entry(int i) { return (uint32_t)i | ((uint32_t)kZeroImage << kIndexBits); }
+// the neighbor's element in an entry of the alloy passes' list
+__device__ inline int entry_elem(uint32_t e) { return (int)(e >> kElemShift & (kAlloyElems - 1)); }
+
+// entries k0 .. k0+G-1 of column i, G = 1, 2 or a multiple of 4 and k0 a
 // multiple of G: the G/4 16-byte blocks, or the part of one block that holds
 // them. The loads are unconditional (a block past the capacity maxb is never
 // read: the last block is read again instead) and entries past the row end
-// become the atom itself, zero image.
+// become `self`, the atom itself at the zero image.
 template <int G>
-__device__ inline void list_entries(const uint4* __restrict__ list4, int ldl, int maxb, int k0, int i, int cnt,
-                                    uint32_t (&e)[G])
+__device__ inline void list_entries(const uint4* __restrict__ list4, int ldl, int maxb, int k0, int i, uint32_t self,
+                                    int cnt, uint32_t (&e)[G])
 {
-    const uint32_t self = (uint32_t)i | ((uint32_t)kZeroImage << kIndexBits);
     if constexpr (G >= 4) {
 #pragma unroll
         for (int q = 0; q < G / 4; ++q) {
@@ -493,32 +501,33 @@ __global__ __launch_bounds__(kBlock) void k_make_records(int n, const double4* _
 // values, over the batches of lane g of the 2^lg that share the atom. Tab
 // supplies the spline rows (global table or an LDS window).
 template <int B, bool ONE, class Tab>
-__device__ inline double rho_atom(int i, const uint4& ri, int cnt, const uint4* __restrict__ rec,
+__device__ inline double rho_atom(int col, uint32_t self, const uint4& ri, int cnt, const uint4* __restrict__ rec,
                                   const uint4* __restrict__ list4, int ldl, int maxb, const EamArgs& P,
                                   const Rec16Frame& R, const Tab& T, int lg, int g)
 {
-    const int ti = ONE ? 0 : (int)ri.w;
+    const int ti = ONE || !Tab::kRows ? 0 : (int)ri.w;
     double rho = 0.0;
     for (int k0 = 4 * g; k0 < cnt; k0 = next_batch<B>(k0, lg)) {
         uint32_t e[B];
         uint4 rj[B];
-        int row[B];
+        int row[B], ej[B];
         float p[B];
         bool in[B];
-        list_entries<B>(list4, ldl, maxb, k0, i, cnt, e);
+        list_entries<B>(list4, ldl, maxb, k0, col, self, cnt, e);
 #pragma unroll
-        for (int b = 0; b < B; ++b) rj[b] = rec[e[b] & kIndexMask];
+        for (int b = 0; b < B; ++b) rj[b] = rec[e[b] & Tab::kMask];
         const bool any_img = wave_has_image(e);
 #pragma unroll
         for (int b = 0; b < B; ++b) {
-            const int tt = ONE ? 0 : ti * P.ne + (int)rj[b].w;
-            const Geo16 g = geo16(ri, rj[b], e[b], any_img, R, R.cut_sq_u[tt], P.nr);
+            ej[b] = ONE ? 0 : Tab::kRows ? (int)rj[b].w : entry_elem(e[b]);
+            const int tt = ONE ? 0 : ti * P.ne + ej[b];
+            const Geo16 g = geo16(ri, rj[b], e[b], any_img, R, T.cut_sq(R, tt, ej[b]), P.nr);
             in[b] = g.in && k0 + b < cnt;
-            row[b] = in[b] ? tt * P.nr + g.m : 0;
+            row[b] = in[b] ? (Tab::kRows ? tt * P.nr : 0) + g.m : 0;
             p[b] = g.p;
         }
         float4 c[B];
-        T.fetch(row, in, c);
+        T.fetch(row, ej, in, c);
 #pragma unroll
         for (int b = 0; b < B; ++b) {
             const float v = ((c[b].w * p[b] + c[b].z) * p[b] + c[b].y) * p[b] + c[b].x;
@@ -530,9 +539,12 @@ __device__ inline double rho_atom(int i, const uint4& ri, int cnt, const uint4* 
 
 // density spline rows from the global table [ne*ne][nr]
 struct RhoRowsGlobal {
+    static constexpr bool kRows = true;
+    static constexpr uint32_t kMask = kIndexMask;
     const float4* tab;
+    __device__ double cut_sq(const Rec16Frame& R, int tt, int) const { return R.cut_sq_u[tt]; }
     template <int B>
-    __device__ void fetch(const int (&row)[B], const bool (&)[B], float4 (&c)[B]) const
+    __device__ void fetch(const int (&row)[B], const int (&)[B], const bool (&)[B], float4 (&c)[B]) const
     {
 #pragma unroll
         for (int b = 0; b < B; ++b) c[b] = *(const float4*)((const char*)tab + (size_t)((uint32_t)row[b] << 4));
@@ -542,11 +554,14 @@ struct RhoRowsGlobal {
 // density spline rows m_lo.. held in LDS (one element); rows below the window,
 // rare in a condensed phase, come from the global table
 struct RhoRowsLds {
+    static constexpr bool kRows = true;
+    static constexpr uint32_t kMask = kIndexMask;
     const float4* tab;
     const float4* win;
     int m_lo;
+    __device__ double cut_sq(const Rec16Frame& R, int tt, int) const { return R.cut_sq_u[tt]; }
     template <int B>
-    __device__ void fetch(const int (&row)[B], const bool (&in)[B], float4 (&c)[B]) const
+    __device__ void fetch(const int (&row)[B], const int (&)[B], const bool (&in)[B], float4 (&c)[B]) const
     {
         bool low[B], any = false;
 #pragma unroll
@@ -572,7 +587,7 @@ struct RhoRowsLds {
 // (coordinates, F'); otherwise the density records (coordinates, element) and
 // F' from dF.
 template <int B, bool ONE, bool EV, class Tab>
-__device__ inline void force_atom(int i, const uint4& ri, int ti, float dFi, int cnt, const uint4* __restrict__ rec,
+__device__ inline void force_atom(int col, uint32_t self, const uint4& ri, int ti, float dFi, int cnt, const uint4* __restrict__ rec,
                                   const uint4* __restrict__ xr, const float* __restrict__ dF,
                                   const uint4* __restrict__ list4, int ldl, int maxb, const EamArgs& P,
                                   const Rec16Frame& R, const Tab& T, int lg, int g0, float& fx, float& fy,
@@ -581,40 +596,41 @@ __device__ inline void force_atom(int i, const uint4& ri, int ti, float dFi, int
     // the list entries of the next batch are loaded one batch ahead (this
     // pass's batches are short, so one memory round trip less per batch pays)
     uint32_t en[B];
-    list_entries<B>(list4, ldl, maxb, 4 * g0, i, cnt, en);
+    list_entries<B>(list4, ldl, maxb, 4 * g0, col, self, cnt, en);
     for (int k0 = 4 * g0; k0 < cnt; k0 = next_batch<B>(k0, lg)) {
         uint32_t e[B];
         uint4 rj[B];
         float dFj[B];
         Geo16 g[B];
-        int row[B];
+        int row[B], ej[B];
         bool in[B];
 #pragma unroll
         for (int b = 0; b < B; ++b) e[b] = en[b];
 #pragma unroll
         for (int b = 0; b < B; ++b) {
-            const uint32_t j = e[b] & kIndexMask;
-            if (ONE) {
+            const uint32_t j = e[b] & Tab::kMask;
+            if (ONE || !Tab::kRows) {
                 rj[b] = xr[j];
             } else {
                 rj[b] = rec[j];
                 dFj[b] = dF[j];
             }
         }
-        list_entries<B>(list4, ldl, maxb, next_batch<B>(k0, lg), i, cnt, en);
+        list_entries<B>(list4, ldl, maxb, next_batch<B>(k0, lg), col, self, cnt, en);
         const bool any_img = wave_has_image(e);
 #pragma unroll
         for (int b = 0; b < B; ++b) {
-            const int tt = ONE ? 0 : ti * P.ne + (int)rj[b].w;
-            g[b] = geo16(ri, rj[b], e[b], any_img, R, R.cut_sq_u[tt], P.nr);
+            ej[b] = ONE ? 0 : Tab::kRows ? (int)rj[b].w : entry_elem(e[b]);
+            const int tt = ONE ? 0 : ti * P.ne + ej[b];
+            g[b] = geo16(ri, rj[b], e[b], any_img, R, T.cut_sq(R, tt, ej[b]), P.nr);
             in[b] = g[b].in && k0 + b < cnt;
-            row[b] = in[b] ? tt * P.nr + g[b].m : 0;
-            if (ONE) dFj[b] = __uint_as_float(rj[b].w);
+            row[b] = in[b] ? (Tab::kRows ? tt * P.nr : 0) + g[b].m : 0;
+            if (ONE || !Tab::kRows) dFj[b] = __uint_as_float(rj[b].w);
         }
         // spline rows: (rho' coefficients at i, r*phi c0), (r*phi c1..c3),
         // and with several elements (rho' coefficients at j)
         float4 ca[B], cz[B], cb[B];
-        T.fetch(row, in, ca, cz, cb);
+        T.fetch(row, ej, in, ca, cz, cb);
 #pragma unroll
         for (int b = 0; b < B; ++b) {
             const float p = g[b].p;
@@ -653,9 +669,12 @@ __device__ inline void force_atom(int i, const uint4& ri, int ti, float dFi, int
 // [ne*ne][nr][3]
 template <bool ONE>
 struct ForceRowsGlobal {
+    static constexpr bool kRows = true;
+    static constexpr uint32_t kMask = kIndexMask;
     const float4* tab;
+    __device__ double cut_sq(const Rec16Frame& R, int tt, int) const { return R.cut_sq_u[tt]; }
     template <int B>
-    __device__ void fetch(const int (&row)[B], const bool (&)[B], float4 (&ca)[B], float4 (&cz)[B],
+    __device__ void fetch(const int (&row)[B], const int (&)[B], const bool (&)[B], float4 (&ca)[B], float4 (&cz)[B],
                           float4 (&cb)[B]) const
     {
 #pragma unroll
@@ -678,13 +697,16 @@ struct ForceRowsGlobal {
 // c0) [nwin] float4, (c1, c2) [nwin] float2, c3 [nwin] float; rows below the
 // window come from the global table
 struct ForceRowsLds {
+    static constexpr bool kRows = true;
+    static constexpr uint32_t kMask = kIndexMask;
     const float4* tab;
     const float4* w4;
     const float2* w2;
     const float* w1;
     int m_lo;
+    __device__ double cut_sq(const Rec16Frame& R, int tt, int) const { return R.cut_sq_u[tt]; }
     template <int B>
-    __device__ void fetch(const int (&row)[B], const bool (&in)[B], float4 (&ca)[B], float4 (&cz)[B],
+    __device__ void fetch(const int (&row)[B], const int (&)[B], const bool (&in)[B], float4 (&ca)[B], float4 (&cz)[B],
                           float4 (&)[B]) const
     {
         bool low[B], any = false;
@@ -762,7 +784,7 @@ __global__ __launch_bounds__(kBlock) void k_eam_rho(int n, int lg, const int* __
         const uint4 ri = rec[i];
         const int ti = ONE ? 0 : (int)ri.w;
         const double rho = lane_sum(
-            rho_atom<B, ONE>(i, ri, nn[i], rec, list4, ldl, maxb, P, R, RhoRowsGlobal{P.tabA}, lg, g), lg);
+            rho_atom<B, ONE>(i, self_entry(i), ri, nn[i], rec, list4, ldl, maxb, P, R, RhoRowsGlobal{P.tabA}, lg, g), lg);
         if (g == 0) {
             double F, dF;
             embed(P, ti, rho, F, dF);
@@ -800,7 +822,7 @@ __global__ __launch_bounds__(kBlock) void k_eam_force(int n, int lg, const int* 
         const int ti = ONE ? 0 : (int)ri.w;
         const float dFi = ONE ? __uint_as_float(ri.w) : dF[i];
         float fx = 0.f, fy = 0.f, fz = 0.f;
-        force_atom<B, ONE, EV>(i, ri, ti, dFi, nn[i], rec, xr, dF, list4, ldl, maxb, P, R,
+        force_atom<B, ONE, EV>(i, self_entry(i), ri, ti, dFi, nn[i], rec, xr, dF, list4, ldl, maxb, P, R,
                                ForceRowsGlobal<ONE>{ONE ? P.tabC : P.tabB}, lg, g, fx, fy, fz, acc);
         fx = lane_sum(fx, lg);
         fy = lane_sum(fy, lg);
@@ -848,6 +870,33 @@ __device__ inline ChunkWalk chunk_walk(int n, int size)
     return w;
 }
 
+// The LDS passes' walk by waves: units of 64 / 2^lg atoms. A workgroup's 16
+// waves take neighboring units, and the units of the last round, too few for
+// every wave, go to the workgroups in turn, so that all CUs share them (by
+// whole workgroups a few CUs had a full round more than the others). q of nq:
+// this workgroup among those of its XCD that share the n atoms.
+constexpr int kBigWaves = kBigBlock / 64;
+struct UnitWalk {
+    int u0, cnt, full, last, q, nq, round;
+    __device__ UnitWalk(int n, int unit, int q_, int nq_) : q(q_), nq(nq_), round(0)
+    {
+        const int nunits = (n + unit - 1) / unit, per = (nunits + kXcd - 1) / kXcd, x = blockIdx.x % kXcd;
+        u0 = x * per;
+        cnt = max(0, min(per, nunits - u0));
+        full = cnt / (nq * kBigWaves);
+        last = cnt - full * nq * kBigWaves;
+    }
+    // the wave's next unit, or -1
+    __device__ int next()
+    {
+        const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+        const int r = round++;
+        if (r < full) return u0 + (r * nq + q) * kBigWaves + w;
+        if (r == full && w * nq + q < last) return u0 + full * nq * kBigWaves + w * nq + q;
+        return -1;
+    }
+};
+
 template <int B>
 __global__ __launch_bounds__(kBigBlock) void k_eam_rho_lds(int n, int lg, const int* __restrict__ stop,
                                                            const uint4* __restrict__ rec,
@@ -869,13 +918,14 @@ __global__ __launch_bounds__(kBigBlock) void k_eam_rho_lds(int n, int lg, const 
     __syncthreads();
     if (stop && *stop) return;
     const RhoRowsLds T{P.tabA, lds_rows, m_lo};
-    const int g = threadIdx.x & ((1 << lg) - 1), size = kBigBlock >> lg;
+    const int g = threadIdx.x & ((1 << lg) - 1), unit = 64 >> lg;
     double acc[1] = {0.0};
-    for (ChunkWalk w = chunk_walk(n, size); w.c < w.end; w.c += w.step) {
-        const int i = w.c * size + (threadIdx.x >> lg);
+    UnitWalk walk(n, unit, (int)blockIdx.x / kXcd, (int)gridDim.x / kXcd);
+    for (int u = walk.next(); u >= 0; u = walk.next()) {
+        const int i = u * unit + ((threadIdx.x & 63) >> lg);
         if (i >= n) continue;
         const uint4 ri = rec[i];
-        const double rho = lane_sum(rho_atom<B, true>(i, ri, nn[i], rec, list4, ldl, maxb, P, R, T, lg, g), lg);
+        const double rho = lane_sum(rho_atom<B, true>(i, self_entry(i), ri, nn[i], rec, list4, ldl, maxb, P, R, T, lg, g), lg);
         if (g != 0) continue;
         double F, dF;
         embed(P, 0, rho, F, dF);
@@ -921,16 +971,17 @@ __global__ __launch_bounds__(kBigBlock) void k_eam_force_lds(int n, int lg, cons
     __syncthreads();
     if (stop && *stop) return;
     const ForceRowsLds T{P.tabC, lds_rows, w2, w1, m_lo};
-    const int g = threadIdx.x & ((1 << lg) - 1), size = kBigBlock >> lg;
+    const int g = threadIdx.x & ((1 << lg) - 1), unit = 64 >> lg;
     double acc[7] = {0, 0, 0, 0, 0, 0, 0};
     double mvv[6] = {0, 0, 0, 0, 0, 0};
     double fm[3] = {0, 0, 0};
-    for (ChunkWalk cw = chunk_walk(n, size); cw.c < cw.end; cw.c += cw.step) {
-        const int i = cw.c * size + (threadIdx.x >> lg);
+    UnitWalk walk(n, unit, (int)blockIdx.x / kXcd, (int)gridDim.x / kXcd);
+    for (int u = walk.next(); u >= 0; u = walk.next()) {
+        const int i = u * unit + ((threadIdx.x & 63) >> lg);
         if (i >= n) continue;
         const uint4 ri = xr[i];
         float fx = 0.f, fy = 0.f, fz = 0.f;
-        force_atom<B, true, EV>(i, ri, 0, __uint_as_float(ri.w), nn[i], nullptr, xr, nullptr, list4, ldl, maxb, P,
+        force_atom<B, true, EV>(i, self_entry(i), ri, 0, __uint_as_float(ri.w), nn[i], nullptr, xr, nullptr, list4, ldl, maxb, P,
                                 R, T, lg, g, fx, fy, fz, acc);
         fx = lane_sum(fx, lg);
         fy = lane_sum(fy, lg);
@@ -950,6 +1001,234 @@ __global__ __launch_bounds__(kBigBlock) void k_eam_force_lds(int n, int lg, cons
         if (EV) __syncthreads();
         kick_rows<kBigBlock>(mvv, fm, part_mvv + (size_t)blockIdx.x * kPartW, part_cv + (size_t)blockIdx.x * kPartW);
     }
+}
+
+// Persistent passes for several elements. ne^2 element pairs' tables do not
+// fit in LDS, but the pairs of one central element a do, so a workgroup works
+// on the atoms of one element: it holds, for every neighbor element b,
+//  * density pass: the float4 rows of the density at a due to b (16 B a knot
+//    and element: all of 4,999 rows for two elements);
+//  * force pass: the knots of that function's derivative and of the density
+//    at b due to a, each 8 bytes, and of r*phi, 12 bytes: 48 B a knot for two
+//    elements with a function per ordered pair, 3,251 knots, r > 1.85 A of the
+//    5.3 A of a 5,000-knot Fe-Ni table. As float4 rows they would take 68 B
+//    and leave the first two neighbor shells of bcc iron to L2.
+// A knot holds the slope s per unit offset and e = (y1 - y0) - s of its
+// interval, rounded to FP32 from FP64; with g = s1 - s from the next knot the
+// interval's cubic has c1 = s, c2 = 3 e - g, c3 = g - 2 e. e and g are small
+// beside s, so the derivative carries the roundings of s and s1 only (a
+// difference of two rounded values y1 - y0 would carry theirs over the knot
+// spacing, 1e-4 eV/A). Rows below the window come from the global tables.
+// Workgroups are dealt to the elements of an XCD's share of the atoms in
+// proportion to their numbers.
+__device__ inline int share_elem(const ElemShare& S, int ne)
+{
+    const int q = (int)blockIdx.x / kXcd;
+    int a = 0;
+    while (a + 1 < ne && q >= S.wg0[a + 1]) ++a;
+    return a;
+}
+
+struct RhoAlloy {
+    static constexpr bool kRows = false;  // the neighbor's element is in the list entry
+    static constexpr uint32_t kMask = kAlloyMask;
+    const float4* tab;    // global rows of the central element, [ne][nr]
+    const float4* win;    // [ne][nwin]
+    const double* cut;    // [ne], LDS
+    int nr, nwin, m_lo;
+    __device__ double cut_sq(const Rec16Frame&, int, int ej) const { return cut[ej]; }
+    template <int B>
+    __device__ void fetch(const int (&m)[B], const int (&ej)[B], const bool (&in)[B], float4 (&c)[B]) const
+    {
+        bool low[B], any = false;
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+            const int r = m[b] - m_lo;
+            low[b] = in[b] && r < 0;
+            any |= low[b];
+            c[b] = win[ej[b] * nwin + (r < 0 ? 0 : r)];
+        }
+        if (__ballot(any) != 0ull) {
+#pragma unroll
+            for (int b = 0; b < B; ++b)
+                if (low[b]) c[b] = tab[(size_t)ej[b] * nr + m[b]];
+        }
+    }
+};
+
+struct ForceAlloy {
+    static constexpr bool kRows = false;  // the neighbor's element is in the list entry
+    static constexpr uint32_t kMask = kAlloyMask;
+    const float4* tab;  // global rows of the central element, [ne][nr][3]
+    const float2* d;    // [nd][nwin]: density derivatives, at the central atom by neighbor element, then at the neighbor
+    const float2* z;    // [ne][nwin]: r*phi
+    const float* y;     // [ne][nwin]: r*phi at the knots
+    const double* cut;
+    int ne, nd, nr, nwin, m_lo, elem;
+    __device__ double cut_sq(const Rec16Frame&, int, int ej) const { return cut[ej]; }
+    // derivative coefficients of the interval from its knots
+    __device__ static float4 slope(const float2* k, float w)
+    {
+        const float s = k[0].x, e = k[0].y, g = k[1].x - s;
+        return make_float4(s, 2.f * (3.f * e - g), 3.f * g - 6.f * e, w);
+    }
+    template <int B>
+    __device__ void fetch(const int (&m)[B], const int (&ej)[B], const bool (&in)[B], float4 (&ca)[B], float4 (&cz)[B],
+                          float4 (&cb)[B]) const
+    {
+        bool low[B], any = false;
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+            int r = m[b] - m_lo;
+            low[b] = in[b] && r < 0;
+            any |= low[b];
+            r = r < 0 ? 0 : r;
+            const int out = nd == ne || ej[b] == elem ? elem : ne + ej[b] - (ej[b] > elem ? 1 : 0);
+            ca[b] = slope(d + ej[b] * nwin + r, y[ej[b] * nwin + r]);
+            cb[b] = slope(d + out * nwin + r, 0.f);
+            const float2* k = z + ej[b] * nwin + r;
+            const float s = k[0].x, e = k[0].y, g = k[1].x - s;
+            cz[b] = make_float4(s, 3.f * e - g, g - 2.f * e, 0.f);
+        }
+        if (__ballot(any) != 0ull) {
+#pragma unroll
+            for (int b = 0; b < B; ++b)
+                if (low[b]) {
+                    const float4* c = tab + ((size_t)ej[b] * nr + m[b]) * 3;
+                    ca[b] = c[0];
+                    cz[b] = c[1];
+                    cb[b] = c[2];
+                }
+        }
+    }
+};
+
+template <int B>
+__global__ __launch_bounds__(kBigBlock) void k_eam_rho_alloy(ElemShare S, int lg, const int* __restrict__ stop,
+                                                             const int* __restrict__ eord,
+                                                             const uint4* __restrict__ rec, const int* __restrict__ nn,
+                                                             const uint4* __restrict__ list4, int ldl, int maxb,
+                                                             EamArgs P, Rec16Frame R, int m_lo, int nwin,
+                                                             double* __restrict__ rho_out, uint4* __restrict__ xr,
+                                                             double* __restrict__ part)
+{
+    extern __shared__ float4 lds_rows[];
+    __shared__ double cut[kMaxElems];
+    const int g = threadIdx.x & ((1 << lg) - 1), unit = 64 >> lg, elem = share_elem(S, P.ne);
+    const float4* tab = P.tabA + (size_t)elem * P.ne * P.nr;
+    for (int b = 0; b < P.ne; ++b)
+        for (int r0 = threadIdx.x; r0 < nwin; r0 += 5 * kBigBlock) {
+            float4 t[5];
+#pragma unroll
+            for (int q = 0; q < 5; ++q) t[q] = tab[(size_t)b * P.nr + m_lo + min(r0 + q * kBigBlock, nwin - 1)];
+#pragma unroll
+            for (int q = 0; q < 5; ++q)
+                if (r0 + q * kBigBlock < nwin) lds_rows[b * nwin + r0 + q * kBigBlock] = t[q];
+        }
+    if ((int)threadIdx.x < P.ne) cut[threadIdx.x] = R.cut_sq_u[elem * P.ne + threadIdx.x];
+    __syncthreads();
+    if (stop && *stop) return;
+    const RhoAlloy T{tab, lds_rows, cut, P.nr, nwin, m_lo};
+    double acc[1] = {0.0};
+    const int at0 = S.at0[elem], na = S.at0[elem + 1] - at0;
+    UnitWalk walk(na, unit, (int)blockIdx.x / kXcd - S.wg0[elem], S.wg0[elem + 1] - S.wg0[elem]);
+    for (int u = walk.next(); u >= 0; u = walk.next()) {
+        const int k = u * unit + ((threadIdx.x & 63) >> lg);
+        if (k >= na) continue;
+        const int i = eord[at0 + k];
+        const uint4 ri = rec[i];
+        const double rho =
+            lane_sum(rho_atom<B, false>(at0 + k, self_entry(i) | (uint32_t)elem << kElemShift, ri, nn[i], rec, list4, ldl, maxb, P, R, T, lg, g), lg);
+        if (g != 0) continue;
+        double F, dF;
+        embed(P, elem, rho, F, dF);
+        rho_out[i] = rho;
+        xr[i] = make_uint4(ri.x, ri.y, ri.z, __float_as_uint((float)dF));
+        acc[0] += F;
+    }
+    block_sum_store<1, kBigBlock>(acc, part + (size_t)blockIdx.x * kPartW);
+}
+
+template <int B, bool EV>
+__global__ __launch_bounds__(kBigBlock) void k_eam_force_alloy(ElemShare S, int lg, const int* __restrict__ stop,
+                                                               const int* __restrict__ eord,
+                                                               const uint4* __restrict__ xr, Rec16Frame R,
+                                                               const int* __restrict__ nn,
+                                                               const uint4* __restrict__ list4, int ldl, int maxb,
+                                                               EamArgs P, int m_lo, int nwin,
+                                                               float4* __restrict__ f_out, double* __restrict__ part,
+                                                               KickArgs K, double4* __restrict__ v,
+                                                               double* __restrict__ part_mvv,
+                                                               double* __restrict__ part_cv)
+{
+    extern __shared__ float4 lds_rows[];
+    __shared__ double cut[kMaxElems];
+    const int g = threadIdx.x & ((1 << lg) - 1), unit = 64 >> lg, elem = share_elem(S, P.ne);
+    const int npair = P.nd + P.ne;
+    float2* d = (float2*)lds_rows;
+    float* y = (float*)(d + (size_t)npair * nwin);
+    {
+        // the element's knots in memory: [nd + ne][nr] float2, then [ne][nr] float
+        const float* base = P.knots + (size_t)elem * P.knot_stride;
+        const float2* src = (const float2*)base;
+        for (int q = 0; q < npair; ++q)
+            for (int r0 = threadIdx.x; r0 < nwin; r0 += 4 * kBigBlock) {
+                float2 t[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) t[u] = src[(size_t)q * P.nr + m_lo + min(r0 + u * kBigBlock, nwin - 1)];
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (r0 + u * kBigBlock < nwin) d[q * nwin + r0 + u * kBigBlock] = t[u];
+            }
+        const float* ys = base + (size_t)2 * npair * P.nr;
+        for (int q = 0; q < P.ne; ++q)
+            for (int r = threadIdx.x; r < nwin; r += kBigBlock) y[q * nwin + r] = ys[(size_t)q * P.nr + m_lo + r];
+    }
+    if ((int)threadIdx.x < P.ne) cut[threadIdx.x] = R.cut_sq_u[elem * P.ne + threadIdx.x];
+    __syncthreads();
+    if (stop && *stop) return;
+    const ForceAlloy T{P.tabB + (size_t)elem * P.ne * P.nr * 3, d, d + P.nd * nwin, y, cut, P.ne, P.nd, P.nr, nwin, m_lo,
+                       elem};
+    double acc[7] = {0, 0, 0, 0, 0, 0, 0};
+    double mvv[6] = {0, 0, 0, 0, 0, 0};
+    double fm[3] = {0, 0, 0};
+    const int at0 = S.at0[elem], na = S.at0[elem + 1] - at0;
+    UnitWalk walk(na, unit, (int)blockIdx.x / kXcd - S.wg0[elem], S.wg0[elem + 1] - S.wg0[elem]);
+    for (int u = walk.next(); u >= 0; u = walk.next()) {
+        const int k = u * unit + ((threadIdx.x & 63) >> lg);
+        if (k >= na) continue;
+        const int i = eord[at0 + k];
+        const uint4 ri = xr[i];
+        float fx = 0.f, fy = 0.f, fz = 0.f;
+        force_atom<B, false, EV>(at0 + k, self_entry(i) | (uint32_t)elem << kElemShift, ri, elem,
+                                 __uint_as_float(ri.w), nn[i], nullptr, xr, nullptr, list4, ldl, maxb, P, R, T, lg, g, fx,
+                                 fy, fz, acc);
+        fx = lane_sum(fx, lg);
+        fy = lane_sum(fy, lg);
+        fz = lane_sum(fz, lg);
+        if (g != 0) continue;
+        f_out[i] = make_float4(fx, fy, fz, 0.f);
+        if (K.on) kick_atom(i, elem, fx, fy, fz, K, v, mvv, fm);
+    }
+    if (EV) {
+        acc[0] *= 0.5;
+        for (int k = 1; k < 7; ++k) acc[k] *= 0.5 * R.q;
+        block_sum_store<7, kBigBlock>(acc, part + (size_t)blockIdx.x * kPartW);
+    }
+    if (K.on) {
+        if (EV) __syncthreads();
+        kick_rows<kBigBlock>(mvv, fm, part_mvv + (size_t)blockIdx.x * kPartW, part_cv + (size_t)blockIdx.x * kPartW);
+    }
+}
+
+// sort keys of the element order
+__global__ __launch_bounds__(kBlock) void k_elem_keys(int n, const uint4* __restrict__ rec, uint32_t* __restrict__ key,
+                                                      int* __restrict__ val)
+{
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= n) return;
+    key[i] = rec[i].w;
+    val[i] = i;
 }
 
 // ---------------- NVT ----------------
@@ -995,7 +1274,7 @@ __global__ __launch_bounds__(kBlock) void k_shift_decide(int n, double4* __restr
 // new v go to part_sv.
 // At most kStepRows workgroups walk the atoms, so that one workgroup can sum
 // their rows (k_nvt_end).
-constexpr int kStepRows = 2048;
+constexpr int kStepRows = 1024;
 __global__ __launch_bounds__(kBlock) void k_step(int n, double4* __restrict__ x, double4* __restrict__ v,
                                                  const float4* __restrict__ f, NvtArgs A,
                                                  const double* __restrict__ nh, const double4* __restrict__ x0,
@@ -1171,6 +1450,7 @@ __global__ __launch_bounds__(kEndThreads) void k_nvt_end(double* __restrict__ nh
     const int nr = col < 3 ? nsv : nf;
     const int rebuild = flags[FL_REBUILD];
     double s[1] = {0.0};
+#pragma unroll 8
     for (int r = lane; r < nr; r += 64) s[0] += rows[(size_t)r * kPartW];
     wave_sums<1>(s);
     if (lane == 0) sum[col] = s[0];
@@ -1303,6 +1583,55 @@ EamForceField::EamForceField(EamTables t) : t_(std::move(t))
     MAPP_HIP(hipMemcpy(tabA_.get(), A.data(), A.size() * sizeof(float4), hipMemcpyHostToDevice));
     MAPP_HIP(hipMemcpy(tabB_.get(), B.data(), B.size() * sizeof(float4), hipMemcpyHostToDevice));
     MAPP_HIP(hipMemcpy(Ftab_.get(), F.data(), F.size() * sizeof(double), hipMemcpyHostToDevice));
+    knot_tables();
+}
+
+// The knots of the alloy passes: for each central element a, (slope, e) of the
+// derivatives (1/dr applied) of the density at a due to b, b = 0..ne-1, and,
+// where the density at b due to a depends on b, of those for b != a; of r*phi;
+// then r*phi itself. Left out where a spline is not the Hermite cubic of its
+// knots.
+void EamForceField::knot_tables()
+{
+    const int ne = t_.ne, nr = t_.nr;
+    if (ne < 2) return;
+    const size_t row = (size_t)nr * 4;
+    bool fs = false;  // one density function per ordered pair
+    for (int a = 0; a < ne; ++a)
+        for (int b = 1; b < ne; ++b) fs = fs || !std::equal(t_.rho_at(a, b), t_.rho_at(a, b) + row, t_.rho_at(a, 0));
+    const int nd = fs ? 2 * ne - 1 : ne;
+    const size_t per = ((size_t)(2 * (nd + ne) + ne) * nr + 3) & ~(size_t)3;  // every element's part 16-byte aligned
+    std::vector<float> out(per * ne);
+    std::vector<double> ys;
+    for (int a = 0; a < ne; ++a) {
+        float* base = out.data() + per * a;
+        int q = 0;
+        const auto put = [&](const double* c, double scale) {
+            if (!hermite_knots(c, nr, ys)) return false;
+            for (int m = 0; m < nr; ++m) {
+                const double s = ys[2 * (size_t)m + 1];
+                const double e = m + 1 < nr ? (ys[2 * (size_t)m + 2] - ys[2 * (size_t)m]) - s : 0.0;
+                base[2 * ((size_t)q * nr + m)] = (float)(s * scale);
+                base[2 * ((size_t)q * nr + m) + 1] = (float)(e * scale);
+            }
+            ++q;
+            return true;
+        };
+        const double dri = 1.0 / t_.dr;
+        bool ok = true;
+        for (int b = 0; b < ne; ++b) ok = ok && put(t_.rho_at(b, a), dri);
+        if (fs)
+            for (int b = 0; b < ne; ++b) ok = ok && (b == a || put(t_.rho_at(a, b), dri));
+        for (int b = 0; b < ne; ++b) ok = ok && put(t_.rphi_at(a, b), 1.0);
+        if (!ok) return;
+        for (int b = 0; b < ne; ++b)
+            for (int m = 0; m < nr; ++m)
+                base[(size_t)2 * (nd + ne) * nr + (size_t)b * nr + m] = (float)t_.rphi_at(a, b)[4 * (size_t)m];
+    }
+    knots_.reserve(out.size());
+    MAPP_HIP(hipMemcpy(knots_.get(), out.data(), out.size() * sizeof(float), hipMemcpyHostToDevice));
+    nd_ = nd;
+    knot_stride_ = per;
 }
 
 EamArgs EamForceField::args() const
@@ -1320,6 +1649,9 @@ EamArgs EamForceField::args() const
     P.tabB = tabB_.get();
     P.tabC = tabC_.get();
     P.Ftab = Ftab_.get();
+    P.knots = nd_ ? knots_.get() : nullptr;
+    P.nd = nd_;
+    P.knot_stride = knot_stride_;
     return P;
 }
 
@@ -1364,6 +1696,7 @@ MDSystem::MDSystem(std::shared_ptr<EamForceField> ff, int natms, const double* H
     MAPP_HIP(hipMemsetAsync(v_.get(), 0, sizeof(double4) * n_, stream_));
     MAPP_HIP(hipMemsetAsync(f_.get(), 0, sizeof(float4) * n_, stream_));
     plan_lds();
+    plan_alloy();
     rebuild();
 }
 
@@ -1486,6 +1819,77 @@ void MDSystem::plan_lds()
         }
     }
     lds_ok_ = use_lds_ = true;
+}
+
+void MDSystem::plan_alloy()
+{
+    alloy_ok_ = false;
+    const EamArgs P = ff_->args();
+    if (!P.knots || P.nr < 2 || P.ne > kAlloyElems) return;
+    int dev = 0, lds_max = 0, ncu = 0;
+    MAPP_HIP(hipGetDevice(&dev));
+    MAPP_HIP(hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
+    MAPP_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+    const long budget = (long)lds_max - 4096;
+    lds_grid_ = std::max(1, ncu / kXcd) * kXcd;
+    if (budget < 16384 || lds_grid_ / kXcd < P.ne) return;  // a workgroup per element on every XCD
+    const int rows = P.nr - 1;  // spline intervals 0 .. nr-2
+    al_rho_nwin_ = (int)std::min<long>(rows, budget / (16L * P.ne));
+    al_rho_lo_ = rows - al_rho_nwin_;
+    al_rho_lds_ = (size_t)al_rho_nwin_ * 16 * P.ne;
+    const long knot = 8L * (P.nd + P.ne) + 4L * P.ne;
+    al_f_nwin_ = (int)std::min<long>(P.nr, budget / knot);  // knots m_lo .. nr-1
+    al_f_lo_ = P.nr - al_f_nwin_;
+    al_f_lds_ = (size_t)al_f_nwin_ * knot;
+    if (al_rho_nwin_ < 1 || al_f_nwin_ < 2) return;
+    const std::pair<const void*, size_t> fns[] = {{(const void*)k_eam_rho_alloy<4>, al_rho_lds_},
+                                                  {(const void*)k_eam_force_alloy<2, true>, al_f_lds_},
+                                                  {(const void*)k_eam_force_alloy<2, false>, al_f_lds_}};
+    for (const auto& f : fns)
+        if (hipFuncSetAttribute(f.first, hipFuncAttributeMaxDynamicSharedMemorySize, (int)f.second) != hipSuccess) {
+            (void)hipGetLastError();
+            return;
+        }
+    alloy_ok_ = true;
+}
+
+// the slots in element order, and each element's share of an XCD's workgroups
+// (in proportion to its atoms, one at least)
+void MDSystem::element_order()
+{
+    const int ne = ff_->tables().ne;
+    std::vector<int> cnt(ne, 0);
+    for (int i = 0; i < n_; ++i) ++cnt[elem_host_[i]];
+    const int W = lds_grid_ / kXcd;
+    std::vector<int> w(ne, 1);
+    for (int left = W - ne; left > 0; --left) {
+        int a = 0;
+        for (int b = 1; b < ne; ++b)
+            if ((double)cnt[b] / w[b] > (double)cnt[a] / w[a]) a = b;
+        ++w[a];
+    }
+    share_ = ElemShare{};
+    for (int a = 0; a < ne; ++a) {
+        share_.wg0[a + 1] = share_.wg0[a] + w[a];
+        share_.at0[a + 1] = share_.at0[a] + cnt[a];
+    }
+    eord_.reserve(n_);
+    eval_.reserve(n_);
+    ekey_.reserve(n_);
+    ekey_alt_.reserve(n_);
+    hipLaunchKernelGGL(k_elem_keys, dim3((n_ + kBlock - 1) / kBlock), dim3(kBlock), 0, stream_, n_, rec_.get(),
+                       ekey_.get(), eval_.get());
+    int bits = 1;
+    while ((1 << bits) < ne) ++bits;
+    size_t bytes = 0;
+    MAPP_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, bytes, ekey_.get(), ekey_alt_.get(), eval_.get(), eord_.get(),
+                                                n_, 0, bits, stream_));
+    if (bytes > sort_tmp_bytes_) {
+        sort_tmp_.reserve(bytes);
+        sort_tmp_bytes_ = bytes;
+    }
+    MAPP_HIP(hipcub::DeviceRadixSort::SortPairs(sort_tmp_.get(), bytes, ekey_.get(), ekey_alt_.get(), eval_.get(),
+                                                eord_.get(), n_, 0, bits, stream_));
 }
 
 bool MDSystem::set_lds(bool on)
@@ -1617,6 +2021,8 @@ void MDSystem::rebuild()
     std::swap(id_.p, id_alt_.p);
     hipLaunchKernelGGL(k_cell_start, dim3((grid_.ncells + 1 + kBlock - 1) / kBlock), dim3(kBlock), 0, stream_, n_,
                        grid_.ncells, keys_alt_.get(), cell_start_.get());
+    alloy_list_ = alloy_ok_ && n_ >= kAlloyMinAtoms && (uint32_t)n_ <= kAlloyMask;
+    if (alloy_list_) element_order();
     prof_.end(stream_);
     build_list();
     ++nrebuild_;
@@ -1657,18 +2063,18 @@ void MDSystem::build_list()
 #define MAPP_BUILD(ONE) hipLaunchKernelGGL(k_build_list_group<ONE>, dim3(ng), dim3(kBlock), 0, stream_, n_, lg, \
                                            s_.get(), rec_.get(), r16_, bd, g, cell_rank_.get(), cell_start_.get(), \
                                            ordered_ ? cell_order_.get() : nullptr, maxn_ / 4, ldl_, list_.get(), \
-                                           nn_.get(), flags_.get())
+                                           nn_.get(), flags_.get(), alloy_list_ ? eord_.get() : nullptr)
             if (t.ne == 1) MAPP_BUILD(true); else MAPP_BUILD(false);
 #undef MAPP_BUILD
         } else if (t.ne == 1)
             hipLaunchKernelGGL(k_build_list<true>, dim3(nb), dim3(kBlock), 0, stream_, n_, s_.get(), rec_.get(), r16_,
                                bd, g, cell_rank_.get(), cell_start_.get(), ordered_ ? cell_order_.get() : nullptr,
-                               maxn_ / 4, ldl_, list4(), nn_.get(), flags_.get());
+                               maxn_ / 4, ldl_, list4(), nn_.get(), flags_.get(), (const int*)nullptr);
         else
             hipLaunchKernelGGL(k_build_list<false>, dim3(nb), dim3(kBlock), 0, stream_, n_, s_.get(), rec_.get(),
                                r16_, bd, g, cell_rank_.get(), cell_start_.get(),
                                ordered_ ? cell_order_.get() : nullptr, maxn_ / 4, ldl_, list4(), nn_.get(),
-                               flags_.get());
+                               flags_.get(), alloy_list_ ? eord_.get() : nullptr);
         prof_.end(stream_);
         int over = 0;
         MAPP_HIP(hipMemcpyAsync(&over, flags_.get(), sizeof(int), hipMemcpyDeviceToHost, stream_));
@@ -1679,20 +2085,48 @@ void MDSystem::build_list()
     throw Error(ERR_STATE, "neighbor list capacity did not converge");
 }
 
-// log2 of the lanes that share an atom: the fewest rounds of 4-entry batches.
-// A workgroup of the LDS passes works on 1024 / 2^lg atoms at a time, and the
-// CUs on as many chunks side by side; a round costs its lane's batches and,
-// for the atom's own loads, embedding and sums, about two more (three once
-// lanes have to meet).
+// Cost of a pass over `units` wave-units on `waves` waves: whole rounds, and a
+// last one that is shared by all CUs (about half a round's time at worst) in
+// 4-entry batches; a unit costs its lane's batches and, for the atom's own
+// loads, embedding and sums, about two more (three once lanes have to meet).
+// Lanes at different ranks of a row gather from more places, so a split pays
+// only where waves would stand idle.
+static double pass_cost(long units, long waves, int batches, int lg)
+{
+    const double left = (double)(units % waves) / waves;
+    const double rounds = (double)(units / waves) + (left > 0.0 ? 0.5 + 0.5 * left : 0.0);
+    return rounds * (((batches - 1) >> lg) + (lg ? 4 : 3));
+}
+
+// log2 of the lanes that share an atom in the LDS passes
 int MDSystem::lanes_lds() const
 {
     const int batches = (int)((maxn_ - 16) / 1.25 / 4.0) + 1;  // the expected row, see setup_grid
     int best = 0;
-    long least = 0;
+    double least = 0.0;
     for (int lg = 0; lg <= 4; ++lg) {
-        const int size = kBigBlock >> lg;
-        const long chunks = (n_ + size - 1) / size;
-        const long cost = ((chunks + lds_grid_ - 1) / lds_grid_) * (((batches - 1) >> lg) + (lg ? 4 : 3));
+        const int unit = 64 >> lg;
+        const double cost = pass_cost((n_ + unit - 1) / unit, (long)lds_grid_ * kBigWaves, batches, lg);
+        if (lg == 0 || cost < least) {
+            least = cost;
+            best = lg;
+        }
+    }
+    return best;
+}
+
+// the same for the element order: the slowest element decides
+int MDSystem::lanes_alloy() const
+{
+    const int ne = ff_->tables().ne, batches = (int)((maxn_ - 16) / 1.25 / 4.0) + 1;
+    int best = 0;
+    double least = 0.0;
+    for (int lg = 0; lg <= 4; ++lg) {
+        const int unit = 64 >> lg;
+        double cost = 0.0;
+        for (int a = 0; a < ne; ++a)
+            cost = std::max(cost, pass_cost((share_.at0[a + 1] - share_.at0[a] + unit - 1) / unit,
+                                            (long)(share_.wg0[a + 1] - share_.wg0[a]) * kXcd * kBigWaves, batches, lg));
         if (lg == 0 || cost < least) {
             least = cost;
             best = lg;
@@ -1732,9 +2166,9 @@ void MDSystem::force_passes(const KickArgs* kick, bool records_fresh, float4* f_
     const int maxb = maxn_ / 4;
     if (lds) {
         const int lg = lanes_lds();
-        const int chunks = (n_ + (kBigBlock >> lg) - 1) / (kBigBlock >> lg);
-        // at most one workgroup per CU, and one per chunk (rounded up to the 8 XCDs)
-        const int G = std::min(lds_grid_, (chunks + kXcd - 1) / kXcd * kXcd);
+        const int units = (n_ + (64 >> lg) - 1) / (64 >> lg);
+        // at most one workgroup per CU, and no more than there are units (rounded up to the 8 XCDs)
+        const int G = std::min(lds_grid_, (units + kXcd - 1) / kXcd * kXcd);
         const int br = lg && batch_rho_ > 4 ? 4 : batch_rho_;
 #define MAPP_RHO(B) hipLaunchKernelGGL((k_eam_rho_lds<B>), dim3(G), dim3(kBigBlock), rho_lds_bytes_, stream_, n_, lg, \
                                        stop, rec_.get(), nn_.get(), list4(), ldl_, maxb, P, r16_, rho_m_lo_, \
@@ -1761,6 +2195,24 @@ void MDSystem::force_passes(const KickArgs* kick, bool records_fresh, float4* f_
         } else {
             if (ev) MAPP_FORCE(2, true); else MAPP_FORCE(2, false);
         }
+#undef MAPP_FORCE
+        prof_.end(stream_);
+        pass_rows_ = G;
+        if (ev) reduce_rows(part_.get(), 2 * G, 7, red_.get());
+        return;
+    }
+    if (alloy_list_) {
+        const int lg = lanes_alloy(), G = lds_grid_;
+        hipLaunchKernelGGL(k_eam_rho_alloy<4>, dim3(G), dim3(kBigBlock), al_rho_lds_, stream_, share_, lg, stop,
+                           eord_.get(), rec_.get(), nn_.get(), list4(), ldl_, maxb, P, r16_, al_rho_lo_, al_rho_nwin_,
+                           ro, xr_.get(), part_.get());
+        prof_.end(stream_);
+        prof_.begin(K_EAM_FORCE, stream_);
+        double* p2 = part_.get() + (size_t)G * kPartW;
+#define MAPP_FORCE(EV) hipLaunchKernelGGL((k_eam_force_alloy<2, EV>), dim3(G), dim3(kBigBlock), al_f_lds_, stream_, \
+                                          share_, lg, stop, eord_.get(), xr_.get(), r16_, nn_.get(), \
+                                          list4(), ldl_, maxb, P, al_f_lo_, al_f_nwin_, fo, p2, K, v_.get(), p3, p4)
+        if (ev) MAPP_FORCE(true); else MAPP_FORCE(false);
 #undef MAPP_FORCE
         prof_.end(stream_);
         pass_rows_ = G;
@@ -1991,10 +2443,14 @@ void MDSystem::list_stats(int* maxn, int64_t* nfull)
 
 namespace {
 struct HostList {
-    std::vector<int> nn, id;
+    std::vector<int> nn, id, eord;
     std::vector<uint32_t> list;
+    uint32_t mask = kIndexMask;
+    int slot(int col) const { return eord.empty() ? col : eord[col]; }
 };
-HostList fetch_list(const int* nn_d, const int* id_d, const uint32_t* list_d, int n, int maxn, int ldl, hipStream_t st)
+// eord_d: the column order of the alloy passes' list, or null
+HostList fetch_list(const int* nn_d, const int* id_d, const uint32_t* list_d, int n, int maxn, int ldl, hipStream_t st,
+                    const int* eord_d)
 {
     HostList h;
     h.nn.resize(n);
@@ -2003,6 +2459,11 @@ HostList fetch_list(const int* nn_d, const int* id_d, const uint32_t* list_d, in
     MAPP_HIP(hipMemcpyAsync(h.nn.data(), nn_d, sizeof(int) * n, hipMemcpyDeviceToHost, st));
     MAPP_HIP(hipMemcpyAsync(h.id.data(), id_d, sizeof(int) * n, hipMemcpyDeviceToHost, st));
     MAPP_HIP(hipMemcpyAsync(h.list.data(), list_d, sizeof(uint32_t) * h.list.size(), hipMemcpyDeviceToHost, st));
+    if (eord_d) {
+        h.eord.resize(n);
+        MAPP_HIP(hipMemcpyAsync(h.eord.data(), eord_d, sizeof(int) * n, hipMemcpyDeviceToHost, st));
+        h.mask = kAlloyMask;
+    }
     MAPP_HIP(hipStreamSynchronize(st));
     return h;
 }
@@ -2019,26 +2480,26 @@ inline void decode_img(uint32_t code, int8_t* img)
 // id_i < id_j.
 int64_t MDSystem::half_pairs_count()
 {
-    HostList h = fetch_list(nn_.get(), id_.get(), list_.get(), n_, maxn_, ldl_, stream_);
+    HostList h = fetch_list(nn_.get(), id_.get(), list_.get(), n_, maxn_, ldl_, stream_, alloy_list_ ? eord_.get() : nullptr);
     int64_t c = 0;
-    for (int s = 0; s < n_; ++s)
-        for (int k = 0; k < h.nn[s]; ++k) {
-            const uint32_t e = h.list[((size_t)(k >> 2) * ldl_ + s) * 4 + (k & 3)];
+    for (int col = 0; col < n_; ++col)
+        for (int s = h.slot(col), k = 0; k < h.nn[s]; ++k) {
+            const uint32_t e = h.list[((size_t)(k >> 2) * ldl_ + col) * 4 + (k & 3)];
             const uint32_t code = e >> kIndexBits;
-            if (code != (uint32_t)kZeroImage || h.id[s] < h.id[e & kIndexMask]) ++c;
+            if (code != (uint32_t)kZeroImage || h.id[s] < h.id[e & h.mask]) ++c;
         }
     return c;
 }
 
 void MDSystem::half_pairs(int32_t* pi, int32_t* pj, int8_t* img)
 {
-    HostList h = fetch_list(nn_.get(), id_.get(), list_.get(), n_, maxn_, ldl_, stream_);
+    HostList h = fetch_list(nn_.get(), id_.get(), list_.get(), n_, maxn_, ldl_, stream_, alloy_list_ ? eord_.get() : nullptr);
     int64_t c = 0;
-    for (int s = 0; s < n_; ++s)
-        for (int k = 0; k < h.nn[s]; ++k) {
-            const uint32_t e = h.list[((size_t)(k >> 2) * ldl_ + s) * 4 + (k & 3)];
+    for (int col = 0; col < n_; ++col)
+        for (int s = h.slot(col), k = 0; k < h.nn[s]; ++k) {
+            const uint32_t e = h.list[((size_t)(k >> 2) * ldl_ + col) * 4 + (k & 3)];
             const uint32_t code = e >> kIndexBits;
-            const int j = h.id[e & kIndexMask];
+            const int j = h.id[e & h.mask];
             if (code != (uint32_t)kZeroImage || h.id[s] < j) {
                 pi[c] = h.id[s];
                 pj[c] = j;

@@ -18,7 +18,11 @@ constexpr uint32_t kIndexMask = (1u << kIndexBits) - 1u;  // image code in the h
 // (an NVT step at 8,788 atoms 36.8 us with LDS, 34.9 without; at 32,000 44.0
 // and 51.7)
 constexpr int kLdsMinAtoms = 12288;
+constexpr int kAlloyMinAtoms = 49152;           // the same for several elements
 constexpr int kMinPartRows = 4096;              // see MDSystem::part_rows
+// the alloy passes' list holds the neighbor's element above a shorter index
+constexpr int kElemShift = 23, kAlloyElems = 4;
+constexpr uint32_t kAlloyMask = (1u << kElemShift) - 1u;
 constexpr int kZeroImage = 62;                  // code of the (0,0,0) shift
 
 // Kernel argument block describing the EAM tables on the device.
@@ -31,6 +35,19 @@ struct EamArgs {
     const float4* tabB;   // [ne*ne][nr][3]: (rho'[tj][ti] d1..d3, r*phi c0), (r*phi c1..c3, 0), (rho'[ti][tj] d1..d3, 0)
     const float4* tabC;   // one element only: [nr][2] = (rho' d1..d3, r*phi c0), (r*phi c1..c3, 0)
     const double* Ftab;   // [ne][nrho][4]
+    // several elements whose splines are Hermite cubics of their knots
+    // (nullptr otherwise): for each central element the knots of its pairs'
+    // functions, see AlloyWindow
+    const float* knots;
+    size_t knot_stride;   // floats of one central element
+    int nd;               // density functions of a central element: ne, or 2 ne - 1 with one per ordered pair
+};
+
+// Workgroups of each XCD that work for each central element, and the atoms of
+// each element (element order: slots sorted by element, each in slot order).
+struct ElemShare {
+    int wg0[kMaxElems + 1];
+    int at0[kMaxElems + 1];
 };
 
 // ForceFieldEAM with its tables uploaded once (pair splines in FP32, the
@@ -41,8 +58,12 @@ public:
     const EamTables& tables() const { return t_; }
     EamArgs args() const;
 private:
+    void knot_tables();
     EamTables t_;
     DevBuf<float4> tabA_, tabB_, tabC_;
+    DevBuf<float> knots_;
+    int nd_ = 0;
+    size_t knot_stride_ = 0;
     DevBuf<double> Ftab_;
 };
 
@@ -277,6 +298,18 @@ private:
     // the minimiser's vectors follow their atoms into a rebuilt slot order
     void min_follow(int nvec, DevBuf<double4>** vecs, int nshift);
     void plan_lds();
+    // the same for several elements: windows per central element, and the
+    // atoms in element order
+    bool alloy_ok_ = false;
+    bool alloy_list_ = false;        // the current list is the alloy passes'
+    int al_rho_lo_ = 0, al_rho_nwin_ = 0, al_f_lo_ = 0, al_f_nwin_ = 0;
+    size_t al_rho_lds_ = 0, al_f_lds_ = 0;
+    DevBuf<int> eord_, eval_;        // slots in element order, and the sort's input
+    DevBuf<uint32_t> ekey_, ekey_alt_;
+    ElemShare share_{};
+    void plan_alloy();
+    void element_order();
+    int lanes_alloy() const;
 };
 
 }  // namespace mapp
