@@ -1419,13 +1419,13 @@ __device__ inline void nhc_update(double* __restrict__ nh, const double* mvv, co
             nh[NH_COM + k] = (nh[NH_FAC] * nh[NH_SV + k] + A.dt2 * nh[NH_SF + k]) * A.dt / A.natms;
 }
 
-// the start of a run: modes 0 and 1
+// the start of a run: mode 0 and, where there are steps, mode 1
 __global__ void k_nhc(double* __restrict__ nh, const double* __restrict__ mvv, const double* __restrict__ cv,
-                      NvtArgs A)
+                      NvtArgs A, int steps)
 {
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
     nhc_update(nh, mvv, cv, A, 0);
-    nhc_update(nh, mvv, cv, A, 1);
+    if (steps > 0) nhc_update(nh, mvv, cv, A, 1);
 }
 
 // The end of an NVT step on one workgroup: the sums of the new velocities
@@ -2546,7 +2546,7 @@ int MDSystem::nvt_run(const double* masses, double kB, double T, double dt, int 
         reduce_rows(region(2), nb, 6, mvv);
         reduce_rows(region(3), nb, 6, cv);
     }
-    hipLaunchKernelGGL(k_nhc, dim3(1), dim3(64), 0, stream_, nh, mvv, cv, A);
+    hipLaunchKernelGGL(k_nhc, dim3(1), dim3(64), 0, stream_, nh, mvv, cv, A, nsteps);
     const double skin_sq4 = 0.25 * skin_ * skin_;
     KickArgs kick{};
     kick.dt2 = A.dt2;

@@ -197,6 +197,24 @@ def test_nvt_matches_oracle_short_run(M, cu_pot):
     assert abs(out[0] - outo[0]) < E_ATOM * len(x)
 
 
+def test_nvt_of_no_steps_changes_nothing(M, cu_pot):
+    # no step: no half of the thermostat either. T_part is the temperature of
+    # the velocities as they are (sums of 864 FP64 products: below 1e-13 relative)
+    x, H = pot.fcc(3.615, (6, 6, 6))
+    elem = np.zeros(len(x), np.uint8)
+    masses = [pot.MASS["Cu"]]
+    v = O.o_create_T(elem, masses, pot.KB_EV, 300.0, 3)
+    g = M.AtomsMD(M.ForceFieldEAM.from_knots(cu_pot), H, jitter(x, 0.05, 11), elem, skin=0.5)
+    x0 = g.x
+    g.x_d = v
+    nvt = M.NVT(900.0, 1.0 * pot.FS)
+    out = nvt.run(g, 0, masses)
+    T = masses[0] * (v * v).sum() / (3 * len(x) * pot.KB_EV)
+    assert np.array_equal(g.x_d, v) and np.array_equal(g.x, x0)
+    assert nvt.rebuilds == 0 and abs(nvt.T_part - T) < 1e-13 * T
+    assert out[0] == g.force_calc()[1]
+
+
 def test_box_change_gives_the_oracle_of_the_new_box(M, cu_pot):
     # what md_nst or a strain step does to atoms->H (src/atoms.cpp:187-194):
     # the handle takes the new box and positions, and its forces, energy and
