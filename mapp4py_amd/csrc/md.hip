@@ -1844,7 +1844,7 @@ void MDSystem::plan_alloy()
     if (al_rho_nwin_ < 1 || al_f_nwin_ < 2) return;
     const std::pair<const void*, size_t> fns[] = {{(const void*)k_eam_rho_alloy<4>, al_rho_lds_},
                                                   {(const void*)k_eam_force_alloy<2, true>, al_f_lds_},
-                                                  {(const void*)k_eam_force_alloy<2, false>, al_f_lds_}};
+                                                  {(const void*)k_eam_force_alloy<4, false>, al_f_lds_}};
     for (const auto& f : fns)
         if (hipFuncSetAttribute(f.first, hipFuncAttributeMaxDynamicSharedMemorySize, (int)f.second) != hipSuccess) {
             (void)hipGetLastError();
@@ -2209,9 +2209,10 @@ void MDSystem::force_passes(const KickArgs* kick, bool records_fresh, float4* f_
         prof_.end(stream_);
         prof_.begin(K_EAM_FORCE, stream_);
         double* p2 = part_.get() + (size_t)G * kPartW;
-#define MAPP_FORCE(EV) hipLaunchKernelGGL((k_eam_force_alloy<2, EV>), dim3(G), dim3(kBigBlock), al_f_lds_, stream_, \
-                                          share_, lg, stop, eord_.get(), xr_.get(), r16_, nn_.get(), \
-                                          list4(), ldl_, maxb, P, al_f_lo_, al_f_nwin_, fo, p2, K, v_.get(), p3, p4)
+#define MAPP_FORCE(EV) hipLaunchKernelGGL((k_eam_force_alloy<(EV ? 2 : 4), EV>), dim3(G), dim3(kBigBlock), \
+                                          al_f_lds_, stream_, share_, lg, stop, eord_.get(), xr_.get(), r16_, \
+                                          nn_.get(), list4(), ldl_, maxb, P, al_f_lo_, al_f_nwin_, fo, p2, K, \
+                                          v_.get(), p3, p4)
         if (ev) MAPP_FORCE(true); else MAPP_FORCE(false);
 #undef MAPP_FORCE
         prof_.end(stream_);
