@@ -21,7 +21,7 @@ struct Box {
 };
 
 // lower-triangular inverse, depth and volume (src/xmath.h:1403-1485, 2399-2415)
-inline Box make_box(const double* Hin)
+__host__ __device__ inline Box make_box(const double* Hin)
 {
 #pragma clang fp contract(off)
     Box bx{};

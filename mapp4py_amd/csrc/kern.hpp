@@ -23,6 +23,25 @@ __device__ inline int xcd_block()
     return (blockIdx.x % kXcd) * q + blockIdx.x / kXcd;
 }
 
+// The walk of persistent workgroups (see the LDS passes of the EAM force
+// field): an XCD's workgroups stride side by side through a contiguous eighth
+// of the chunks.
+struct ChunkWalk {
+    int c, end, step;
+};
+// chunks of `size` atoms
+__device__ inline ChunkWalk chunk_walk(int n, int size)
+{
+    const int nchunks = (n + size - 1) / size;
+    const int per = (nchunks + kXcd - 1) / kXcd;
+    const int x = blockIdx.x % kXcd;
+    ChunkWalk w;
+    w.c = x * per + (int)blockIdx.x / kXcd;
+    w.end = min((x + 1) * per, nchunks);
+    w.step = gridDim.x / kXcd;
+    return w;
+}
+
 // P sums (a power of two) over the 64 lanes of a wave, in a fixed order: lanes
 // a bit apart each keep half of the values and give the other half away, until
 // one is left, so 8 values take 4 + 2 + 1 + 3 exchanges instead of 48. Lane l

@@ -39,9 +39,6 @@ struct GridArgs {
     // every pair the record quantisation could misplace)
     double rec_in_sq[kMaxElems * kMaxElems], rec_out_sq[kMaxElems * kMaxElems];
 };
-// flags: the largest row of a list build that overflowed, an atom moved half
-// the skin, a run's steps are halted there, steps a run has finished
-enum { FL_OVER = 0, FL_REBUILD = 1, FL_HALT = 2, FL_DONE = 3 };
 
 // ---------------- neighbor build ----------------
 
@@ -854,22 +851,6 @@ __global__ __launch_bounds__(kBlock) void k_eam_force(int n, int lg, const int* 
 // contiguous run per workgroup measured 15-25% more HBM fetch).
 constexpr int kBigBlock = 1024;
 
-struct ChunkWalk {
-    int c, end, step;
-};
-// chunks of `size` atoms
-__device__ inline ChunkWalk chunk_walk(int n, int size)
-{
-    const int nchunks = (n + size - 1) / size;
-    const int per = (nchunks + kXcd - 1) / kXcd;
-    const int x = blockIdx.x % kXcd;
-    ChunkWalk w;
-    w.c = x * per + (int)blockIdx.x / kXcd;
-    w.end = min((x + 1) * per, nchunks);
-    w.step = gridDim.x / kXcd;
-    return w;
-}
-
 // The LDS passes' walk by waves: units of 64 / 2^lg atoms. A workgroup's 16
 // waves take neighboring units, and the units of the last round, too few for
 // every wave, go to the workgroups in turn, so that all CUs share them (by
@@ -1274,7 +1255,6 @@ __global__ __launch_bounds__(kBlock) void k_shift_decide(int n, double4* __restr
 // new v go to part_sv.
 // At most kStepRows workgroups walk the atoms, so that one workgroup can sum
 // their rows (k_nvt_end).
-constexpr int kStepRows = 1024;
 __global__ __launch_bounds__(kBlock) void k_step(int n, double4* __restrict__ x, double4* __restrict__ v,
                                                  const float4* __restrict__ f, NvtArgs A,
                                                  const double* __restrict__ nh, const double4* __restrict__ x0,
@@ -2145,7 +2125,7 @@ int MDSystem::lanes_global() const
 }
 
 void MDSystem::force_passes(const KickArgs* kick, bool records_fresh, float4* f_out, double* rho_out, bool ev,
-                            const int* stop)
+                            const int* stop, bool defer)
 {
     float4* fo = f_out ? f_out : f_.get();
     double* ro = rho_out ? rho_out : rho_.get();
@@ -2198,7 +2178,7 @@ void MDSystem::force_passes(const KickArgs* kick, bool records_fresh, float4* f_
 #undef MAPP_FORCE
         prof_.end(stream_);
         pass_rows_ = G;
-        if (ev) reduce_rows(part_.get(), 2 * G, 7, red_.get());
+        if (ev && !(defer && 2 * G <= kStepRows)) reduce_rows(part_.get(), 2 * G, 7, red_.get());
         return;
     }
     if (alloy_list_) {
@@ -2217,7 +2197,7 @@ void MDSystem::force_passes(const KickArgs* kick, bool records_fresh, float4* f_
 #undef MAPP_FORCE
         prof_.end(stream_);
         pass_rows_ = G;
-        if (ev) reduce_rows(part_.get(), 2 * G, 7, red_.get());
+        if (ev && !(defer && 2 * G <= kStepRows)) reduce_rows(part_.get(), 2 * G, 7, red_.get());
         return;
     }
     const int lg = lanes_global();
@@ -2256,7 +2236,7 @@ void MDSystem::force_passes(const KickArgs* kick, bool records_fresh, float4* f_
 #undef MAPP_FORCE
     prof_.end(stream_);
     pass_rows_ = nb;
-    if (ev) reduce_rows(part_.get(), 2 * nb, 7, red_.get());
+    if (ev && !(defer && 2 * nb <= kStepRows)) reduce_rows(part_.get(), 2 * nb, 7, red_.get());
 }
 
 MDReport MDSystem::reduce_report(int)

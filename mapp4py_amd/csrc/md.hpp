@@ -19,6 +19,7 @@ constexpr uint32_t kIndexMask = (1u << kIndexBits) - 1u;  // image code in the h
 // and 51.7)
 constexpr int kLdsMinAtoms = 12288;
 constexpr int kAlloyMinAtoms = 49152;           // the same for several elements
+constexpr int kStepRows = 1024;                 // rows of sums that one workgroup adds up at the end of a step
 constexpr int kMinPartRows = 4096;              // see MDSystem::part_rows
 // the alloy passes' list holds the neighbor's element above a shorter index
 constexpr int kElemShift = 23, kAlloyElems = 4;
@@ -66,6 +67,10 @@ private:
     size_t knot_stride_ = 0;
     DevBuf<double> Ftab_;
 };
+
+// flags: the largest row of a list build that overflowed, an atom moved half
+// the skin, a run's steps are halted there, steps a run has finished
+enum { FL_OVER = 0, FL_REBUILD = 1, FL_HALT = 2, FL_DONE = 3 };
 
 // Box, cell grid and search radius of one neighbor build.
 struct CellGrid {
@@ -226,9 +231,11 @@ private:
     void build_list();
     // records_fresh: rec_ already holds the current positions (written by the skin check or a rebuild)
     // the two EAM passes; f_out / rho_out (nullptr: f_ and rho_) receive the
-    // forces and densities; nothing is computed where *stop is set
+    // forces and densities; nothing is computed where *stop is set; defer:
+    // at most kStepRows rows of energies and virials (2 pass_rows_, at part_)
+    // are left for the caller to add up
     void force_passes(const KickArgs* kick, bool records_fresh = false, float4* f_out = nullptr,
-                      double* rho_out = nullptr, bool ev = true, const int* stop = nullptr);
+                      double* rho_out = nullptr, bool ev = true, const int* stop = nullptr, bool defer = false);
     int part_rows() const;
     int lanes_lds() const;
     int lanes_global() const;
@@ -289,6 +296,7 @@ private:
     size_t rho_lds_bytes_ = 0, f_lds_bytes_ = 0;
     int pass_rows_ = 0;              // rows of kinetic partial sums written by the last force pass
     DevBuf<double> hist_;            // a run's T_part after each step
+    DevBuf<double> nst_;             // box, thermostats and sums of an NST run
     HostBuf<int> told_;              // what a run's steps tell the host
     // minimiser vectors in slot order: line-search origin, direction, forces
     // at the origin, L-BFGS pairs; a spare for permutations

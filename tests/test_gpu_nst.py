@@ -96,6 +96,38 @@ def test_immobile_box_gives_the_gpu_nvt_trajectory(M):
     assert abs(nst.T_part - nvt.T_part) < 1e-9 * nvt.T_part
 
 
+@pytest.mark.parametrize("cells,nreset", [(2, 3), (14, 0), (15, 4)])
+def test_step_ends_for_every_way_to_sum_the_rows(M, cells, nreset):
+    # 32 atoms; 10,976 (global tables, more rows of energies than the step's
+    # end adds up itself); 13,500 (splines in LDS). The virial bar of a single
+    # call, 2e-7 eV an atom from FP32 pair forces, moves a box edge of H by up
+    # to H (N dt / tau)^2 / 2 times 2e-7 / (3 kB T): 7e-6 A at H = 54 A over 10
+    # steps; held to the 1e-6 A of the longer runs
+    T, dt, nsteps = 300.0, 2.0 * pot.FS, 10
+    p, H, g, o, v, masses = setup(M, cells, 5, T)
+    S = np.full((3, 3), np.nan)
+    np.fill_diagonal(S, [0.02, 0.0, -0.01])
+    S[2, 1] = 0.01
+    tau = np.full((3, 3), 60.0 * pot.FS)
+    nst = M.NST(S, T, dt, kB=pot.KB_EV, tau=tau, nreset=nreset)
+    nst.run(g, nsteps, masses)
+    vo, Ho, Tpo, outo, histo, nro = o.nst_run(v, masses, pot.KB_EV, T, dt, S, nsteps, tau=tau, nreset=nreset)
+    say(f"{len(v)} atoms: max|dH| {np.abs(g.H - Ho).max():.2e} A, max|dx| {np.abs(g.x - o.x).max():.2e} A")
+    assert np.abs(g.H - Ho).max() < 1e-6 and np.abs(g.x - o.x).max() < 1e-6
+    assert np.abs(g.x_d - vo).max() < 1e-6
+    np.testing.assert_allclose(nst.hist[:, 1], histo[:, 1], rtol=0, atol=5e-8 * len(v) + 1e-6)
+    np.testing.assert_allclose(nst.hist[:, 0], histo[:, 0], rtol=1e-6)
+
+
+def test_a_box_that_leaves_its_bounds_stops_the_run(M):
+    p, H, g, o, v, masses = setup(M, 5, 3, 300.0)
+    S = np.full((3, 3), np.nan)
+    np.fill_diagonal(S, 0.2)
+    nst = M.NST(S, 300.0, 2.0 * pot.FS, kB=pot.KB_EV, tau=np.full((3, 3), 60.0 * pot.FS))
+    with pytest.raises(M.MappError, match="the box left"):
+        nst.run(g, 100, masses)
+
+
 def test_rejects_a_target_with_no_component(M):
     p, H, g, o, v, masses = setup(M, 4, 1, 300.0)
     nst = M.NST(np.full((3, 3), np.nan), 300.0, pot.FS, kB=pot.KB_EV)
