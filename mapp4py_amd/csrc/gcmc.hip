@@ -502,12 +502,442 @@ __global__ __launch_bounds__(256) void k_gcmc(GcmcArgs A, GcmcCell* cells, const
     }
 }
 
-// A batch of one cell (the grand-canonical exchange of an MD system, up to
-// 16,384 atoms) over one workgroup of 16 waves: each attempt's sweep over the
-// atoms takes a quarter of the steps of four waves.
+// ---- one large cell: several attempts at a time ----
+// A chain is serial, but most attempts are rejected and a rejected attempt
+// changes nothing except the random stream. So the waves of a workgroup take
+// the next attempts of the chain together, each from the stream as it is after
+// the attempts before it were rejected; the results count up to the first one
+// that was accepted, which its wave then carries out, and the chain goes on
+// after it. Decisions, stream and atom order are those of one attempt at a
+// time. A wave finds the atoms in reach of its trial point through bins of
+// about half a cut-off (some 200 candidates in a metal in place of all atoms);
+// what is inserted later is kept in a row of its own that every trial tests.
+// Needs a box wider than twice the gas cut-off, so that a trial point meets an
+// atom in one image only. 500 attempts in 11,000 atoms: 0.88 ms and
+// 0.04 for the bins; 6.0 with one attempt at a time over all atoms.
 constexpr int kGcmcOneWaves = 16;
-__global__ __launch_bounds__(64 * kGcmcOneWaves) void k_gcmc_one(GcmcArgs A, GcmcCell* cells, int nattempts,
-                                                                 int8_t* dec, double* dU, Arrays R)
+constexpr int kMaxBins = 8192;
+
+struct GcmcBins {
+    int nb[3], cap;
+    int* start;  // [bins + 1] first entry of a bin
+    int* ent;    // [2 cap] atoms by bin (-1: deleted), then those inserted since; a scratch half while binning
+    int* where;  // [cap] entry of an atom
+};
+
+__device__ inline int bin_coord(double s, int nb)
+{
+    const int b = (int)(s * (double)nb);
+    return b < 0 ? 0 : b < nb - 1 ? b : nb - 1;
+}
+__device__ inline int bin_of(const GcmcBins& B, const double4& s)
+{
+    return (bin_coord(s.z, B.nb[2]) * B.nb[1] + bin_coord(s.y, B.nb[1])) * B.nb[0] + bin_coord(s.x, B.nb[0]);
+}
+
+// bins [lo, lo + num) that lie within cs of t
+__device__ inline void bin_range(double t, double cs, int nb, int& lo, int& num)
+{
+    const double a = floor((t - cs - 1e-9) * (double)nb), b = floor((t + cs + 1e-9) * (double)nb);
+    lo = a < 0.0 ? 0 : (int)a;
+    num = (b < (double)nb ? (int)b : nb - 1) - lo + 1;
+}
+
+// The atoms of the cell by bin, in index order within a bin (an atom's place
+// is the number of smaller indices in its bin, so the order is the same in
+// every run).
+__global__ __launch_bounds__(1024) void k_gcmc_bins(const GcmcCell* __restrict__ cells, GcmcBins B, Arrays R)
+{
+    __shared__ int cnt[kMaxBins];
+    __shared__ int wsum[16];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int nbins = B.nb[0] * B.nb[1] * B.nb[2], n = cells[0].n;
+    const double4* s = R.s + cells[0].off;
+    int* tmp = B.ent + B.cap;
+    for (int b = t; b < kMaxBins; b += 1024) cnt[b] = 0;
+    __syncthreads();
+    for (int i = t; i < n; i += 1024) atomicAdd(&cnt[bin_of(B, s[i])], 1);
+    __syncthreads();
+    constexpr int P = kMaxBins / 1024;
+    int c[P], sum = 0;
+    for (int q = 0; q < P; ++q) {
+        c[q] = cnt[P * t + q];
+        sum += c[q];
+    }
+    int v = sum;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int u = __shfl(v, (lane - o) & 63, 64);
+        if (lane >= o) v += u;
+    }
+    if (lane == 63) wsum[w] = v;
+    __syncthreads();
+    int base = v - sum;
+    for (int q = 0; q < w; ++q) base += wsum[q];
+    for (int q = 0; q < P; ++q) {
+        cnt[P * t + q] = base;
+        if (P * t + q < nbins) B.start[P * t + q] = base;
+        base += c[q];
+    }
+    if (t == 0) B.start[nbins] = n;
+    __syncthreads();
+    for (int i = t; i < n; i += 1024) tmp[atomicAdd(&cnt[bin_of(B, s[i])], 1)] = i;
+    __syncthreads();
+    for (int i = t; i < n; i += 1024) {
+        const int b = bin_of(B, s[i]), first = B.start[b], last = cnt[b];
+        int rank = 0;
+        for (int k = first; k < last; ++k) rank += tmp[k] < i;
+        B.ent[first + rank] = i;
+        B.where[i] = first + rank;
+    }
+}
+
+constexpr int kModulus = 2147483647;
+__device__ inline int mulmod(int a, int b)
+{
+    const unsigned long long p = (unsigned long long)(unsigned)a * (unsigned)b;
+    unsigned long long r = (p & kModulus) + (p >> 31);
+    if (r >= kModulus) r -= kModulus;
+    return (int)r;
+}
+
+struct OneShared {
+    unsigned long long gas[4 * kGcmcWaveCap / 64];  // bit j % 64 of word j / 64: atom j is gas
+    double r2[kGcmcOneWaves][128];                  // pairs in reach: squared distance, atom and element
+    int hit[kGcmcOneWaves][128];
+    int first[kGcmcOneWaves][64], scan[kGcmcOneWaves][64];  // rows of candidates: first entry, candidates before it
+    double gval;
+    int n, ngas, nx, seed, chk, status, ev[kGcmcOneWaves];
+};
+constexpr int kElemBit = 14;  // above an atom's index in OneShared::hit
+
+// The exchange energy's sums for a trial point with images im of sb, one wave:
+// sum = pair energies, changes of F of the atoms in reach, density at the
+// point. Commit: those atoms take their new densities and F instead.
+template <bool Commit>
+__device__ inline void one_energy(const GcmcArgs& A, const double* h, const double* cs, const GcmcBins& B,
+                                  const Arrays& R, OneShared& S, int n0, int nx, const double* sb, const Images& im,
+                                  double c0, int del_idx, int w, int lane, double (&sum)[4])
+{
+    const int gas = A.gas, ne = A.ne, nr = A.nr;
+    double en = 0.0, en0 = 0.0, rhoi = 0.0;
+    // the first m pairs of the list, one a lane
+    const auto take = [&](int m) {
+        if (lane < m) {
+            const int j = S.hit[w][lane] & ((1 << kElemBit) - 1), ej = S.hit[w][lane] >> kElemBit;
+            const double r = sqrt(S.r2[w][lane]);
+            int k;
+            double p;
+            spline_at(r, A.dr_inv, nr, k, p);
+            en += hval(A.phi[(size_t)(gas * ne + ej) * nr + k], p) / r;
+            rhoi += hval(A.rho[(size_t)(ej * ne + gas) * nr + k], p);
+            const double rx = R.rho[j] + c0 * hval(A.rho[(size_t)(gas * ne + ej) * nr + k], p);
+            const double fx = f_embed(A, ej, rx, true);
+            en0 += fx - R.F[j];
+            if (Commit) {
+                R.rho[j] = rx;
+                R.F[j] = fx;
+            }
+        }
+    };
+    int cnt = 0;
+    const int ntrial = im.total();
+    for (int k = 0; k < ntrial; ++k) {
+        const int ik[3] = {k % im.cnt[0], (k / im.cnt[0]) % im.cnt[1], k / (im.cnt[0] * im.cnt[1])};
+        double x[3];
+        image_x(h, sb, im, k, x);
+        int lo[3], num[3];
+        for (int d = 0; d < 3; ++d) bin_range(image_coord(sb[d], im.up[d], ik[d]), cs[d], B.nb[d], lo[d], num[d]);
+        if (uni((int)(num[0] <= 0 || num[1] <= 0 || num[2] <= 0))) num[0] = num[1] = num[2] = 0;
+        // rows of bins along the first dimension, then the inserted atoms
+        const int nrow = num[1] * num[2];
+        int first = 0, len = 0;
+        if (lane < nrow) {
+            const int row = ((lo[2] + lane / num[1]) * B.nb[1] + lo[1] + lane % num[1]) * B.nb[0] + lo[0];
+            first = B.start[row];
+            len = B.start[row + num[0]] - first;
+        } else if (lane == nrow) {
+            first = n0;
+            len = nx;
+        }
+        int v = len;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int u = __shfl(v, (lane - o) & 63, 64);
+            if (lane >= o) v += u;
+        }
+        group_sync<1>();
+        S.first[w][lane] = first;
+        S.scan[w][lane] = v - len;
+        const int total = uni(__shfl(v, 63, 64));
+        group_sync<1>();
+        for (int q0 = 0; q0 < total; q0 += 128) {
+            int j[2];
+            double4 xj[2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const int q = q0 + 64 * u + lane;
+                int r = 0;
+#pragma unroll
+                for (int step = 32; step > 0; step >>= 1)
+                    if (S.scan[w][r + step] <= q) r += step;
+                j[u] = q < total ? B.ent[S.first[w][r] + (q - S.scan[w][r])] : -1;
+            }
+#pragma unroll
+            for (int u = 0; u < 2; ++u) xj[u] = R.xe[j[u] < 0 ? 0 : j[u]];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const int ej = (int)xj[u].w;
+                const double rsq = rsq_of(x[0], x[1], x[2], xj[u].x, xj[u].y, xj[u].z);
+                const bool hit = j[u] >= 0 && rsq < A.cut_sq[gas * ne + ej] && !(k == 0 && j[u] == del_idx);
+                const unsigned long long m = __ballot(hit);
+                if (hit) {
+                    const int at = cnt + __popcll(m & ((1ull << lane) - 1ull));
+                    S.r2[w][at] = rsq;
+                    S.hit[w][at] = j[u] | (ej << kElemBit);
+                }
+                cnt += __popcll(m);
+                if (cnt >= 64) {
+                    group_sync<1>();
+                    take(64);
+                    const double r2 = S.r2[w][64 + lane];
+                    const int hj = S.hit[w][64 + lane];
+                    group_sync<1>();
+                    S.r2[w][lane] = r2;
+                    S.hit[w][lane] = hj;
+                    cnt -= 64;
+                }
+            }
+        }
+    }
+    group_sync<1>();
+    take(cnt);
+    group_sync<1>();
+    sum[0] = en;
+    sum[1] = en0;
+    sum[2] = rhoi;
+    sum[3] = 0.0;
+    if (!Commit) wave_sums<4>(sum);
+}
+
+__global__ __launch_bounds__(64 * kGcmcOneWaves) void k_gcmc_one(GcmcArgs A, GcmcCell* cells, GcmcBins B,
+                                                                 int nattempts, int8_t* dec, double* dU, Arrays R)
+{
+    __shared__ OneShared S;
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int gas = A.gas, n0 = uni(cells[0].n), off = uni(cells[0].off), cap = uni(cells[0].cap);
+    double h[6], lo[3], hi[3], cs[3];
+    for (int k = 0; k < 6; ++k) h[k] = uni(cells[0].h[k]);
+    for (int d = 0; d < 3; ++d) {
+        lo[d] = uni(cells[0].lo[d]);
+        hi[d] = uni(cells[0].hi[d]);
+        cs[d] = -lo[d];
+    }
+    const double zv = uni(cells[0].zv);
+    R.xe += off;
+    R.s += off;
+    R.v += off;
+    R.rho += off;
+    R.F += off;
+    R.el += off;
+    if (threadIdx.x == 0) {
+        S.n = n0;
+        S.ngas = cells[0].ngas;
+        S.nx = 0;
+        S.seed = cells[0].seed;
+        S.chk = cells[0].gchk;
+        S.gval = cells[0].gval;
+        S.status = 0;
+    }
+    for (int q = w; q < 4 * kGcmcWaveCap / 64; q += kGcmcOneWaves) {
+        const int j = 64 * q + lane;
+        const unsigned long long m = __ballot(j < n0 ? R.el[j] == gas : 0);
+        if (lane == 0) S.gas[q] = m;
+    }
+    // a draw k steps ahead is the seed times 16807^(k + 1): lane k has draws k and 64 + k
+    int pw[2] = {16807, 16807};
+    for (int k = 0; k < 127; ++k) {
+        if (k < lane) pw[0] = mulmod(pw[0], 16807);
+        if (k < 64 + lane) pw[1] = mulmod(pw[1], 16807);
+    }
+    __syncthreads();
+    int a = 0;
+    while (a < nattempts) {
+        const int n = uni(S.n), ngas = uni(S.ngas), nx = uni(S.nx), seed = uni(S.seed);
+        int sd[2];
+        double un[2];
+        for (int q = 0; q < 2; ++q) {
+            if (seed > 0 && seed < kModulus) {
+                sd[q] = mulmod(seed, pw[q]);
+            } else {  // outside the generator's cycle: step by step
+                Stream st{seed, 0, 0.0};
+                for (int k = 0; k <= 64 * q + lane; ++k) (void)st.uniform();
+                sd[q] = st.seed;
+            }
+            un[q] = sd[q] * 1.0 / 2147483647;
+        }
+        const auto draw = [&](int k) { return uni(__shfl(k < 64 ? un[0] : un[1], k & 63, 64)); };
+        const auto seed_after = [&](int k) { return uni(__shfl(k <= 64 ? sd[0] : sd[1], (k - 1) & 63, 64)); };
+        const unsigned long long b0 = __ballot(un[0] < 0.5), b1 = __ballot(un[1] < 0.5);
+        const auto is_ins = [&](int k) { return (int)(((k < 64 ? b0 : b1) >> (k & 63)) & 1ull); };
+        int pos = 0;
+        for (int q = 0; q < w; ++q) pos += is_ins(pos) ? 5 : ngas ? 3 : 1;
+        const bool ins = uni(is_ins(pos)), on = a + w < nattempts;
+        int next = pos + (ins ? 5 : ngas ? 3 : 1);
+        int ev = 0, status = 0, del_idx = -1, d8 = 0;
+        double du = 0.0, rhoi = 0.0, sb[3];
+        const double c0 = ins ? 1.0 : -1.0;
+        Images im{};
+        if (on && (ins || ngas)) {
+            if (ins) {
+                for (int d = 0; d < 3; ++d) sb[d] = draw(pos + 1 + d);
+            } else {
+                // igas-th gas atom in index order: lane l has the words 4 l ... 4 l + 3
+                const int igas = (int)(ngas * draw(pos + 1));
+                unsigned long long g[4];
+                int mine = 0;
+                for (int q = 0; q < 4; ++q) {
+                    g[q] = S.gas[4 * lane + q];
+                    mine += __popcll(g[q]);
+                }
+                int v = mine;
+                for (int o = 1; o < 64; o <<= 1) {
+                    const int u = __shfl(v, (lane - o) & 63, 64);
+                    if (lane >= o) v += u;
+                }
+                int k = igas - (v - mine), idx = -1;
+                if (k >= 0 && k < mine)
+                    for (int q = 0; q < 4 && idx < 0; ++q) {
+                        const int c = __popcll(g[q]);
+                        if (k < c) {
+                            unsigned long long m = g[q];
+                            for (int t = 0; t < k; ++t) m &= m - 1;
+                            idx = 64 * (4 * lane + q) + __ffsll((long long)m) - 1;
+                        }
+                        k -= c;
+                    }
+                const unsigned long long has = __ballot(idx >= 0);
+                del_idx = has ? uni(__shfl(idx, __ffsll((long long)has) - 1, 64)) : -1;
+                if (del_idx < 0) {  // gas count and element array disagree: stop this chain
+                    ev = 1;
+                    status = 2;
+                    next = pos + 2;
+                } else {
+                    const double4 s4 = R.s[del_idx];
+                    sb[0] = uni(s4.x);
+                    sb[1] = uni(s4.y);
+                    sb[2] = uni(s4.z);
+                }
+            }
+            if (!status) {
+                im = count_images(sb, lo, hi);
+                double sum[4];
+                one_energy<false>(A, h, cs, B, R, S, n0, nx, sb, im, c0, del_idx, w, lane, sum);
+                const double en = uni(__shfl(sum[0], 0, 64)), en0 = uni(__shfl(sum[0], 2, 64));
+                rhoi = uni(__shfl(sum[0], 1, 64));
+                du = en + en0 * c0;
+                du = du + f_embed(A, gas, rhoi, true);
+                const double u = draw(next - 1);
+                const bool acc = ins ? u < zv / (((double)ngas + 1.0) * exp(A.beta * du))
+                                     : u < (double)ngas * exp(A.beta * du) / zv;
+                ev = acc;
+                d8 = ins ? (acc ? 1 : -1) : (acc ? 2 : -2);
+            }
+        }
+        if (lane == 0) S.ev[w] = ev;
+        __syncthreads();
+        const unsigned long long evs = __ballot(lane < kGcmcOneWaves && S.ev[lane & (kGcmcOneWaves - 1)] != 0);
+        const int left = nattempts - a;
+        const int done = evs ? __ffsll((long long)evs) : left < kGcmcOneWaves ? left : kGcmcOneWaves;
+        if (w < done && dec && !status && lane == 0) {
+            dec[a + w] = (int8_t)d8;
+            dU[a + w] = du;
+        }
+        if (w == done - 1) {
+            int seed1 = seed_after(next);
+            if (ev && !status && ins && n == cap) status = 1;
+            if (ev && !status) {
+                double sum[4];
+                one_energy<true>(A, h, cs, B, R, S, n0, nx, sb, im, c0, del_idx, w, lane, sum);
+                group_sync<1>();
+                if (ins) {
+                    Stream st{seed1, uni(S.chk), uni(S.gval)};
+                    double vel[3], x[3];
+                    for (int d = 0; d < 3; ++d) vel[d] = st.gaussian() * A.sigma;
+                    image_x(h, sb, im, 0, x);
+                    const double F = f_embed(A, gas, rhoi, true);
+                    seed1 = st.seed;
+                    group_sync<1>();
+                    if (lane == 0) {
+                        R.xe[n] = make_double4(x[0], x[1], x[2], (double)gas);
+                        R.s[n] = make_double4(sb[0], sb[1], sb[2], 0.0);
+                        R.v[n] = make_double4(vel[0], vel[1], vel[2], 0.0);
+                        R.rho[n] = rhoi;
+                        R.F[n] = F;
+                        R.el[n] = (uint8_t)gas;
+                        B.ent[n0 + nx] = n;
+                        B.where[n] = n0 + nx;
+                        S.gas[n >> 6] |= 1ull << (n & 63);
+                        S.nx = nx + 1;
+                        S.n = n + 1;
+                        S.ngas = ngas + 1;
+                        S.chk = st.chk;
+                        S.gval = st.keep;
+                    }
+                } else if (lane == 0) {
+                    // the deleted atom's entry goes; the last atom takes its index
+                    const int e = B.where[del_idx], last = n - 1;
+                    if (e < n0) {
+                        B.ent[e] = -1;
+                    } else {
+                        const int j = B.ent[n0 + nx - 1];
+                        B.ent[e] = j;
+                        B.where[j] = e;
+                        S.nx = nx - 1;
+                    }
+                    S.gas[del_idx >> 6] &= ~(1ull << (del_idx & 63));
+                    if (del_idx != last) {
+                        const int el = B.where[last];
+                        B.ent[el] = del_idx;
+                        B.where[del_idx] = el;
+                        R.xe[del_idx] = R.xe[last];
+                        R.s[del_idx] = R.s[last];
+                        R.v[del_idx] = R.v[last];
+                        R.rho[del_idx] = R.rho[last];
+                        R.F[del_idx] = R.F[last];
+                        R.el[del_idx] = R.el[last];
+                        if ((S.gas[last >> 6] >> (last & 63)) & 1ull) {
+                            S.gas[last >> 6] &= ~(1ull << (last & 63));
+                            S.gas[del_idx >> 6] |= 1ull << (del_idx & 63);
+                        }
+                    }
+                    S.n = last;
+                    S.ngas = ngas - 1;
+                }
+            }
+            if (lane == 0) {
+                S.seed = seed1;
+                S.status = status;
+            }
+        }
+        __syncthreads();
+        if (uni(S.status)) break;
+        a += done;
+    }
+    if (threadIdx.x == 0) {
+        GcmcCell& o = cells[0];
+        o.n = S.n;
+        o.ngas = S.ngas;
+        o.seed = S.seed;
+        o.gchk = S.chk;
+        o.gval = S.gval;
+        o.status = S.status;
+    }
+}
+
+// One cell in a narrower box: one attempt at a time, 16 waves on all atoms.
+__global__ __launch_bounds__(64 * kGcmcOneWaves) void k_gcmc_one_sweep(GcmcArgs A, GcmcCell* cells,
+                                                                       int nattempts, int8_t* dec, double* dU,
+                                                                       Arrays R)
 {
     __shared__ double trial[3 * kGcmcMaxTrials];
     __shared__ double red[4 * kGcmcOneWaves];
@@ -599,6 +1029,53 @@ __global__ __launch_bounds__(256) void k_gcmc_init_cell(GcmcArgs A, const GcmcCe
     const GcmcCell hd = cells[c];
     const int i = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);  // uniform over the wave
     if (i < hd.n) init_atom_wave(A, hd, R, i, (int)(threadIdx.x & 63));
+}
+
+// the same from the bins (k_gcmc_bins): eight lanes take a row of bins, and
+// only the atoms in reach are tested (11,000 atoms: 608 us over all pairs, 73
+// with the binning)
+__global__ __launch_bounds__(256) void k_gcmc_init_binned(GcmcArgs A, const GcmcCell* __restrict__ cells, GcmcBins B,
+                                                          Arrays R)
+{
+    const GcmcCell& hd = cells[0];
+    const int i = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);  // uniform over the wave
+    const int lane = threadIdx.x & 63, off = hd.off, ne = A.ne, nr = A.nr;
+    if (i >= hd.n) return;
+    const double4 si4 = R.s[off + i];
+    const double si[3] = {si4.x, si4.y, si4.z};
+    const int ei = (int)R.xe[off + i].w;
+    const Images im = count_images(si, hd.lo2, hd.hi2);
+    double rho = 0.0;
+    for (int k = 0; k < im.total(); ++k) {
+        const int ik[3] = {k % im.cnt[0], (k / im.cnt[0]) % im.cnt[1], k / (im.cnt[0] * im.cnt[1])};
+        double xi[3];
+        image_x(hd.h, si, im, k, xi);
+        int lo[3], num[3];
+        for (int d = 0; d < 3; ++d)
+            bin_range(image_coord(si[d], im.up[d], ik[d]), -hd.lo2[d], B.nb[d], lo[d], num[d]);
+        if (num[0] <= 0 || num[1] <= 0 || num[2] <= 0) continue;
+        for (int q = lane >> 3; q < num[1] * num[2]; q += 8) {
+            const int row = ((lo[2] + q / num[1]) * B.nb[1] + lo[1] + q % num[1]) * B.nb[0] + lo[0];
+            const int last = B.start[row + num[0]];
+            for (int e = B.start[row] + (lane & 7); e < last; e += 8) {
+                const int j = B.ent[e];
+                if (k == 0 && j == i) continue;
+                const double4 xj = R.xe[off + j];
+                const int ej = (int)xj.w;
+                const double rsq = rsq_of(xi[0], xi[1], xi[2], xj.x, xj.y, xj.z);
+                if (rsq >= A.cut_sq[ei * ne + ej]) continue;
+                int m;
+                double p;
+                spline_at(sqrt(rsq), A.dr_inv, nr, m, p);
+                rho += hval(A.rho[(size_t)(ej * ne + ei) * nr + m], p);
+            }
+        }
+    }
+    for (int o = 32; o > 0; o >>= 1) rho += __shfl_xor(rho, o, 64);
+    if (lane == 0) {
+        R.rho[off + i] = rho;
+        R.F[off + i] = f_embed(A, ei, rho, false);
+    }
 }
 
 // ---- single-trial hooks (one cell, one trial, driven by the caller) ----
@@ -781,8 +1258,18 @@ Arrays arrays_of(GcmcState& st)
                   st.el.get()};
 }
 
-void alloc_state(GcmcState& st, int nc, size_t cap)
+GcmcBins bins_of(GcmcState& st, const int* nb, size_t cap)
 {
+    return GcmcBins{{nb[0], nb[1], nb[2]}, (int)cap, st.bin_start.get(), st.bin_ent.get(), st.bin_where.get()};
+}
+
+void alloc_state(GcmcState& st, int nc, size_t cap, bool binned)
+{
+    if (binned) {
+        st.bin_start.reserve(kMaxBins + 1);
+        st.bin_ent.reserve(2 * cap);
+        st.bin_where.reserve(cap);
+    }
     st.cells.reserve(nc);
     st.xe.reserve(cap);
     st.s.reserve(cap);
@@ -900,7 +1387,20 @@ GcmcBatch::GcmcBatch(std::shared_ptr<EamForceField> ff, int ncells, const int* n
         natot += natms[c];
     }
     total_cap_ = off;
-    alloc_state(st_, ncells, total_cap_);
+    // bins of at least half the gas cut-off, at most kMaxBins of them
+    const GcmcCell& c0 = host_cells_[0];
+    binned_ = ncells == 1 && -c0.lo[0] < 0.5 && -c0.lo[1] < 0.5 && -c0.lo[2] < 0.5;
+    if (binned_) {
+        double nb[3], total = 1.0;
+        for (int d = 0; d < 3; ++d) total *= nb[d] = std::min(1e6, std::floor(2.0 / -c0.lo[d]));
+        while (total > kMaxBins) {
+            const double f = std::cbrt(kMaxBins / total);
+            total = 1.0;
+            for (int d = 0; d < 3; ++d) total *= nb[d] = std::max(1.0, std::floor(nb[d] * f));
+        }
+        for (int d = 0; d < 3; ++d) nbins_[d] = (int)nb[d];
+    }
+    alloc_state(st_, ncells, total_cap_, binned_);
     {
         std::vector<double4> xe(total_cap_), sv(total_cap_), vv(total_cap_, make_double4(0, 0, 0, 0));
         std::vector<uint8_t> el(total_cap_, 0);
@@ -930,9 +1430,7 @@ GcmcBatch::GcmcBatch(std::shared_ptr<EamForceField> ff, int ncells, const int* n
     MAPP_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
     queue_.reserve(2);
     if (ncells == 1) {
-        if (host_cells_[0].n)
-            k_gcmc_init_cell<<<(host_cells_[0].n + 3) / 4, 256, 0, stream_>>>(A_, st_.cells.get(), 0,
-                                                                             arrays_of(st_));
+        init_cell(0);
     } else {
         k_gcmc_init<<<ncells, 256, 0, stream_>>>(A_, st_.cells.get(), arrays_of(st_));
     }
@@ -952,6 +1450,21 @@ GcmcBatch::~GcmcBatch()
         (void)hipStreamSynchronize(stream_);
         (void)hipStreamDestroy(stream_);
     }
+}
+
+// densities and F of cell c's atoms
+void GcmcBatch::init_cell(int c)
+{
+    const int n = host_cells_[c].n;
+    if (n == 0) return;
+    if (binned_) {
+        const GcmcBins B = bins_of(st_, nbins_, total_cap_);
+        k_gcmc_bins<<<1, 1024, 0, stream_>>>(st_.cells.get(), B, arrays_of(st_));
+        k_gcmc_init_binned<<<(n + 3) / 4, 256, 0, stream_>>>(A_, st_.cells.get(), B, arrays_of(st_));
+    } else {
+        k_gcmc_init_cell<<<(n + 3) / 4, 256, 0, stream_>>>(A_, st_.cells.get(), c, arrays_of(st_));
+    }
+    MAPP_HIP(hipGetLastError());
 }
 
 void GcmcBatch::set_waves(const int* waves)
@@ -998,7 +1511,15 @@ void GcmcBatch::launch(GcmcState& st, int nattempts, int8_t* dec, double* du, co
                        int n1)
 {
     if (nc_ == 1) {
-        k_gcmc_one<<<1, 64 * kGcmcOneWaves, 0, stream_>>>(A_, st.cells.get(), nattempts, dec, du, arrays_of(st));
+        if (binned_) {
+            const GcmcBins B = bins_of(st, nbins_, total_cap_);
+            k_gcmc_bins<<<1, 1024, 0, stream_>>>(st.cells.get(), B, arrays_of(st));
+            k_gcmc_one<<<1, 64 * kGcmcOneWaves, 0, stream_>>>(A_, st.cells.get(), B, nattempts, dec, du,
+                                                              arrays_of(st));
+        } else {
+            k_gcmc_one_sweep<<<1, 64 * kGcmcOneWaves, 0, stream_>>>(A_, st.cells.get(), nattempts, dec, du,
+                                                                    arrays_of(st));
+        }
         MAPP_HIP(hipGetLastError());
         return;
     }
@@ -1068,7 +1589,7 @@ void GcmcBatch::attempts(int nattempts, int8_t* decisions, double* dU)
 
 void GcmcBatch::copy_state(GcmcState& dst, const GcmcState& src)
 {
-    alloc_state(dst, nc_, total_cap_);
+    alloc_state(dst, nc_, total_cap_, binned_);
     MAPP_HIP(hipMemcpyAsync(dst.cells.get(), src.cells.get(), nc_ * sizeof(GcmcCell), hipMemcpyDeviceToDevice,
                             stream_));
     MAPP_HIP(hipMemcpyAsync(dst.xe.get(), src.xe.get(), total_cap_ * sizeof(double4), hipMemcpyDeviceToDevice,
@@ -1242,10 +1763,7 @@ void GcmcBatch::load_cell(int c, int n, const double* x, const uint8_t* elem, co
     MAPP_HIP(hipMemcpy(st_.cells.get() + c, &hc, sizeof(GcmcCell), hipMemcpyHostToDevice));
     host_cells_[c].n = n;
     host_cells_[c].ngas = ngas;
-    if (n) {
-        k_gcmc_init_cell<<<(n + 3) / 4, 256, 0, stream_>>>(A_, st_.cells.get(), c, arrays_of(st_));
-        MAPP_HIP(hipGetLastError());
-    }
+    init_cell(c);
     MAPP_HIP(hipStreamSynchronize(stream_));
     ++ver_;
     pending_.cell = -1;

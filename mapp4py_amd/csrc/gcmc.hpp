@@ -46,6 +46,7 @@ struct GcmcState {
     DevBuf<double4> v;
     DevBuf<double> rho, F, rho_x, F_x;
     DevBuf<uint8_t> el;
+    DevBuf<int> bin_start, bin_ent, bin_where;  // one cell: its atoms by bin
 };
 
 struct GcmcTuneReport {
@@ -83,6 +84,7 @@ public:
 private:
     void split_cells(const int* waves, std::vector<int>& q4, std::vector<int>& q1) const;
     void build_queues();
+    void init_cell(int c);
     void launch(GcmcState& st, int nattempts, int8_t* dec, double* du, const int* q4, int n4, const int* q1, int n1);
     void copy_state(GcmcState& dst, const GcmcState& src);
     void check_status(GcmcState& st);
@@ -90,6 +92,8 @@ private:
     std::shared_ptr<EamForceField> ff_;
     int nc_ = 0;
     size_t total_cap_ = 0;
+    bool binned_ = false;  // one cell in a box wider than twice the gas cut-off
+    int nbins_[3] = {1, 1, 1};
     GcmcArgs A_{};
     hipStream_t stream_ = nullptr;
     std::vector<GcmcCell> host_cells_;

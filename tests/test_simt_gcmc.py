@@ -139,6 +139,31 @@ def test_emulated_one_cell_batch_reproduces_the_oracle_chain(emu):
     assert states[0]["seed"] == g.rng_seed and states[0]["ngas"] == g.ngas
 
 
+@pytest.mark.parametrize("mu,seed,gas_share", [(-2.3, 4242, 0.05), (-0.5, 7, 0.0), (-3.5, 99, 0.3),
+                                                (-2.0, -17, 0.1)])
+def test_emulated_attempts_of_a_wide_cell_reproduce_the_oracle_chain(emu, mu, seed, gas_share):
+    # a box wider than twice the gas cut-off: 16 attempts at a time over bins.
+    # Many insertions, many deletions (of first and of inserted atoms, the
+    # last one included), no gas at first, a seed outside the generator's cycle
+    rng = np.random.default_rng(5)
+    H = np.array([[14.1, 0, 0], [1.5, 15.2, 0], [-0.8, 1.1, 13.9]])
+    x = (rng.uniform(0, 1, (70, 3))) @ H
+    e = np.where(rng.uniform(0, 1, 70) < gas_share, GAS, 0).astype(np.uint8)
+    ks = [7, 45]
+    dec, du, states = run(emu, [(x, H, e)], mu, np.array([seed], np.int32), ks, 4, False)
+    g = O.OGCMC(O.OEam.read(pot.NIALH_JEA), H, x, e, GAS, mu, 300.0, MASSES, seed=seed)
+    got = [g.attempts(k) for k in ks]
+    np.testing.assert_array_equal(dec[0], np.concatenate([d for d, _ in got]))
+    u = np.concatenate([u for _, u in got])
+    assert np.abs(du[0] - u).max() < 1e-9 * max(1.0, np.abs(u).max())
+    print(f"mu {mu} seed {seed}: {np.bincount(dec[0] + 2, minlength=5)} of -2 ... 2")
+    st = g.state()
+    np.testing.assert_array_equal(states[0]["elem"], st["elem"])
+    np.testing.assert_array_equal(states[0]["x"], st["x"])
+    np.testing.assert_allclose(states[0]["rho"], st["rho"], rtol=1e-10, atol=1e-12)
+    assert states[0]["seed"] == g.rng_seed and states[0]["ngas"] == g.ngas
+
+
 def test_emulated_single_trial_hooks_follow_the_oracle_chain(emu):
     # the hook kernels (one trial's exchange energy, its commit) driven by a
     # caller-side SGCMC::attmpt with the reference's draw order: the oracle's
