@@ -728,7 +728,7 @@ __global__ void k_replica_reset(int* queue)
 
 ReplicaBatch::ReplicaBatch(std::shared_ptr<EamForceField> ff, int nrep, const int* natms, const double* H,
                            const double* x, const uint8_t* elem, double skin)
-    : ff_(std::move(ff)), nr_(nrep), skin_(skin)
+    : ff_(std::move(ff)), nr_(nrep)
 {
     const EamTables& tb = ff_->tables();
     MAPP_REQUIRE(!tb.dmd, ERR_ARG, "replica minimisation needs a plain (non-DMD) EAM force field");

@@ -93,7 +93,6 @@ private:
     std::shared_ptr<EamForceField> ff_;
     int nr_ = 0;
     size_t natot_ = 0, ltot_ = 0;
-    double skin_ = 0.0;
     RepArgs A0_{};
     hipStream_t stream_ = nullptr;
     std::vector<RepCell> host_cells_;
