@@ -164,6 +164,27 @@ def test_emulated_attempts_of_a_wide_cell_reproduce_the_oracle_chain(emu, mu, se
     assert states[0]["seed"] == g.rng_seed and states[0]["ngas"] == g.ngas
 
 
+@pytest.mark.parametrize("waves", [1, 4])
+def test_emulated_cells_with_more_pairs_than_the_list_holds(emu, waves):
+    # 256 pairs a wave are listed; a dense cell (about 300 atoms in reach of a
+    # point) is swept in place, next to one that fits
+    rng = np.random.default_rng(8)
+    H = np.diag([10.6, 10.7, 10.8])
+    cells = [((rng.uniform(0, 1, (n, 3))) @ H, H, np.where(rng.uniform(0, 1, n) < 0.1, GAS, 0).astype(np.uint8))
+             for n in (560 * waves, 40)]
+    seeds = np.array([5, 6], np.int32)
+    dec, du, states = run(emu, cells, -2.0, seeds, [8], waves, False)
+    off = O.OEam.read(pot.NIALH_JEA)
+    for c, (x, Hc, e) in enumerate(cells):
+        g = O.OGCMC(off, Hc, x, e, GAS, -2.0, 300.0, MASSES, seed=int(seeds[c]))
+        d, u = g.attempts(8)
+        np.testing.assert_array_equal(dec[c], d)
+        assert np.abs(du[c] - u).max() < 1e-9 * max(1.0, np.abs(u).max())
+        st = g.state()
+        np.testing.assert_array_equal(states[c]["x"], st["x"])
+        np.testing.assert_allclose(states[c]["rho"], st["rho"], rtol=1e-10, atol=1e-12)
+
+
 def test_emulated_single_trial_hooks_follow_the_oracle_chain(emu):
     # the hook kernels (one trial's exchange energy, its commit) driven by a
     # caller-side SGCMC::attmpt with the reference's draw order: the oracle's
