@@ -1291,16 +1291,20 @@ __global__ __launch_bounds__(kBlock) void k_dmd_jex(int nc, int lg, const double
 // of F'(rho_i), times c_i); every component sums its own list (the
 // reference's half list adds the j side of each pair in the same loop). The
 // thread of a site's first component also writes xs of the site.
-__global__ __launch_bounds__(kBlock) void k_dmd_ja1(int nc, int lg, int C, const double* __restrict__ cc, int ldl, JState J,
+// Split: 2^lg lanes a row, four entries of a lane in flight; else one lane and
+// the loop as it is (524,288 components: a product with its copies 1.36 ms, unrolled 1.57)
+template <bool Split>
+__global__ __launch_bounds__(kBlock) void k_dmd_ja1(int nc, int lg_, int C, const double* __restrict__ cc, int ldl, JState J,
                                                     const double* __restrict__ xv, double2* __restrict__ a1x,
                                                     double* __restrict__ xs)
 {
+    const int lg = Split ? lg_ : 0;
     const int ic = (int)(((long)xcd_block() * kBlock + threadIdx.x) >> lg), g = threadIdx.x & ((1 << lg) - 1);
     if (ic >= nc) return;
     const double ci = cc[ic];
     double s = 0.0;
     const int cnt = J.cnt[ic];
-#pragma unroll 4
+#pragma unroll (Split ? 4 : 1)
     for (int k = g; k < cnt; k += 1 << lg) {
         const size_t slot = (size_t)k * ldl + ic;
         s += J.r2[slot] * xv[J.idx[slot]];
@@ -1319,14 +1323,16 @@ __global__ __launch_bounds__(kBlock) void k_dmd_ja1(int nc, int lg, int C, const
 
 // product, second sum: b0_i = sum_j rho_{i->j} A1_j + t0 x_j, the change of
 // the chemical potential mu_i
-__global__ __launch_bounds__(kBlock) void k_dmd_jb0(int nc, int lg, int ldl, JState J, const double2* __restrict__ a1x,
+template <bool Split>
+__global__ __launch_bounds__(kBlock) void k_dmd_jb0(int nc, int lg_, int ldl, JState J, const double2* __restrict__ a1x,
                                                     double* __restrict__ b0)
 {
+    const int lg = Split ? lg_ : 0;
     const int ic = (int)(((long)xcd_block() * kBlock + threadIdx.x) >> lg), g = threadIdx.x & ((1 << lg) - 1);
     if (ic >= nc) return;
     double s = 0.0;
     const int cnt = J.cnt[ic];
-#pragma unroll 4
+#pragma unroll (Split ? 4 : 1)
     for (int k = g; k < cnt; k += 1 << lg) {
         const size_t slot = (size_t)k * ldl + ic;
         const double2 v = a1x[J.idx[slot]];
@@ -2910,9 +2916,11 @@ void DMDSystem::J_dev(const double* x, double* ax)
     const JState js = jstate();
     prof_.begin(K_DMD_J, stream_);
     const int lg = lanes(nc_, kWalkThreads), nbl = grid_lanes(nc_, lg);
-    hipLaunchKernelGGL(k_dmd_ja1, dim3(nbl), dim3(kBlock), 0, stream_, nc_, lg, C_, c_.get(), ldl_, js, x, ja1_.get(),
+    const auto first = lg ? k_dmd_ja1<true> : k_dmd_ja1<false>;
+    const auto second = lg ? k_dmd_jb0<true> : k_dmd_jb0<false>;
+    hipLaunchKernelGGL(first, dim3(nbl), dim3(kBlock), 0, stream_, nc_, lg, C_, c_.get(), ldl_, js, x, ja1_.get(),
                        jxs_.get());
-    hipLaunchKernelGGL(k_dmd_jb0, dim3(nbl), dim3(kBlock), 0, stream_, nc_, lg, ldl_, js, ja1_.get(), jb0_.get());
+    hipLaunchKernelGGL(second, dim3(nbl), dim3(kBlock), 0, stream_, nc_, lg, ldl_, js, ja1_.get(), jb0_.get());
     hipLaunchKernelGGL(k_dmd_jax, dim3(nbc), dim3(kBlock), 0, stream_, nc_, C_, ldl_, js, jb0_.get(), x, jxs_.get(),
                        ax);
     prof_.end(stream_);
