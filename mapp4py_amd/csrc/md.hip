@@ -9,6 +9,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <iterator>
 #include <numeric>
 
 #include <mutex>
@@ -878,8 +879,10 @@ struct UnitWalk {
     }
 };
 
-template <int B>
-__global__ __launch_bounds__(kBigBlock) void k_eam_rho_lds(int n, int lg, const int* __restrict__ stop,
+// Split: 2^lg lanes an atom; else one, known to the compiler (1,048,574 atoms with
+// energies: 119 and 155 us a pass so, 120 and 163 with lg at run time)
+template <int B, bool Split>
+__global__ __launch_bounds__(kBigBlock) void k_eam_rho_lds(int n, int lg_, const int* __restrict__ stop,
                                                            const uint4* __restrict__ rec,
                                                            const int* __restrict__ nn,
                                                            const uint4* __restrict__ list4, int ldl, int maxb,
@@ -899,6 +902,7 @@ __global__ __launch_bounds__(kBigBlock) void k_eam_rho_lds(int n, int lg, const 
     __syncthreads();
     if (stop && *stop) return;
     const RhoRowsLds T{P.tabA, lds_rows, m_lo};
+    const int lg = Split ? lg_ : 0;
     const int g = threadIdx.x & ((1 << lg) - 1), unit = 64 >> lg;
     double acc[1] = {0.0};
     UnitWalk walk(n, unit, (int)blockIdx.x / kXcd, (int)gridDim.x / kXcd);
@@ -917,8 +921,8 @@ __global__ __launch_bounds__(kBigBlock) void k_eam_rho_lds(int n, int lg, const 
     block_sum_store<1, kBigBlock>(acc, part + (size_t)blockIdx.x * kPartW);
 }
 
-template <int B, bool EV>
-__global__ __launch_bounds__(kBigBlock) void k_eam_force_lds(int n, int lg, const int* __restrict__ stop,
+template <int B, bool EV, bool Split>
+__global__ __launch_bounds__(kBigBlock) void k_eam_force_lds(int n, int lg_, const int* __restrict__ stop,
                                                              const uint4* __restrict__ xr, Rec16Frame R,
                                                              const int* __restrict__ nn,
                                                              const uint4* __restrict__ list4, int ldl, int maxb,
@@ -952,6 +956,7 @@ __global__ __launch_bounds__(kBigBlock) void k_eam_force_lds(int n, int lg, cons
     __syncthreads();
     if (stop && *stop) return;
     const ForceRowsLds T{P.tabC, lds_rows, w2, w1, m_lo};
+    const int lg = Split ? lg_ : 0;
     const int g = threadIdx.x & ((1 << lg) - 1), unit = 64 >> lg;
     double acc[7] = {0, 0, 0, 0, 0, 0, 0};
     double mvv[6] = {0, 0, 0, 0, 0, 0};
@@ -1786,13 +1791,25 @@ void MDSystem::plan_lds()
     rho_lds_bytes_ = (size_t)rho_nwin_ * 16;
     f_lds_bytes_ = (size_t)f_nwin_ * 28;
     lds_grid_ = std::max(1, ncu / kXcd) * kXcd;
-    const void* fns[] = {(const void*)k_eam_rho_lds<1>,         (const void*)k_eam_rho_lds<2>,
-                         (const void*)k_eam_rho_lds<4>,         (const void*)k_eam_rho_lds<8>,
-                         (const void*)k_eam_force_lds<1, true>, (const void*)k_eam_force_lds<2, true>,
-                         (const void*)k_eam_force_lds<1, false>, (const void*)k_eam_force_lds<2, false>,
-                         (const void*)k_eam_force_lds<4, false>};
-    for (int k = 0; k < 9; ++k) {
-        const size_t bytes = k < 4 ? rho_lds_bytes_ : f_lds_bytes_;
+    const void* fns[] = {(const void*)k_eam_rho_lds<1, false>,
+                         (const void*)k_eam_rho_lds<2, false>,
+                         (const void*)k_eam_rho_lds<4, false>,
+                         (const void*)k_eam_rho_lds<8, false>,
+                         (const void*)k_eam_rho_lds<1, true>,
+                         (const void*)k_eam_rho_lds<2, true>,
+                         (const void*)k_eam_rho_lds<4, true>,
+                         (const void*)k_eam_force_lds<1, true, false>,
+                         (const void*)k_eam_force_lds<1, true, true>,
+                         (const void*)k_eam_force_lds<2, true, false>,
+                         (const void*)k_eam_force_lds<2, true, true>,
+                         (const void*)k_eam_force_lds<1, false, false>,
+                         (const void*)k_eam_force_lds<1, false, true>,
+                         (const void*)k_eam_force_lds<2, false, false>,
+                         (const void*)k_eam_force_lds<2, false, true>,
+                         (const void*)k_eam_force_lds<4, false, false>,
+                         (const void*)k_eam_force_lds<4, false, true>};
+    for (size_t k = 0; k < std::size(fns); ++k) {
+        const size_t bytes = k < 7 ? rho_lds_bytes_ : f_lds_bytes_;
         if (hipFuncSetAttribute(fns[k], hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess) {
             (void)hipGetLastError();
             return;
@@ -2150,21 +2167,17 @@ void MDSystem::force_passes(const KickArgs* kick, bool records_fresh, float4* f_
         // at most one workgroup per CU, and no more than there are units (rounded up to the 8 XCDs)
         const int G = std::min(lds_grid_, (units + kXcd - 1) / kXcd * kXcd);
         const int br = lg && batch_rho_ > 4 ? 4 : batch_rho_;
-#define MAPP_RHO(B) hipLaunchKernelGGL((k_eam_rho_lds<B>), dim3(G), dim3(kBigBlock), rho_lds_bytes_, stream_, n_, lg, \
-                                       stop, rec_.get(), nn_.get(), list4(), ldl_, maxb, P, r16_, rho_m_lo_, \
-                                       rho_nwin_, ro, xr_.get(), part_.get())
-        switch (br) {
-            case 1: MAPP_RHO(1); break;
-            case 2: MAPP_RHO(2); break;
-            case 4: MAPP_RHO(4); break;
-            default: MAPP_RHO(8); break;
-        }
-#undef MAPP_RHO
+        const auto rho_pass = br == 1   ? (lg ? k_eam_rho_lds<1, true> : k_eam_rho_lds<1, false>)
+                              : br == 2 ? (lg ? k_eam_rho_lds<2, true> : k_eam_rho_lds<2, false>)
+                              : br == 4 ? (lg ? k_eam_rho_lds<4, true> : k_eam_rho_lds<4, false>)
+                                        : k_eam_rho_lds<8, false>;  // only one lane an atom takes 8
+        hipLaunchKernelGGL(rho_pass, dim3(G), dim3(kBigBlock), rho_lds_bytes_, stream_, n_, lg, stop, rec_.get(),
+                           nn_.get(), list4(), ldl_, maxb, P, r16_, rho_m_lo_, rho_nwin_, ro, xr_.get(), part_.get());
         prof_.end(stream_);
         prof_.begin(K_EAM_FORCE, stream_);
         double* p2 = part_.get() + (size_t)G * kPartW;
-#define MAPP_FORCE(B, EV) hipLaunchKernelGGL((k_eam_force_lds<B, EV>), dim3(G), dim3(kBigBlock), f_lds_bytes_, \
-                                             stream_, n_, lg, stop, xr_.get(), r16_, nn_.get(), list4(), ldl_, maxb, \
+#define MAPP_FORCE(B, EV) hipLaunchKernelGGL((lg ? k_eam_force_lds<B, EV, true> : k_eam_force_lds<B, EV, false>), \
+                                             dim3(G), dim3(kBigBlock), f_lds_bytes_, stream_, n_, lg, stop, xr_.get(), r16_, nn_.get(), list4(), ldl_, maxb, \
                                              P, f_m_lo_, f_nwin_, fo, p2, K, v_.get(), p3, p4)
         // 1024-thread workgroups leave 128 VGPRs per lane: batches of 4 fit
         // without the FP64 energy and virial sums only
