@@ -178,15 +178,19 @@ __device__ inline double root64(double rsq)
 }
 
 // r = sqrt(x) and 1 / r to an ulp or so: the hardware's reciprocal root
-// (about 24 bits), one third-order step for the inverse, one for the root
+// (about 24 bits), one third-order step for the inverse, one for the root.
+// The steps multiply 0 by infinity at x = 0 and x = infinity, which are their
+// own roots and have the hardware's inverses: a caller's comparison takes such
+// a distance as it takes sqrt's.
 __device__ inline void root_inv(double x, double& r, double& r_inv)
 {
-    double y = __builtin_amdgcn_rsq(x);
-    const double e = fma(-(x * y), y, 1.0);
-    y = fma(y * e, fma(0.375, e, 0.5), y);
+    const double y0 = __builtin_amdgcn_rsq(x);
+    const double e = fma(-(x * y0), y0, 1.0);
+    const double y = fma(y0 * e, fma(0.375, e, 0.5), y0);
     const double t = x * y;
-    r = fma(fma(-t, t, x), 0.5 * y, t);
-    r_inv = y;
+    const bool inside = e < 1.0;  // not for 0, infinity and NaN
+    r = inside ? fma(fma(-t, t, x), 0.5 * y, t) : x;
+    r_inv = inside ? y : y0;
 }
 
 inline uint32_t morton3(uint32_t a, uint32_t b, uint32_t c)

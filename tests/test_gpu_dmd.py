@@ -90,6 +90,30 @@ def test_box_change_and_static_force_calc_match_oracle(M, cuh):
     close(f2, fo, "f_x after a rejected box")
 
 
+@pytest.mark.parametrize("face", [False, True])
+def test_coincident_sites_have_no_finite_gradient(M, cuh, face):
+    # a site given twice, or on both faces of the box: r = 0 stays a pair, and
+    # its 1 / r makes the totals and the two sites' gradient non-finite, in
+    # every table mode; what the oracle has finite stays so
+    x, H, elem, alpha, c = pot.dmd_cuh_sites((3, 3, 3), seed=3)
+    x = x - x[0]
+    x = np.concatenate([x, [H[0] if face else x[0]]])
+    elem, alpha, c = (np.concatenate([v, v[:1]]) for v in (elem, alpha, c))
+    g, o = both(M, cuh, x, H, elem, alpha, c)
+    fo, fao, muo, feo, FHo, So = o.force()
+    assert not np.isfinite(feo) and 0 < np.isfinite(fo).all(1).sum() < len(x)
+    for mode in ("FP64", "batch 2", "single pairs", "FP32 knots", "FP32 rows"):
+        g.set_batch({"batch 2": 2, "single pairs": 1}.get(mode, 4))
+        g.set_fp32(mode.startswith("FP32"), rows=mode == "FP32 rows")
+        f, fa, mu, fe, FH, S = g.derivative()
+        say(f"DMD coincident sites, {mode}: fe {fe}, {np.isfinite(f).all(1).sum()} of {len(x)} sites with finite f")
+        assert not np.isfinite(fe) and not np.isfinite(FH).any() and not np.isfinite(g.value())
+        for a, b in ((f, fo), (fa, fao), (mu, muo)):
+            assert not np.isfinite(a[[0, -1]]).all(1).any()
+            assert np.isfinite(a[np.isfinite(b)]).all()
+        assert abs(S - So) < 1e-12 * abs(So)
+
+
 @pytest.mark.parametrize("nr,rows", [(5000, True), (5000, False), (20000, False)])
 def test_fp32_tables_stay_within_the_stated_bars(M, nr, rows):
     # FP32 pair splines, FP64 moments and sums: the free energy and gradient
