@@ -330,14 +330,22 @@ __device__ int build_list(const RepArgs& A, Ctx& C, const RepArrays& R)
                     visit(j, xj, (uint32_t)(int)(n0 + 5.0 * n1 + 25.0 * n2 + (double)kZeroImage));
                 continue;
             }
-            for (double n2 = ceil(ds[2] - C.cs[2]); n2 <= floor(ds[2] + C.cs[2]); n2 += 1.0)
-                for (double n1 = ceil(ds[1] - C.cs[1]); n1 <= floor(ds[1] + C.cs[1]); n1 += 1.0)
-                    for (double n0 = ceil(ds[0] - C.cs[0]); n0 <= floor(ds[0] + C.cs[0]); n0 += 1.0) {
-                        if (fmax(fabs(n0), fmax(fabs(n1), fabs(n2))) > (double)kRepMaxImages)
-                            fail = fmax(fail, (double)FAIL_IMAGE);
-                        else
-                            visit(j, xj, (uint32_t)(int)(n0 + 5.0 * n1 + 25.0 * n2 + (double)kZeroImage));
-                    }
+            // the images in reach along every vector, of those that have a code
+            double lo[3], hi[3];
+            bool any = true, far = false;
+            for (int d = 0; d < 3; ++d) {
+                const double a = ceil(ds[d] - C.cs[d]), b = floor(ds[d] + C.cs[d]);
+                any = any && a <= b;
+                far = far || a < -(double)kRepMaxImages || b > (double)kRepMaxImages;
+                lo[d] = fmax(a, -(double)kRepMaxImages);
+                hi[d] = fmin(b, (double)kRepMaxImages);
+            }
+            if (any && far) fail = fmax(fail, (double)FAIL_IMAGE);
+            if (!any) continue;
+            for (double n2 = lo[2]; n2 <= hi[2]; n2 += 1.0)
+                for (double n1 = lo[1]; n1 <= hi[1]; n1 += 1.0)
+                    for (double n0 = lo[0]; n0 <= hi[0]; n0 += 1.0)
+                        visit(j, xj, (uint32_t)(int)(n0 + 5.0 * n1 + 25.0 * n2 + (double)kZeroImage));
         }
         if (cnt > C.maxn) fail = fmax(fail, (double)FAIL_LIST);
         R.nn[C.off + i] = cnt < C.maxn ? cnt : C.maxn;

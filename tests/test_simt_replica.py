@@ -109,3 +109,22 @@ def test_emulated_replicas_take_the_oracle_steps(emu, cells, waves, graph):
         ds = (xs[r] - xo) @ np.linalg.inv(H)
         ds -= np.round(ds)
         assert np.abs(ds @ H).max() < 1e-8
+
+
+@pytest.mark.timeout(120)
+@pytest.mark.parametrize("waves", [1, 4])
+@pytest.mark.parametrize("max_dx", [1e3, 1e20])
+def test_emulated_replica_refuses_atoms_thrown_out_of_the_box(emu, cells, waves, max_dx):
+    # a box thinner than twice the list cut-off, whose atoms the first trial
+    # moves by max_dx: past 2^53 boxes the next image is the same number
+    H, x, elem = cells[0][0]
+    h = emu.emu_replica_create(pot.NIALH_JEA.encode(), 1, P(np.array([len(x)], np.int32), ip),
+                               P(np.ascontiguousarray(H)), P(np.ascontiguousarray(x)),
+                               P(elem.astype(np.uint8), u8p), 0.5)
+    assert h
+    emu.emu_replica_set_waves(h, P(np.full(5, waves, np.int32), ip))
+    steps, status = np.zeros(1, np.int32), np.zeros(1, np.int32)
+    e0, e = np.zeros(1), np.zeros(1)
+    rc = emu.emu_replica_min_cg(h, NSTEPS, 0.0, max_dx, P(steps, ip), P(status, ip), P(e0), P(e))
+    emu.emu_replica_free(h)
+    assert rc == 5 and status[0] == 102 and steps[0] == 0
