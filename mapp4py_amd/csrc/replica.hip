@@ -695,10 +695,12 @@ __device__ void run_rep(const RepArgs& A, RepCell* __restrict__ cells, int r, co
 // workgroup owns (largest first) from queue[0]; then each wave takes one-wave
 // replicas from queue[1] on its own. Every lane of a wave joins the queue
 // atomic (lane 0 adds 1, the others 0) and the ticket is read from the first
-// lane, so the replica index is wave-uniform.
+// lane, so the replica index is wave-uniform. Only the first w1 waves of a
+// workgroup take one-wave replicas, w1 as few as spread them over all
+// workgroups.
 __global__ __launch_bounds__(64 * kWide) void k_replica_cg(RepArgs A, RepCell* cells, const int* __restrict__ q4,
-                                                           int n4, const int* __restrict__ q1, int n1, int* queue,
-                                                           RepArrays R)
+                                                           int n4, const int* __restrict__ q1, int n1, int w1,
+                                                           int* queue, RepArrays R)
 {
     __shared__ Shared S;
     const int lane = threadIdx.x & 63;
@@ -719,7 +721,7 @@ __global__ __launch_bounds__(64 * kWide) void k_replica_cg(RepArgs A, RepCell* c
         run_rep<kWide>(A, cells, q4[t], R, S, w, lane);
         __syncthreads();
     }
-    while (true) {
+    while (w < w1) {
         const int t = __builtin_amdgcn_readfirstlane(atomicAdd(&queue[1], lane == 0 ? 1 : 0));
         if (t >= n1) break;
         run_rep<1>(A, cells, q1[t], R, S, w, lane);
@@ -902,8 +904,10 @@ void ReplicaBatch::launch(State& st, const RepArgs& A, const int* q4, int n4, co
     RepArrays R{st.x.get(), x0_.get(), xb_.get(), h_.get(), f_.get(), f0_.get(), dF_.get(), list_.get(), nn_.get(),
                 cid_.get(), ord_.get(), cand_.get()};
     k_replica_reset<<<1, 64, 0, stream_>>>(queue_.get());
-    const int blocks = std::max(1, std::min(grid_, std::max(n4, (n1 + kWide - 1) / kWide)));
-    k_replica_cg<<<blocks, 64 * kWide, 0, stream_>>>(A, st.cells.get(), q4, n4, q1, n1, queue_.get(), R);
+    // one workgroup per replica up to what the chip holds at once, of either shape
+    const int blocks = std::max(1, std::min(grid_, std::max(n4, n1)));
+    const int w1 = std::min(kWide, (n1 + blocks - 1) / blocks);
+    k_replica_cg<<<blocks, 64 * kWide, 0, stream_>>>(A, st.cells.get(), q4, n4, q1, n1, w1, queue_.get(), R);
     MAPP_HIP(hipGetLastError());
 }
 

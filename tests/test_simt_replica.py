@@ -128,3 +128,16 @@ def test_emulated_replica_refuses_atoms_thrown_out_of_the_box(emu, cells, waves,
     rc = emu.emu_replica_min_cg(h, NSTEPS, 0.0, max_dx, P(steps, ip), P(status, ip), P(e0), P(e))
     emu.emu_replica_free(h)
     assert rc == 5 and status[0] == 102 and steps[0] == 0
+
+
+@pytest.mark.parametrize("waves", [1, 4])
+def test_emulated_replicas_beyond_the_workgroups_take_the_same_steps(emu, cells, waves):
+    # more replicas than the two emulated workgroups: several one-wave replicas
+    # a workgroup, or several rounds; equal cells give equal results
+    cl, ref = cells
+    steps, status, e0, e, xs = run(emu, [cl[k % 2] for k in range(5)], waves)
+    for r in range(5):
+        ro, xo = ref[r % 2]
+        assert steps[r] == ro["steps"] and status[r] == ro["status"]
+        assert abs(e[r] - ro["e"]) < 1e-10 * abs(ro["e"])
+        assert e[r] == e[r % 2] and np.array_equal(xs[r], xs[r % 2])
