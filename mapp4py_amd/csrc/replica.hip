@@ -8,13 +8,13 @@
 //   DynamicMD::decide (skin check, rebuild)           src/dynamic_md.cpp:90-105
 //
 // Design: a replica's minimisation is sequential, so the parallelism is
-// across replicas and, inside one, across its atoms. One wave or
-// a whole 1024-thread workgroup owns a replica for
-// the entire minimisation: its full neighbor list (every periodic image,
-// 7-bit image codes), both EAM passes in FP64, the inner products and the
-// line search all run inside the one persistent launch, with no host round
-// trip per step. The size classes are split between the two shapes by a
-// tuner that times every threshold on a copy of the batch. All arithmetic is
+// across replicas and, inside one, across its atoms. One wave or a whole
+// workgroup of 4 or 16 waves owns a replica for the entire minimisation: its
+// full neighbor list (every periodic image, 7-bit image codes), both EAM
+// passes in FP64, the inner products and the line search all run inside the
+// one persistent launch, with no host round trip per step. The size classes
+// are split between the shapes by a rule on the batch (default_waves) or by a
+// tuner that times every threshold on a copy of it. All arithmetic is
 // FP64 with contraction off, so energies and line-search decisions are the
 // reference's to the rounding of the sums.
 #include <algorithm>
@@ -68,21 +68,24 @@ __device__ inline double uni(double v)
     return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
 }
 
-// Waves of the workgroup that owns a replica. The largest replica's chain of
-// steps ends the launch, so it gets every wave a CU can hold at 128 registers
-// a lane. 1024 Ni-H cells of 108 to 4,076 atoms, 20 steps each: 390 ms with
-// four waves, all-pairs list builds and one entry after another in the passes,
-// 59 ms now. In the largest cell a density pass takes 0.31 ms (its issue
-// bound, 4 atoms a lane, is about 0.15), a force pass 0.44 and a list build
-// 2.3, of 20 steps' 40 density and 20 force passes and 8 builds.
-constexpr int kWide = 16;
+// Waves of the workgroup that owns a replica. Where the largest replica's
+// chain of steps ends the launch, it gets every wave a CU can hold at 128
+// registers a lane. 1024 Ni-H cells of 108 to 4,076 atoms, 20 steps each: 390
+// ms with four waves, all-pairs list builds and one entry after another in the
+// passes, 59 ms now. In the largest cell a density pass takes 0.31 ms (its
+// issue bound, 4 atoms a lane, is about 0.15), a force pass 0.44 and a list
+// build 2.3, of 20 steps' 40 density and 20 force passes and 8 builds.
+// Where there are more small replicas than CUs, four workgroups of 4 waves a
+// CU (wide_workgroup).
+constexpr int kWide = 16, kNarrow = 4;
 constexpr int kShifts = 125;  // image codes
 
+template <int K>  // waves of the workgroup
 struct Shared {
-    double red[2][kWide];             // partial sums, two rows in turn
-    double shift[kWide][kShifts][3];  // n H of every image code: row 0 of a workgroup's replica, row w of a wave's
-    int own0[65 * kWide];             // list build: where each cell's (segment's) atoms start in ord,
-    int cand0[65 * kWide];            // and its candidates; 65 a wave or all for a workgroup
+    double red[2][K];             // partial sums, two rows in turn
+    double shift[K][kShifts][3];  // n H of every image code: row 0 of a workgroup's replica, row w of a wave's
+    int own0[65 * K];             // list build: where each cell's (segment's) atoms start in ord,
+    int cand0[65 * K];            // and its candidates; 65 a wave or all for a workgroup
     double cut_sq[kMaxElems * kMaxElems], cutsk_sq[kMaxElems * kMaxElems];
     int next;
 };
@@ -101,10 +104,14 @@ __device__ inline void group_sync()
 struct Ctx {
     int off, n, maxn, nt, t, w;
     int lg;    // log2 of the lanes that share an atom in the EAM passes
-    int flip;  // row of Shared::red of the next sum
+    int flip;  // row of red of the next sum
     long long loff;
     double h[6], b[6], cs[3];
-    Shared* S;
+    // the replica's parts of Shared
+    double* red;
+    double (*shift)[3];
+    int *own0, *cand0;
+    const double *cut_sq, *cutsk_sq;
 };
 
 // sums and maxima over the replica's lanes, in a fixed order, returned alike
@@ -120,7 +127,7 @@ __device__ inline double group_fold(double v, Ctx& C, Op op)
         group_sync<1>();
         return v;
     } else {
-        double* row = C.S->red[C.flip];
+        double* row = C.red + C.flip * W;
         C.flip ^= 1;
         row[C.w] = v;
         __syncthreads();
@@ -174,9 +181,7 @@ __device__ int build_list(const RepArgs& A, Ctx& C, const RepArrays& R)
 {
     constexpr int kCells = 64 * W;  // most cells, and cells times segments
     const int ne = A.ne;
-    const double(*shift)[3] = C.S->shift[W == 1 ? C.w : 0];
-    int* own0 = C.S->own0 + (W == 1 ? (64 + 1) * C.w : 0);
-    int* cand0 = C.S->cand0 + (W == 1 ? (64 + 1) * C.w : 0);
+    int *own0 = C.own0, *cand0 = C.cand0;
     int* ord = R.ord + C.off;
     uint32_t* cand = R.cand + 27 * (size_t)C.off;
     int nc[3];
@@ -293,9 +298,9 @@ __device__ int build_list(const RepArgs& A, Ctx& C, const RepArrays& R)
         int cnt = 0;
         auto visit = [&](int j, const double4& xj, uint32_t code) {
             double dx, dy, dz;
-            image_dx(shift, xi, xj, code, dx, dy, dz);
+            image_dx(C.shift, xi, xj, code, dx, dy, dz);
             const double rsq = dx * dx + (dy * dy + dz * dz);
-            if (rsq < C.S->cutsk_sq[ei * ne + (int)xj.w] && (j != i || code != (uint32_t)kZeroImage)) {
+            if (rsq < C.cutsk_sq[ei * ne + (int)xj.w] && (j != i || code != (uint32_t)kZeroImage)) {
                 if (cnt < C.maxn) R.list[C.loff + (long long)cnt * C.n + i] = (uint32_t)j | (code << kIndexBits);
                 ++cnt;
             }
@@ -376,7 +381,6 @@ __device__ double eam_energy(const RepArgs& A, Ctx& C, const RepArrays& R)
 {
     constexpr int B = 4;
     const int ne = A.ne, nr = A.nr, G = 1 << C.lg, g = C.t & (G - 1), units = C.nt >> C.lg;
-    const double(*shift)[3] = C.S->shift[W == 1 ? C.w : 0];
     double part = 0.0;
     for (int i0 = 0; i0 < C.n; i0 += units) {
         const int i = i0 + (C.t >> C.lg);
@@ -394,9 +398,9 @@ __device__ double eam_energy(const RepArgs& A, Ctx& C, const RepArrays& R)
             for (int b = 0; b < B; ++b) {
                 const int ej = (int)xj[b].w;
                 double dx, dy, dz, r;
-                image_dx(shift, xi, xj[b], e[b] >> kIndexBits, dx, dy, dz);
+                image_dx(C.shift, xi, xj[b], e[b] >> kIndexBits, dx, dy, dz);
                 const double rsq = dx * dx + (dy * dy + dz * dz);
-                in[b] = k0 + b < cnt && rsq < C.S->cut_sq[ei * ne + ej];
+                in[b] = k0 + b < cnt && rsq < C.cut_sq[ei * ne + ej];
                 int m;
                 root_inv(in[b] ? rsq : 1.0, r, ri[b]);
                 spline_at(r, A.dr_inv, nr, m, p[b]);
@@ -433,7 +437,6 @@ __device__ void eam_force(const RepArgs& A, Ctx& C, const RepArrays& R)
 {
     constexpr int B = 2;
     const int ne = A.ne, nr = A.nr, G = 1 << C.lg, g = C.t & (G - 1), units = C.nt >> C.lg;
-    const double(*shift)[3] = C.S->shift[W == 1 ? C.w : 0];
     for (int i0 = 0; i0 < C.n; i0 += units) {
         const int i = i0 + (C.t >> C.lg);
         const bool own = i < C.n;
@@ -452,9 +455,9 @@ __device__ void eam_force(const RepArgs& A, Ctx& C, const RepArrays& R)
                 const int ej = (int)xj[b].w;
                 double r;
                 dFj[b] = R.dF[C.off + (int)(e[b] & kIndexMask)];
-                image_dx(shift, xi, xj[b], e[b] >> kIndexBits, dx[b], dy[b], dz[b]);
+                image_dx(C.shift, xi, xj[b], e[b] >> kIndexBits, dx[b], dy[b], dz[b]);
                 const double rsq = dx[b] * dx[b] + (dy[b] * dy[b] + dz[b] * dz[b]);
-                in[b] = k0 + b < cnt && rsq < C.S->cut_sq[ei * ne + ej];
+                in[b] = k0 + b < cnt && rsq < C.cut_sq[ei * ne + ej];
                 int m;
                 root_inv(in[b] ? rsq : 1.0, r, ri[b]);
                 spline_at(r, A.dr_inv, nr, m, p[b]);
@@ -512,8 +515,8 @@ __device__ double trial(const RepArgs& A, Ctx& C, const RepArrays& R, double alp
 // condition derives from the header (read through readfirstlane) or from
 // group sums that every lane receives alike, and every lane stores the
 // results alike.
-template <int W>
-__device__ void run_rep(const RepArgs& A, RepCell* __restrict__ cells, int r, const RepArrays& R, Shared& S, int w,
+template <int W, int K>
+__device__ void run_rep(const RepArgs& A, RepCell* __restrict__ cells, int r, const RepArrays& R, Shared<K>& S, int w,
                         int lane)
 {
     Ctx C;
@@ -535,7 +538,12 @@ __device__ void run_rep(const RepArgs& A, RepCell* __restrict__ cells, int r, co
     C.w = w;
     C.t = W == 1 ? lane : w * 64 + lane;
     C.flip = 0;
-    C.S = &S;
+    C.red = &S.red[0][0];
+    C.shift = S.shift[W == 1 ? w : 0];
+    C.own0 = S.own0 + (W == 1 ? 65 * w : 0);
+    C.cand0 = S.cand0 + (W == 1 ? 65 * w : 0);
+    C.cut_sq = S.cut_sq;
+    C.cutsk_sq = S.cutsk_sq;
     // lanes per atom: the fewest rounds of a pass over about 70 entries in
     // batches of 4, with the constant work of a round (its loads and sums)
     // taken as 8 entries
@@ -549,7 +557,7 @@ __device__ void run_rep(const RepArgs& A, RepCell* __restrict__ cells, int r, co
     }
     for (int c = C.t; c < kShifts; c += C.nt) {
         const int n2 = c / 25 - 2, n1 = c % 25 / 5 - 2, n0 = c % 5 - 2;
-        double* sh = S.shift[W == 1 ? w : 0][c];
+        double* sh = C.shift[c];
         sh[0] = C.h[0] * n0 + C.h[1] * n1 + C.h[2] * n2;
         sh[1] = C.h[3] * n1 + C.h[4] * n2;
         sh[2] = C.h[5] * n2;
@@ -698,14 +706,15 @@ __device__ void run_rep(const RepArgs& A, RepCell* __restrict__ cells, int r, co
 // lane, so the replica index is wave-uniform. Only the first w1 waves of a
 // workgroup take one-wave replicas, w1 as few as spread them over all
 // workgroups.
-__global__ __launch_bounds__(64 * kWide) void k_replica_cg(RepArgs A, RepCell* cells, const int* __restrict__ q4,
-                                                           int n4, const int* __restrict__ q1, int n1, int w1,
-                                                           int* queue, RepArrays R)
+template <int K>
+__global__ __launch_bounds__(64 * K, 4) void k_replica_cg(RepArgs A, RepCell* cells, const int* __restrict__ q4,
+                                                          int n4, const int* __restrict__ q1, int n1, int w1,
+                                                          int* queue, RepArrays R)
 {
-    __shared__ Shared S;
+    __shared__ Shared<K> S;
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    for (int k = threadIdx.x; k < A.ne * A.ne; k += 64 * kWide) {
+    for (int k = threadIdx.x; k < A.ne * A.ne; k += 64 * K) {
         S.cut_sq[k] = A.cut_sq[k];
         S.cutsk_sq[k] = A.cutsk_sq[k];
     }
@@ -718,7 +727,7 @@ __global__ __launch_bounds__(64 * kWide) void k_replica_cg(RepArgs A, RepCell* c
         const int t = __builtin_amdgcn_readfirstlane(S.next);
         __syncthreads();
         if (t >= n4) break;
-        run_rep<kWide>(A, cells, q4[t], R, S, w, lane);
+        run_rep<K>(A, cells, q4[t], R, S, w, lane);
         __syncthreads();
     }
     while (w < w1) {
@@ -851,11 +860,13 @@ ReplicaBatch::ReplicaBatch(std::shared_ptr<EamForceField> ff, int nrep, const in
         MAPP_HIP(hipMemcpy(st_.cells.get(), host_cells_.data(), nrep * sizeof(RepCell), hipMemcpyHostToDevice));
     }
     MAPP_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
-    int dev = 0, ncu = 0, per = 0;
+    int dev = 0, per[2] = {0, 0};
     MAPP_HIP(hipGetDevice(&dev));
-    MAPP_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-    MAPP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_replica_cg, 64 * kWide, 0));
-    grid_ = std::max(1, ncu * std::max(1, per));
+    MAPP_HIP(hipDeviceGetAttribute(&ncu_, hipDeviceAttributeMultiprocessorCount, dev));
+    MAPP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per[0], k_replica_cg<kNarrow>, 64 * kNarrow, 0));
+    MAPP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per[1], k_replica_cg<kWide>, 64 * kWide, 0));
+    for (int k = 0; k < 2; ++k) grid_[k] = std::max(1, ncu_ * std::max(1, per[k]));
+    default_waves();
 }
 
 ReplicaBatch::~ReplicaBatch()
@@ -883,7 +894,33 @@ RepArgs ReplicaBatch::args(int max_nsteps, double e_tol, double max_dx, double c
     return A;
 }
 
-void ReplicaBatch::build_queues(const int* waves, DevBuf<int>& q4, int& n4, DevBuf<int>& q1, int& n1) const
+// Whether workgroups of 16 waves take the num replicas of which the largest has
+// nmax atoms. A small replica leaves most of 16 waves waiting at barriers; a
+// large one's chain is twice as long on 4. 10 steps, 4 waves and 16:
+//   384 cells of 108 atoms  3.0 and 4.8 ms, of 256  3.6 and  5.5, of 500 10.1 and 10.6
+// 1,024 cells of 108 atoms  3.7 and 9.8 ms, of 256  5.8 and 10.9, of 500 16.5 and 21.0
+//   256 cells of 108 atoms  2.6 and 2.7 ms, of 500  8.6 and  6.1
+//   864 atoms: 512 cells 26.9 and 24.4, 768 32.7 and 34.7; 1,372 atoms: 768 45.7 and 41.7, 1,024 54.3 and 55.3
+bool ReplicaBatch::wide_workgroup(int num, int nmax) const
+{
+    return !(nmax < 512 ? num > ncu_ : nmax < 1024 && num >= 3 * ncu_);
+}
+
+// The shapes until set_waves or tune: workgroups, except for small cells in
+// numbers beside large ones, which hold the workgroups at 16 waves (10 steps,
+// one wave and 16 waves a cell: 1,024 cells of 108 atoms 6.0 and 9.8 ms, of 256
+// 11.5 and 10.9; 2,048 of 256 14.6 and 20.9, of 400 32 and 33, of 500 45 and 41)
+void ReplicaBatch::default_waves()
+{
+    int cnt[5] = {0, 0, 0, 0, 0};
+    for (const RepCell& c : host_cells_) ++cnt[c.cls];
+    std::fill(waves_, waves_ + 5, 4);
+    if (cnt[2] + cnt[3] + cnt[4] == 0) return;
+    if (cnt[0] >= 4 * ncu_) waves_[0] = 1;
+    if (cnt[1] >= 8 * ncu_) waves_[1] = 1;
+}
+
+void ReplicaBatch::build_queues(const int* waves, DevBuf<int>& q4, int& n4, DevBuf<int>& q1, int& n1, bool& wide) const
 {
     std::vector<int> order(nr_);
     std::iota(order.begin(), order.end(), 0);
@@ -893,21 +930,24 @@ void ReplicaBatch::build_queues(const int* waves, DevBuf<int>& q4, int& n4, DevB
     for (int r : order) (waves[host_cells_[r].cls] == 4 ? v4 : v1).push_back(r);
     n4 = (int)v4.size();
     n1 = (int)v1.size();
+    wide = wide_workgroup(n4, n4 ? host_cells_[v4[0]].n : 0);
     q4.reserve(std::max(1, n4));
     q1.reserve(std::max(1, n1));
     if (n4) MAPP_HIP(hipMemcpy(q4.get(), v4.data(), n4 * sizeof(int), hipMemcpyHostToDevice));
     if (n1) MAPP_HIP(hipMemcpy(q1.get(), v1.data(), n1 * sizeof(int), hipMemcpyHostToDevice));
 }
 
-void ReplicaBatch::launch(State& st, const RepArgs& A, const int* q4, int n4, const int* q1, int n1)
+void ReplicaBatch::launch(State& st, const RepArgs& A, const int* q4, int n4, const int* q1, int n1, bool wide)
 {
     RepArrays R{st.x.get(), x0_.get(), xb_.get(), h_.get(), f_.get(), f0_.get(), dF_.get(), list_.get(), nn_.get(),
                 cid_.get(), ord_.get(), cand_.get()};
     k_replica_reset<<<1, 64, 0, stream_>>>(queue_.get());
+    const auto run = wide ? k_replica_cg<kWide> : k_replica_cg<kNarrow>;
+    const int K = wide ? kWide : kNarrow;
     // one workgroup per replica up to what the chip holds at once, of either shape
-    const int blocks = std::max(1, std::min(grid_, std::max(n4, n1)));
-    const int w1 = std::min(kWide, (n1 + blocks - 1) / blocks);
-    k_replica_cg<<<blocks, 64 * kWide, 0, stream_>>>(A, st.cells.get(), q4, n4, q1, n1, w1, queue_.get(), R);
+    const int blocks = std::max(1, std::min(grid_[wide], std::max(n4, n1)));
+    const int w1 = std::min(K, (n1 + blocks - 1) / blocks);
+    run<<<blocks, 64 * K, 0, stream_>>>(A, st.cells.get(), q4, n4, q1, n1, w1, queue_.get(), R);
     MAPP_HIP(hipGetLastError());
 }
 
@@ -932,7 +972,7 @@ void ReplicaBatch::min_cg(int max_nsteps, double e_tol, double max_dx, double c,
 {
     const RepArgs A = args(max_nsteps, e_tol, max_dx, c, rho, min_alpha);
     if (queues_dirty_) {
-        build_queues(waves_, q4_, n4_, q1_, n1_);
+        build_queues(waves_, q4_, n4_, q1_, n1_, wide_);
         queues_dirty_ = false;
         if (graph_) {
             (void)hipGraphExecDestroy(graph_);
@@ -946,7 +986,7 @@ void ReplicaBatch::min_cg(int max_nsteps, double e_tol, double max_dx, double c,
             graph_ = nullptr;
             hipGraph_t g;
             MAPP_HIP(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
-            launch(st_, A, q4_.get(), n4_, q1_.get(), n1_);
+            launch(st_, A, q4_.get(), n4_, q1_.get(), n1_, wide_);
             MAPP_HIP(hipStreamEndCapture(stream_, &g));
             MAPP_HIP(hipGraphInstantiate(&graph_, g, nullptr, nullptr, 0));
             MAPP_HIP(hipGraphDestroy(g));
@@ -954,7 +994,7 @@ void ReplicaBatch::min_cg(int max_nsteps, double e_tol, double max_dx, double c,
         }
         MAPP_HIP(hipGraphLaunch(graph_, stream_));
     } else {
-        launch(st_, A, q4_.get(), n4_, q1_.get(), n1_);
+        launch(st_, A, q4_.get(), n4_, q1_.get(), n1_, wide_);
     }
     prof_.end(stream_);
     MAPP_HIP(hipStreamSynchronize(stream_));
@@ -977,7 +1017,7 @@ void ReplicaBatch::min_cg(int max_nsteps, double e_tol, double max_dx, double c,
 }
 
 // Tile tuner: one wave per replica for the size classes below a threshold,
-// four from there up. Every threshold is timed on a copy of the batch (the
+// a workgroup from there up. Every threshold is timed on a copy of the batch (the
 // production positions are not moved) and the fastest is kept.
 RepTuneReport ReplicaBatch::tune(int max_nsteps, double e_tol, double max_dx, double c, double rho, double min_alpha)
 {
@@ -997,7 +1037,8 @@ RepTuneReport ReplicaBatch::tune(int max_nsteps, double e_tol, double max_dx, do
         for (int k = 0; k < 5; ++k) wv[k] = k < th ? 1 : 4;
         DevBuf<int> d4, d1;
         int n4 = 0, n1 = 0;
-        build_queues(wv, d4, n4, d1, n1);
+        bool wide = true;
+        build_queues(wv, d4, n4, d1, n1, wide);
         float ms = 1e30f;
         for (int k = 0; k < (th < 0 ? 1 : 2); ++k) {
             MAPP_HIP(hipMemcpyAsync(scratch_.cells.get(), st_.cells.get(), nr_ * sizeof(RepCell),
@@ -1005,7 +1046,7 @@ RepTuneReport ReplicaBatch::tune(int max_nsteps, double e_tol, double max_dx, do
             MAPP_HIP(hipMemcpyAsync(scratch_.x.get(), st_.x.get(), natot_ * sizeof(double4), hipMemcpyDeviceToDevice,
                                     stream_));
             MAPP_HIP(hipEventRecord(e0, stream_));
-            launch(scratch_, A, d4.get(), n4, d1.get(), n1);
+            launch(scratch_, A, d4.get(), n4, d1.get(), n1, wide);
             MAPP_HIP(hipEventRecord(e1, stream_));
             MAPP_HIP(hipEventSynchronize(e1));
             float t = 0.f;

@@ -86,8 +86,10 @@ private:
         DevBuf<RepCell> cells;
         DevBuf<double4> x;
     };
-    void launch(State& st, const RepArgs& A, const int* q4, int n4, const int* q1, int n1);
-    void build_queues(const int* waves, DevBuf<int>& q4, int& n4, DevBuf<int>& q1, int& n1) const;
+    void launch(State& st, const RepArgs& A, const int* q4, int n4, const int* q1, int n1, bool wide);
+    void build_queues(const int* waves, DevBuf<int>& q4, int& n4, DevBuf<int>& q1, int& n1, bool& wide) const;
+    bool wide_workgroup(int num, int nmax) const;
+    void default_waves();
     RepArgs args(int max_nsteps, double e_tol, double max_dx, double c, double rho, double min_alpha) const;
 
     std::shared_ptr<EamForceField> ff_;
@@ -96,16 +98,16 @@ private:
     RepArgs A0_{};
     hipStream_t stream_ = nullptr;
     std::vector<RepCell> host_cells_;
-    int waves_[5] = {4, 4, 4, 4, 4};  // whole workgroups: 59 ms for 1024 cells of 108 to 4,076 atoms, 122 with one wave for those below 512
+    int waves_[5];
     State st_, scratch_;
     DevBuf<double4> x0_, xb_, h_, f_, f0_;
     DevBuf<double> dF_;
     DevBuf<uint32_t> list_, cand_;
     DevBuf<int> nn_, cid_, ord_, queue_, q4_, q1_;
     int n4_ = 0, n1_ = 0;
-    bool queues_dirty_ = true;
+    bool wide_ = true, queues_dirty_ = true;
     DevBuf<double4> phi_, rho4_, F4_;
-    int grid_ = 0;
+    int ncu_ = 0, grid_[2] = {0, 0};  // CUs, and workgroups of 4 and 16 waves they hold
     bool graph_on_ = false;
     hipGraphExec_t graph_ = nullptr;
     RepArgs graph_args_{};

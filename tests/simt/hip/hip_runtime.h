@@ -21,7 +21,7 @@
 #define __host__
 #define __global__
 #define __shared__ static
-#define __launch_bounds__(x)
+#define __launch_bounds__(...)
 #define __forceinline__ inline
 
 struct double4 { double x, y, z, w; };

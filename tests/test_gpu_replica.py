@@ -114,6 +114,27 @@ def test_three_element_replicas(M):
     check(b, cells, res, oracle, "Ni-H")
 
 
+@pytest.mark.parametrize("count,waves", [(261, None), (261, [4] * 5), (4100, [1] * 5), (1030, None)])
+def test_more_small_replicas_than_workgroups(M, count, waves):
+    # 256 CUs: from 257 small replicas on workgroups of 4 waves, several
+    # rounds of them from 1,025; one-wave replicas in more than one round.
+    # Equal cells give equal results
+    ff = O.OEam.read(pot.NIALH_JEA)
+    cells = []
+    for s, f in ((3, 0.1), (4, 0.3)):
+        x, H, elem = small_cell(s, k=(3, 3, 3), h_frac=f)
+        cells.append((H, x, elem))
+    oracle = [oracle_min(ff, *c) for c in cells]
+    b = M.ReplicaBatch(M.ForceFieldEAM.setfl(pot.NIALH_JEA), [cells[k % 2] for k in range(count)], skin=0.5)
+    if waves:
+        b.set_waves(waves)
+    res = b.min_cg(NSTEPS, e_tol=0.0, max_dx=1.0)
+    check(b, cells, res, oracle, f"{count} replicas")
+    for k in range(2):
+        assert np.all(res["steps"][k::2] == res["steps"][k]) and np.all(res["e"][k::2] == res["e"][k])
+        assert np.array_equal(b.x(count - 2 + (count + k) % 2), b.x(k))
+
+
 def test_tuner_and_graph_replays(M, batch_inputs):
     p, cells, oracle = batch_inputs
     b = M.ReplicaBatch(M.ForceFieldEAM.from_knots(p), cells, skin=0.5)
