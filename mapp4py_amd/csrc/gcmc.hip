@@ -599,6 +599,13 @@ __global__ __launch_bounds__(256) void k_gcmc(GcmcArgs A, GcmcCell* cells, const
 constexpr int kGcmcOneWaves = 16;
 constexpr int kMaxBins = 8192;
 
+// Attempts of a launch from which the bins pay: fewer sweep all atoms one
+// attempt at a time (k_gcmc_one_sweep). A call of 1, 6, 8 and 12 attempts takes
+// 60, 80, 88 and 102 us by sweeps and 87, 93, 95 and 96 by bins in 260 atoms;
+// 63, 97, 109 and 122, and 88, 94, 94 and 96, in 878; 69, 133, 153 and 203, and
+// 115, 141, 147 and 157, in 11,158.
+inline bool take_bins(int nattempts, int n) { return nattempts >= (n < 512 ? 10 : 7); }
+
 struct GcmcBins {
     int nb[3], cap;
     int* start;  // [bins + 1] first entry of a bin
@@ -1014,7 +1021,8 @@ __global__ __launch_bounds__(64 * kGcmcOneWaves) void k_gcmc_one(GcmcArgs A, Gcm
     }
 }
 
-// One cell in a narrower box: one attempt at a time, 16 waves on all atoms.
+// One cell in a narrower box, or for a few attempts: one attempt at a time, 16
+// waves on all atoms.
 __global__ __launch_bounds__(64 * kGcmcOneWaves) void k_gcmc_one_sweep(GcmcArgs A, GcmcCell* cells,
                                                                        int nattempts, int8_t* dec, double* dU,
                                                                        Arrays R)
@@ -1592,7 +1600,7 @@ void GcmcBatch::launch(GcmcState& st, int nattempts, int8_t* dec, double* du, co
                        int n1)
 {
     if (nc_ == 1) {
-        if (binned_) {
+        if (binned_ && take_bins(nattempts, host_cells_[0].n)) {
             const GcmcBins B = bins_of(st, nbins_, total_cap_);
             k_gcmc_bins<<<1, 1024, 0, stream_>>>(st.cells.get(), B, arrays_of(st));
             k_gcmc_one<<<1, 64 * kGcmcOneWaves, 0, stream_>>>(A_, st.cells.get(), B, nattempts, dec, du,

@@ -164,6 +164,27 @@ def test_emulated_attempts_of_a_wide_cell_reproduce_the_oracle_chain(emu, mu, se
     assert states[0]["seed"] == g.rng_seed and states[0]["ngas"] == g.ngas
 
 
+def test_emulated_launches_of_few_and_many_attempts_are_one_chain(emu):
+    # fewer than 10 attempts sweep the atoms, more take the bins; launches of
+    # both kinds in turn on one wide cell continue one chain
+    rng = np.random.default_rng(15)
+    H = np.array([[14.1, 0, 0], [1.5, 15.2, 0], [-0.8, 1.1, 13.9]])
+    x = (rng.uniform(0, 1, (70, 3))) @ H
+    e = np.where(rng.uniform(0, 1, 70) < 0.1, GAS, 0).astype(np.uint8)
+    ks = [9, 10, 1, 21, 4]
+    dec, du, states = run(emu, [(x, H, e)], -1.5, np.array([31], np.int32), ks, 4, False)
+    g = O.OGCMC(O.OEam.read(pot.NIALH_JEA), H, x, e, GAS, -1.5, 300.0, MASSES, seed=31)
+    got = [g.attempts(k) for k in ks]
+    np.testing.assert_array_equal(dec[0], np.concatenate([d for d, _ in got]))
+    u = np.concatenate([u for _, u in got])
+    assert np.abs(du[0] - u).max() < 1e-9 * max(1.0, np.abs(u).max())
+    st = g.state()
+    np.testing.assert_array_equal(states[0]["elem"], st["elem"])
+    np.testing.assert_array_equal(states[0]["x"], st["x"])
+    np.testing.assert_allclose(states[0]["rho"], st["rho"], rtol=1e-10, atol=1e-12)
+    assert states[0]["seed"] == g.rng_seed and states[0]["ngas"] == g.ngas
+
+
 @pytest.mark.parametrize("waves", [1, 4])
 def test_emulated_cells_with_more_pairs_than_the_list_holds(emu, waves):
     # 256 pairs a wave are listed; a dense cell (about 300 atoms in reach of a
