@@ -1682,6 +1682,7 @@ MDSystem::MDSystem(std::shared_ptr<EamForceField> ff, int natms, const double* H
     MAPP_HIP(hipMemsetAsync(f_.get(), 0, sizeof(float4) * n_, stream_));
     plan_lds();
     plan_alloy();
+    share_elements();
     rebuild();
 }
 
@@ -1718,6 +1719,7 @@ void MDSystem::reset_atoms(int natms, const double* x, const uint8_t* elem, cons
     sync();
     n_ = natms;
     elem_host_.assign(elem, elem + natms);
+    share_elements();
     x_.reserve(n_); x_alt_.reserve(n_); s_.reserve(n_); x0_.reserve(n_);
     v_.reserve(n_); v_alt_.reserve(n_); id_.reserve(n_); id_alt_.reserve(n_); slot_of_.reserve(n_);
     f_.reserve(n_); rho_.reserve(n_); dF_.reserve(n_); xr_.reserve(n_); rec_.reserve(n_);
@@ -1850,13 +1852,15 @@ void MDSystem::plan_alloy()
     alloy_ok_ = true;
 }
 
-// the slots in element order, and each element's share of an XCD's workgroups
-// (in proportion to its atoms, one at least)
-void MDSystem::element_order()
+// the atoms of each element, and its share of an XCD's workgroups (in
+// proportion to its atoms, one at least); for a new set of atoms
+void MDSystem::share_elements()
 {
+    share_ = ElemShare{};
+    if (!alloy_ok_) return;
     const int ne = ff_->tables().ne;
-    std::vector<int> cnt(ne, 0);
-    for (int i = 0; i < n_; ++i) ++cnt[elem_host_[i]];
+    std::vector<long> cnt(ne);
+    for (int a = 0; a < ne; ++a) cnt[a] = std::count(elem_host_.begin(), elem_host_.end(), (uint8_t)a);
     const int W = lds_grid_ / kXcd;
     std::vector<int> w(ne, 1);
     for (int left = W - ne; left > 0; --left) {
@@ -1865,11 +1869,16 @@ void MDSystem::element_order()
             if ((double)cnt[b] / w[b] > (double)cnt[a] / w[a]) a = b;
         ++w[a];
     }
-    share_ = ElemShare{};
     for (int a = 0; a < ne; ++a) {
         share_.wg0[a + 1] = share_.wg0[a] + w[a];
-        share_.at0[a + 1] = share_.at0[a] + cnt[a];
+        share_.at0[a + 1] = share_.at0[a] + (int)cnt[a];
     }
+}
+
+// the slots in element order
+void MDSystem::element_order()
+{
+    const int ne = ff_->tables().ne;
     eord_.reserve(n_);
     eval_.reserve(n_);
     ekey_.reserve(n_);

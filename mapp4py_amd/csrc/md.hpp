@@ -316,6 +316,7 @@ private:
     DevBuf<uint32_t> ekey_, ekey_alt_;
     ElemShare share_{};
     void plan_alloy();
+    void share_elements();
     void element_order();
     int lanes_alloy() const;
 };
