@@ -215,7 +215,6 @@ __global__ __launch_bounds__(kBlock) void k_build_list(int n, const double4* __r
     double xi0, xi1, xi2;
     s_to_x(bd.h, si.x, si.y, si.z, xi0, xi1, xi2);
     const int c0 = cell_coord(si.x, g.nc[0]), c1 = cell_coord(si.y, g.nc[1]), c2 = cell_coord(si.z, g.nc[2]);
-    const ListTest<ONE> listed{g, cut_lds, bd, s4, ti, xi0, xi1, xi2};
     int cnt = 0;
     uint32_t p0 = 0u, p1 = 0u, p2 = 0u, p3 = 0u;  // the block being filled
     // candidates of the stencil cell at offset (o0, o1, o2)
@@ -236,7 +235,18 @@ __global__ __launch_bounds__(kBlock) void k_build_list(int n, const double4* __r
             const uint4 rj = rn;
             rn = rec[j + 1 < je ? j + 1 : j];
             if (self_img && j == i) continue;
-            const bool in = listed(rs, rj, j, n0, n1, n2);
+            // ListTest, written out
+            const double dx = (double)(int)(rs.x - rj.x), dy = (double)(int)(rs.y - rj.y),
+                         dz = (double)(int)(rs.z - rj.z);
+            const double rsq_u = dx * dx + dy * dy + dz * dz;
+            const int tt = ONE ? 0 : ti * g.ne + (int)rj.w;
+            bool in = rsq_u < (ONE ? g.rec_in_sq[0] : cut_lds[0][tt]);
+            if (!in && rsq_u <= (ONE ? g.rec_out_sq[0] : cut_lds[1][tt])) {
+                const double4 sj = s4[j];
+                double xj0, xj1, xj2;
+                s_to_x(bd.h, shift_unit(sj.x, n0), shift_unit(sj.y, n1), shift_unit(sj.z, n2), xj0, xj1, xj2);
+                in = rsq_exact(xi0, xi1, xi2, xj0, xj1, xj2) < (ONE ? g.cut_sk_sq[0] : cut_lds[2][tt]);
+            }
             if (in) {
                 const uint32_t e = (uint32_t)j | code | (!ONE && eord ? rj.w << kElemShift : 0u);
                 const int q = cnt & 3;
