@@ -2074,7 +2074,7 @@ void MDSystem::build_list()
         list_.reserve((size_t)maxn_ * ldl_);
         MAPP_HIP(hipMemsetAsync(flags_.get(), 0, sizeof(int), stream_));
         prof_.begin(K_BUILD_LIST, stream_);
-        if (const int lg = lanes_global(); lg > 0) {
+        if (const int lg = n_ > kListLaneAtoms ? 0 : lanes_global(); lg > 0) {
             const int ng = grid_lanes(n_, lg);
 #define MAPP_BUILD(ONE) hipLaunchKernelGGL(k_build_list_group<ONE>, dim3(ng), dim3(kBlock), 0, stream_, n_, lg, \
                                            s_.get(), rec_.get(), r16_, bd, g, cell_rank_.get(), cell_start_.get(), \

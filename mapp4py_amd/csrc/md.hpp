@@ -19,6 +19,9 @@ constexpr uint32_t kIndexMask = (1u << kIndexBits) - 1u;  // image code in the h
 // and 51.7)
 constexpr int kLdsMinAtoms = 12288;
 constexpr int kAlloyMinAtoms = 49152;           // the same for several elements
+// Largest system whose list several lanes an atom build (a build at 202,612
+// atoms 170 us with two lanes, 191 with one; at 237,276 221 and 209)
+constexpr int kListLaneAtoms = 212992;
 constexpr int kStepRows = 1024;                 // rows of sums that one workgroup adds up at the end of a step
 constexpr int kMinPartRows = 4096;              // see MDSystem::part_rows
 // the alloy passes' list holds the neighbor's element above a shorter index
