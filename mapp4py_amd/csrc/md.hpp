@@ -315,8 +315,7 @@ private:
     bool alloy_list_ = false;        // the current list is the alloy passes'
     int al_rho_lo_ = 0, al_rho_nwin_ = 0, al_f_lo_ = 0, al_f_nwin_ = 0;
     size_t al_rho_lds_ = 0, al_f_lds_ = 0;
-    DevBuf<int> eord_, eval_;        // slots in element order, and the sort's input
-    DevBuf<uint32_t> ekey_, ekey_alt_;
+    DevBuf<int> eord_, epos_, ecnt_;  // slots in element order, each slot's place in it, counts by block
     ElemShare share_{};
     void plan_alloy();
     void share_elements();
