@@ -63,6 +63,21 @@ bool hermite_knots(const double* c, int nr, std::vector<double>& ys)
     return true;
 }
 
+void slope_knots(const std::vector<double>& ys, int nr, double scale, float* out)
+{
+    for (int m = 0; m < nr; ++m) out[2 * (size_t)m] = (float)(ys[2 * (size_t)m + 1] * scale);
+    for (int m = 0; m < nr; ++m) {
+        double e = 0.0;
+        if (m + 1 < nr) {
+            const double *k = &ys[2 * (size_t)m], *k1 = k + 2;
+            const double d0 = (double)out[2 * (size_t)m] - k[1] * scale;
+            const double d1 = (double)out[2 * (size_t)m + 2] - k1[1] * scale;
+            e = ((k1[0] - k[0]) - k[1]) * scale + 0.5 * (d1 - d0);
+        }
+        out[2 * (size_t)m + 1] = (float)e;
+    }
+}
+
 namespace {
 
 EamTables alloc_tables(int ne, int nr, int nrho, double dr, double drho, bool dmd)
