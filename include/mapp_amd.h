@@ -209,18 +209,19 @@ mapp_status mapp_md_profile_read(mapp_md* md, const char* kernel, double* total_
 /* Launch-shape knobs (no counterpart in the reference): neighbors resolved
  * per batch in the density pass (1, 2, 4, 8) and the force pass (1, 2, 4, 8;
  * the LDS force pass uses at most 4 in the integrator's steps, which sum no
- * energy or virial, and at most 2 otherwise). Any value gives the same
- * results to rounding. */
+ * energy or virial, and at most 2 otherwise; where several lanes share an
+ * atom, at most 4; the LDS passes of several elements have theirs fixed).
+ * Any value gives the same results to rounding. */
 mapp_status mapp_md_set_batch(mapp_md* md, int rho_batch, int force_batch);
-/* Where the passes of a one-element table read their spline rows (no
- * counterpart in the reference): on != 0 keeps a window of rows in LDS and
- * runs one persistent 1024-thread workgroup per CU (the default when the
- * device has the LDS); 0 reads the global tables. *in_use (may be NULL)
- * reports the mode in effect. */
+/* Where the passes read their splines (no counterpart in the reference):
+ * on != 0 keeps a window of them in LDS and runs one persistent 1024-thread
+ * workgroup per CU (a central element's for several elements, whose list is
+ * rebuilt when the choice changes); 0 reads the global tables. Until it is
+ * called, LDS from 12,288 atoms of one element, or 49,152 of several, where
+ * the device has it. *in_use (may be NULL) reports the mode in effect. */
 mapp_status mapp_md_set_lds(mapp_md* md, int on, int* in_use);
-/* First spline interval of the LDS row windows of the density and force
- * passes (rows from there to nr-2 are in LDS; -1 when the LDS passes are not
- * available). No counterpart in the reference. */
+/* First spline interval of the LDS windows of the density and force passes
+ * (those from there on are in LDS; -1 when the LDS passes are not available). No counterpart in the reference. */
 mapp_status mapp_md_lds_window(mapp_md* md, int* rho_first_row, int* force_first_row);
 /* AtomsMD::create_T (src/atoms_md.cpp:130-160): Maxwell velocities from the
  * Park-Miller / Marsaglia stream of src/random.cpp:7-68 seeded with seed. */

@@ -203,8 +203,10 @@ class AtomsMD:
         return a.value, b.value
 
     def set_lds(self, on):
-        """Spline rows of a one-element table in LDS (True) or read from the
-        global tables (False); returns the mode in effect."""
+        """Splines of the passes in LDS (True) or read from the global tables
+        (False), in place of the choice by the number of atoms; a change of the
+        passes of several elements rebuilds their list. Returns the mode in
+        effect."""
         used = C.c_int(0)
         check(lib().mapp_md_set_lds(self._h, int(bool(on)), C.byref(used)))
         return bool(used.value)

@@ -1846,7 +1846,7 @@ void MDSystem::reduce_rows(const double* part, int nrows, int ncols, double* out
 // per force row), leaving room for the static reduction arrays
 void MDSystem::plan_lds()
 {
-    lds_ok_ = use_lds_ = false;
+    lds_ok_ = false;
     const EamArgs P = ff_->args();
     if (P.ne != 1 || P.nr < 2) return;
     int dev = 0, lds_max = 0, ncu = 0;
@@ -1887,7 +1887,7 @@ void MDSystem::plan_lds()
             return;
         }
     }
-    lds_ok_ = use_lds_ = true;
+    lds_ok_ = true;
 }
 
 void MDSystem::plan_alloy()
@@ -1958,11 +1958,20 @@ void MDSystem::element_order()
                        eord_.get(), epos_.get());
 }
 
+// whether the next list is the alloy passes'
+bool MDSystem::want_alloy() const
+{
+    return alloy_ok_ && (uint32_t)n_ <= kAlloyMask && (lds_auto_ ? n_ >= kAlloyMinAtoms : use_lds_);
+}
+
+bool MDSystem::lds() const { return alloy_list_ || (lds_ok_ && (lds_auto_ ? n_ >= kLdsMinAtoms : use_lds_)); }
+
 bool MDSystem::set_lds(bool on)
 {
-    use_lds_ = on && lds_ok_;
+    use_lds_ = on;
     lds_auto_ = false;
-    return use_lds_;
+    if (want_alloy() != alloy_list_) rebuild();  // the two lists differ
+    return lds();
 }
 
 void MDSystem::set_batch(int rho, int force)
@@ -2087,7 +2096,7 @@ void MDSystem::rebuild()
     std::swap(id_.p, id_alt_.p);
     hipLaunchKernelGGL(k_cell_start, dim3((grid_.ncells + 1 + kBlock - 1) / kBlock), dim3(kBlock), 0, stream_, n_,
                        grid_.ncells, keys_alt_.get(), cell_start_.get());
-    alloy_list_ = alloy_ok_ && n_ >= kAlloyMinAtoms && (uint32_t)n_ <= kAlloyMask;
+    alloy_list_ = want_alloy();
     if (alloy_list_) element_order();
     prof_.end(stream_);
     build_list();
@@ -2221,7 +2230,7 @@ void MDSystem::force_passes(const KickArgs* kick, bool records_fresh, float4* f_
         hipLaunchKernelGGL(k_make_records, dim3(grid_for(n_)), dim3(kBlock), 0, stream_, n_, x_.get(), r16_,
                            rec_.get());
     const bool one = P.ne == 1;
-    const bool lds = one && use_lds_ && (!lds_auto_ || n_ >= kLdsMinAtoms);
+    const bool lds = one && this->lds();
     KickArgs K{};
     if (kick) {
         K = *kick;

@@ -41,7 +41,7 @@ struct EamArgs {
     const double* Ftab;   // [ne][nrho][4]
     // several elements whose splines are Hermite cubics of their knots
     // (nullptr otherwise): for each central element the knots of its pairs'
-    // functions, see AlloyWindow
+    // functions, see EamForceField::knot_tables
     const float* knots;
     size_t knot_stride;   // floats of one central element
     int nd;               // density functions of a central element: ne, or 2 ne - 1 with one per ordered pair
@@ -212,15 +212,16 @@ public:
     Profiler& profiler() { return prof_; }
     // launch-shape knobs picked by the tuner: neighbors resolved per batch
     void set_batch(int rho, int force);
-    // one-element tables: spline rows in LDS (persistent passes) or read from
-    // the global tables; returns whether the LDS passes are in use
+    // spline rows (of one element) or a central element's knots (of several) in
+    // LDS by persistent passes, or read from the global tables; by the number
+    // of atoms until set. Returns whether the LDS passes are in use
     bool set_lds(bool on);
-    bool lds() const { return use_lds_; }
+    bool lds() const;
     // first spline interval held in LDS by the density and force passes (-1: no LDS passes)
     void lds_window(int* rho_first, int* force_first) const
     {
-        *rho_first = lds_ok_ ? rho_m_lo_ : -1;
-        *force_first = lds_ok_ ? f_m_lo_ : -1;
+        *rho_first = lds_ok_ ? rho_m_lo_ : alloy_ok_ ? al_rho_lo_ : -1;
+        *force_first = lds_ok_ ? f_m_lo_ : alloy_ok_ ? al_f_lo_ : -1;
     }
     int batch_rho() const { return batch_rho_; }
     int batch_force() const { return batch_force_; }
@@ -292,8 +293,8 @@ private:
     Profiler prof_;
     int batch_rho_ = 8, batch_force_ = 8;
     // persistent one-element passes: LDS row windows [m_lo, m_lo + nwin)
-    bool lds_ok_ = false, use_lds_ = false;
-    bool lds_auto_ = true;           // LDS passes from kLdsMinAtoms on, until set_lds has chosen
+    bool lds_ok_ = false, use_lds_ = true;
+    bool lds_auto_ = true;           // LDS passes by the number of atoms, until set_lds has chosen use_lds_
     int lds_grid_ = 0;
     int rho_m_lo_ = 0, rho_nwin_ = 0, f_m_lo_ = 0, f_nwin_ = 0;
     size_t rho_lds_bytes_ = 0, f_lds_bytes_ = 0;
@@ -319,6 +320,7 @@ private:
     ElemShare share_{};
     void plan_alloy();
     void share_elements();
+    bool want_alloy() const;
     void element_order();
     int lanes_alloy() const;
 };
