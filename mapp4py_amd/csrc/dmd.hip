@@ -2541,7 +2541,12 @@ int DMDSystem::part_rows() const
     return std::max(grid_for(std::max(n_, nc_)), (std::max(kPassThreads, kWalkThreads) / kBlock + kXcd));
 }
 
-// the batched passes from knots in LDS: FP32 (mode 1) or FP64 (mode 0)
+// The batched passes from knots in LDS: FP32 (mode 1) or FP64 (mode 0), however
+// few knots the window holds. A gradient in FP64 from knots and from rows, 3
+// points: 256,000 sites of two elements (1,996 of 5,000 knots in LDS) 2.68 and
+// 4.74 ms; 62,500 of three (665 knots) 0.99 and 2.08; 54,000 of four with a
+// density per pair 3.07 and 3.67; 16,384 of two 0.23 and 0.32. The rows' lanes
+// would be quicker below some 8,000 sites (4,000 of two: 0.22 and 0.12).
 bool DMDSystem::use_knots(int f32) const { return f32 != 2 && knots_ok_ && !surr_ && batch_ != 1; }
 
 // the same for the LDS passes of nt threads a workgroup: the fewest rounds of

@@ -15,10 +15,15 @@ constexpr int kIndexBits = 25;                 // neighbor entry: j in the low b
 constexpr uint32_t kIndexMask = (1u << kIndexBits) - 1u;  // image code in the high 7
 // Smallest one-element system whose passes hold the spline rows in LDS: below
 // it, filling 160 KB a workgroup takes longer than reading the rows from L2
-// (an NVT step at 8,788 atoms 36.8 us with LDS, 34.9 without; at 32,000 44.0
-// and 51.7)
+// (an NVT step with LDS and without: 31.1 and 29.7 us at 6,912 atoms, 32.9 and
+// 32.9 at 11,760, 34.7 and 36.5 at 12,600, 41.5 and 52.6 at 32,000)
 constexpr int kLdsMinAtoms = 12288;
-constexpr int kAlloyMinAtoms = 49152;           // the same for several elements
+// The same for several elements, whose list also takes an element order: above
+// the sizes at which every call that was measured gains. NVT step of Fe-Ni
+// 37.5 and 31.3 us at 8,192 atoms, 46.4 and 52.5 at 24,334, 65.5 and 81.0 at
+// 54,000; force call of Ni-Al-H 74.9 and 71.2 at 32,000, 78.2 and 79.4 at
+// 42,592, 84.6 and 88.3 at 55,296.
+constexpr int kAlloyMinAtoms = 49152;
 // Largest system whose list several lanes an atom build (a build at 202,612
 // atoms 170 us with two lanes, 191 with one; at 237,276 221 and 209)
 constexpr int kListLaneAtoms = 212992;
