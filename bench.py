@@ -280,7 +280,7 @@ def muvt_cpu_baseline():
 def feni_run(steps=1000, warmup=20):
     """Binary Fe-Ni eam/fs alloy: bcc 128 x 64 x 64 cells x 2 = 1,048,576 atoms, Ni on a random
     20% of sites, Nr = Nrho = 5000, r_c = 5.3 A, NVT at 600 K and 1 fs with
-    on-device rebuilds (the multi-element passes: global spline tables)."""
+    on-device rebuilds (a central element's splines in LDS)."""
     import mapp4py_amd as M
     from mapp4py_amd import potentials as pot
 
@@ -448,7 +448,7 @@ def dmd_run(evals=10):
     ms = dt / evals * 1e3
     # FP32 pair splines (FP64 moments and sums): the same evaluations from
     # FP32 knots held in LDS and from FP32 coefficient rows, with their error
-    # against the FP64 rows (which equal the oracle to 1e-9)
+    # against the FP64 tables (which equal the oracle to 1e-9)
     def fp32_leg(rows):
         d.set_fp32(True, rows=rows)
         d.evaluate()
@@ -466,7 +466,7 @@ def dmd_run(evals=10):
                 "free_energy_rel_err": abs(fe32 - fe0) / abs(fe0),
                 "virial_rel_err": float(np.abs(FH32 - FH0).max() / np.abs(FH0).max()),
                 "dtype": what,
-                "errors_against": "the FP64 rows on the GPU (equal to the FP64 oracle to 1e-9 relative)"}
+                "errors_against": "the FP64 tables on the GPU (equal to the FP64 oracle to 1e-9 relative)"}
 
     fp32_knots = fp32_leg(False)
     fp32 = fp32_leg(True)
@@ -493,7 +493,7 @@ def dmd_run(evals=10):
     del d16
     # the accuracy / speed frontier: for each Gauss-Hermite order, networks
     # trained from that rule (box over its whole list range) against its
-    # quadrature with FP64 rows and FP32 knots, same sites
+    # quadrature in FP64 and with FP32 knots, same sites
     frontier = []
     for N in (3, 5, 8, 16):
         dn = M.AtomsDMD(M.ForceFieldEAM.from_knots(p, dmd=True), H, x, elem, alpha, c, nquad=N, masses=p.masses)
@@ -620,7 +620,7 @@ def dmd_run(evals=10):
                                                          "errors_against")},
             "fp64_rows": {"value": n * evals / dt, "ms_per_eval": ms, "pass1_ms": k1[0] / max(k1[1], 1),
                           "pass2_ms": k2[0] / max(k2[1], 1),
-                          "dtype": "f64 table rows, moments and sums (the parity mode: the FP64 oracle to 1e-9)"},
+                          "dtype": "f64 tables (knots in LDS), moments and sums (the parity mode: the FP64 oracle to 1e-9)"},
             "fp32_knots": fp32_knots, "fp32_rows": fp32,
             "host_copy_inclusive": {"value": n * evals / dt_host, "ms_per_eval": dt_host / evals * 1e3,
                                     "note": "f, f_alpha, mu gathered to caller order and copied to host each time"},
@@ -659,7 +659,7 @@ def dmd_run(evals=10):
 
 def dmd_evals_only(evals=5):
     """the 262,144-site DMD free-energy + gradient evaluations alone: FP64
-    rows, FP32 knots in LDS, FP32 rows (a short run for kernel traces and
+    and FP32 knots in LDS, FP32 rows (a short run for kernel traces and
     counters)"""
     import mapp4py_amd as M
     from mapp4py_amd import potentials as pot
@@ -1016,7 +1016,7 @@ def main():
     ap.add_argument("--no-muvt", action="store_true", help="skip the muVT measurement")
     ap.add_argument("--no-replica", action="store_true", help="skip the batched replica minimisation")
     ap.add_argument("--dmd-evals-only", action="store_true",
-                    help="only the DMD evaluations at 262,144 sites, FP64 and FP32 rows (for profiling)")
+                    help="only the DMD evaluations at 262,144 sites, FP64 and FP32 tables (for profiling)")
     ap.add_argument("--copy-calibration", action="store_true",
                     help="only run the plain copy kernel (256 MiB, 20 launches) used to calibrate HBM counters")
     args = ap.parse_args()
