@@ -553,18 +553,9 @@ struct KnotsLds {
     }
     using Acc1 = double;
     using Acc2 = F;
-    struct Basis {
-        F h1, h2, h3;
-    };
-    __device__ static Basis basis(double p)
-    {
-        const F q = (F)p, q1 = (F)1 - q, q2 = q * q;
-        return Basis{q2 * ((F)3 - (F)2 * q), q * q1 * q1, -q2 * q1};
-    }
-    __device__ static F eval(const Row& c, const Basis& h)
-    {
-        return c.y0 + (c.y1 - c.y0) * h.h1 + c.s0 * h.h2 + c.s1 * h.h3;
-    }
+    using Basis = HermiteBasis<F>;
+    __device__ static Basis basis(double p) { return hermite_basis<F>(p); }
+    __device__ static F eval(const Row& c, const Basis& h) { return hermite_eval(c.y0, c.s0, c.y1, c.s1, h); }
 };
 
 // Neighbor data of the batched passes: width, concentration and element of

@@ -193,6 +193,30 @@ __device__ inline void root_inv(double x, double& r, double& r_inv)
     r_inv = inside ? y : y0;
 }
 
+// A cubic from its end values and slopes (per unit offset) at offset p: the
+// basis, shared by the functions of an interval, and the value. In FP64 y0
+// comes last, so that only one rounding is of its size, as in the Horner scheme
+// of a coefficient row (the same rms error; 1.73 times it with y0 first; 1% of a
+// DMD gradient's time).
+template <class F>
+struct HermiteBasis {
+    F h1, h2, h3;
+};
+template <class F>
+__device__ inline HermiteBasis<F> hermite_basis(double p)
+{
+    const F q = (F)p, q1 = (F)1 - q, q2 = q * q;
+    return HermiteBasis<F>{q2 * ((F)3 - (F)2 * q), q * q1 * q1, -q2 * q1};
+}
+template <class F>
+__device__ inline F hermite_eval(F y0, F s0, F y1, F s1, const HermiteBasis<F>& h)
+{
+    if constexpr (sizeof(F) == sizeof(double))
+        return y0 + ((y1 - y0) * h.h1 + s0 * h.h2 + s1 * h.h3);
+    else
+        return y0 + (y1 - y0) * h.h1 + s0 * h.h2 + s1 * h.h3;
+}
+
 inline uint32_t morton3(uint32_t a, uint32_t b, uint32_t c)
 {
     auto spread = [](uint32_t v) {
