@@ -85,10 +85,10 @@ public:
     // free energy, F_H and entropy of the state of the last c_d (no new passes)
     DMDReport force_calc_static();
     // table evaluation of the free energy and gradient (derivative, value,
-    // the minimisers): 0 FP64 rows; 1 FP32 knots with the window in LDS (the
-    // FP32 rows where the table is not a Hermite spline of its knots); 2 FP32
+    // the minimisers): 0 FP64 and 1 FP32 knots with the window in LDS (rows
+    // where the table is not a Hermite spline of its knots); 2 FP32
     // rows. FP32 modes keep FP64 moments and sums. The concentration-rate
-    // path (c_d, J, the implicit and BDF steps) always reads the FP64 rows.
+    // path (c_d, J, the implicit and BDF steps) is always FP64.
     void set_f32(int mode);
     int f32() const { return f32_; }
     // whether mode 1 holds the knots in LDS, and the window's first knot
