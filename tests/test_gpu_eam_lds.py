@@ -216,3 +216,32 @@ def test_barostat_and_minimiser_on_the_alloy_passes(M):
         f"L-BFGS: {sa} steps, max|dx| {np.abs(ma - mb).max():.1e}, dE {abs(ea - eb):.1e}")
     assert ra == rb and np.abs(xa - xb).max() < 1e-6 and np.abs(Ha - Hb).max() < 1e-6
     assert sa == sb and np.abs(ma - mb).max() < 1e-5 and abs(ea - eb) < E_ATOM * len(x) + 1e-6
+
+
+@pytest.mark.parametrize("kind", ["cu", "feni"])
+def test_profiled_runs_time_every_pass_once(M, kind):
+    # with the kernels timed a run counts one pass a step and the first, none
+    # for the steps that find the list due, and takes the steps of one untimed
+    if kind == "cu":
+        p = pot.johnson_cu(nr=5000, nrho=5000)
+        x, H = pot.fcc(3.615, (6, 6, 7))
+        ff, x, elem, masses = M.ForceFieldEAM.from_knots(p), jitter(x, 0.05, 3), np.zeros(len(x), np.uint8), p.masses
+    else:
+        ff, _, H, x, elem, masses = system("feni", (8, 9, 8), (0.8, 0.2))
+    v = O.o_create_T(elem, masses, pot.KB_EV, 900.0, 3)
+    for run in (M.NVT(900.0, pot.FS), M.NST(np.zeros((3, 3)), 900.0, pot.FS)):
+        got = []
+        for timed in (True, False):
+            g = M.AtomsMD(ff, H, x, elem, skin=0.3)
+            g.set_lds(True)
+            g.x_d = v
+            g.profile(timed)
+            run.run(g, 40, masses)
+            if timed:
+                counts = {k: g.profile_read(k)[1] for k in ("eam_rho", "eam_force", "build_list")}
+            got.append((g.x, g.x_d, run.T_part, run.rebuilds))
+        (xa, va, Ta, ra), (xb, vb, Tb, rb) = got
+        say(f"{kind} {type(run).__name__}: launches {counts}, {ra} rebuilds")
+        assert ra == rb and ra >= 1
+        assert counts["eam_rho"] == counts["eam_force"] == 41 and counts["build_list"] == ra
+        assert np.array_equal(xa, xb) and np.array_equal(va, vb) and Ta == Tb
