@@ -160,6 +160,16 @@ public:
         if (!on || recs_.empty()) return;
         MAPP_HIP(hipEventRecord(recs_.back().b, s));
     }
+    // what has been recorded since the mark, and not flushed, does not count
+    // (launches of a halted step)
+    size_t mark() const { return recs_.size(); }
+    void drop(size_t mark)
+    {
+        for (; recs_.size() > mark; recs_.pop_back()) {
+            pool_.push_back(recs_.back().a);
+            pool_.push_back(recs_.back().b);
+        }
+    }
     // waits for the recorded events and folds them into the totals
     void flush()
     {

@@ -2658,7 +2658,7 @@ int MDSystem::nvt_run(const double* masses, double kB, double T, double dt, int 
     // each): once a step finds that the list is to be rebuilt, the launches
     // after it return at once. The first group after a rebuild ends two steps
     // before the next rebuild is due, if it comes after as many steps as the
-    // last one; then come groups of two.
+    // last one; then come groups of two. With the kernels timed, one step.
     volatile int* told = told_.get();
     int interval = 12, since = 0, step = 0, base = 0;
     told[0] = told[1] = 0;
@@ -2686,28 +2686,16 @@ int MDSystem::nvt_run(const double* masses, double kB, double T, double dt, int 
             resume();
             continue;
         }
-        if (prof_.on) {  // one step at a time, without launches that a due rebuild would halt
-            first_half();
-            int due = 0;
-            MAPP_HIP(hipMemcpyAsync(&due, flags_.get() + FL_REBUILD, sizeof(int), hipMemcpyDeviceToHost, stream_));
-            MAPP_HIP(hipStreamSynchronize(stream_));
-            if (due) {
-                rebuild();
-                resume();
-            } else {
-                second_half(step);
-                ++step;
-                ++base;
-            }
-            continue;
-        }
-        const int group =
-            std::min(std::min(std::max(2, std::min(64, interval - 2 - since)), nsteps - step), to_exchange);
+        int group = prof_.on ? 1 : std::max(2, std::min(64, interval - 2 - since));
+        group = std::min(std::min(group, nsteps - step), to_exchange);
+        size_t timed = 0;
         for (int k = 0; k < group; ++k) {
             first_half();
+            timed = prof_.mark();
             second_half(step + k);
         }
         MAPP_HIP(hipStreamSynchronize(stream_));
+        if (told[1]) prof_.drop(timed);  // its passes returned at once
         const int done = told[0] - base;
         step += done;
         since += done;

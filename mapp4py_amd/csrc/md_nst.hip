@@ -558,8 +558,28 @@ int MDSystem::nst_run(const double* masses, double kB, double T, double dt, cons
     int interval = 12, since = 0, step = 0, base = 0;
     told[0] = told[1] = 0;
     finish(-1);
-    // the list that the step's drift found due, and the rest of that step
-    const auto regrid = [&]() {
+    while (step < nsteps) {
+        int group = prof_.on ? 1 : std::max(2, std::min(64, interval - 2 - since));
+        group = std::min(group, nsteps - step);
+        size_t timed = 0;
+        for (int k = 0; k < group; ++k) {
+            drift();
+            timed = prof_.mark();
+            finish(step + k);
+        }
+        MAPP_HIP(hipStreamSynchronize(stream_));
+        if (told[1] == 1) prof_.drop(timed);  // its passes returned at once
+        prof_.flush();
+        const int done = told[0] - base;
+        step += done;
+        since += done;
+        base += done;
+        if (!told[1]) continue;
+        fetch();
+        if (told[1] == 2) {
+            refresh_frame();
+            throw Error(ERR_STATE, "the box left [vol0 / 8, 8 vol0]: NST run stopped");
+        }
         setup_grid();
         rebuild();  // the permute rewrites the records
         interval = since + 1;
@@ -569,40 +589,6 @@ int MDSystem::nst_run(const double* masses, double kB, double T, double dt, cons
         ++step;
         since = 0;
         base = 1;
-    };
-    while (step < nsteps) {
-        int due = 0;
-        if (prof_.on) {  // one step at a time, without launches that a due rebuild would halt
-            drift();
-            MAPP_HIP(hipMemcpyAsync(&due, flags_.get() + FL_REBUILD, sizeof(int), hipMemcpyDeviceToHost, stream_));
-        } else {
-            const int group = std::min(std::max(2, std::min(64, interval - 2 - since)), nsteps - step);
-            for (int k = 0; k < group; ++k) {
-                drift();
-                finish(step + k);
-            }
-        }
-        MAPP_HIP(hipStreamSynchronize(stream_));
-        prof_.flush();
-        if (prof_.on && !told[1] && !due) {
-            finish(step);
-            ++step;
-            ++base;
-            continue;
-        }
-        if (!prof_.on) {
-            const int done = told[0] - base;
-            step += done;
-            since += done;
-            base += done;
-            if (!told[1]) continue;
-        }
-        fetch();
-        if (told[1] == 2) {
-            refresh_frame();
-            throw Error(ERR_STATE, "the box left [vol0 / 8, 8 vol0]: NST run stopped");
-        }
-        regrid();
     }
     hipLaunchKernelGGL(k_nst_scale_v, dim3(nb), dim3(kBlock), 0, stream_, n_, v_.get(), st);
     if (hist && nsteps > 0)
